@@ -2,8 +2,9 @@
 // accumulated in fp32 and each output rounded once (round to nearest even for bf16), behind the reference's C-ABI
 // `launch` (softmax/kernel.cu:520-527, softmax/seed.cu:68-81).
 //
-// Tiers, chosen by row length in 16-byte vectors (4 fp32 or 8 bf16 elements), for rows whose length is a multiple of
-// the vector width and whose x and y are 16-byte aligned:
+// Tiers, chosen by row length in 16-byte vectors (4 fp32 or 8 bf16 elements). The first two have an instantiation for rows
+// whose length is a multiple of the vector width and whose x and y are 16-byte aligned, and one for any other rows of
+// at least one vector (AnyRow):
 //  - row tier (rows up to 16 waves x 64 lanes x 8 vectors = 32768 fp32 / 65536 bf16 columns): a group of WAVES waves
 //    holds one row in registers, NV 16-byte vectors per lane. A max and a sum of exp(x - max) are reduced over the
 //    group (DPP inside each wave, one LDS slot per wave across waves) and y = exp(x - max) / sum is written from the
@@ -11,8 +12,9 @@
 //    of the grid and loads its next row while it reduces and stores the current one.
 //  - co-resident tier (longer rows, up to 64 chunks of 16384 elements): one pass over x for any number of rows; see
 //    softmax_coop.
-//  - stream tier (longer rows still): one workgroup per row, two passes, no workspace; see softmax_stream.
-//  - generic tier (any length or alignment): one workgroup per row, three scalar passes (max, sum, write).
+//  - stream tier (longer rows still, aligned): one workgroup per row, two passes, no workspace; see softmax_stream.
+//  - generic tier (what is left: rows shorter than a vector, and unaligned rows beyond the co-resident tier): one
+//    workgroup per row, three scalar passes (max, sum, write).
 // The library allocates no device memory: the co-resident tier exchanges its chunk pairs through a static device
 // table whose entries carry a per-launch tag, so nothing has to be cleared between launches; launches recorded into a
 // HIP graph take fresh tags at every replay (see softmax_coop).
@@ -96,6 +98,28 @@ __device__ __forceinline__ void scale_store(float (&f)[NV][T::V], float s, void*
   }
 }
 
+// The sum of a vector's elements from the first `skip` on, in pairs.
+template <typename T>
+__device__ __forceinline__ float sum_vector(const float (&f)[T::V], int skip) {
+  float a[T::V];
+#pragma unroll
+  for (int i = 0; i < T::V; ++i) a[i] = i >= skip ? f[i] : 0.0f;
+#pragma unroll
+  for (int d = 1; d < T::V; d *= 2)
+#pragma unroll
+    for (int i = 0; i < T::V; i += 2 * d) a[i] += a[i + d];
+  return a[0];
+}
+
+// e / s within a correctly rounded division's last bit, from inv = 1 / s: the product and one step of its remainder for
+// fp32 results; for 16-bit results the product alone, whose fp32 ulp their rounding does not see.
+template <typename T>
+__device__ __forceinline__ float quotient(float e, float s, float inv) {
+  const float q = e * inv;
+  if constexpr (T::bytes == 2) return q;
+  else return __builtin_fmaf(__builtin_fmaf(-q, s, e), inv, q);
+}
+
 template <typename T, int WAVES, int NV, bool FULL, bool NTS>
 __device__ __forceinline__ void softmax_row(const Regs<NV>& r, void* y, long long row, long long nvec, int t,
                                             bool active, float* slots0, float* slots1, int wave, int first) {
@@ -138,6 +162,98 @@ __global__ void __launch_bounds__((WAVES < 4 ? 4 : WAVES) * 64)
     const long long rc = ra + step;
     load_vectors<G, NV, FULL, NTL>(a, x, (rc < rows ? rc : last) * nvec, nvec, t);
     softmax_row<T, WAVES, NV, FULL, NTS>(b, y, ra, nvec, t, ra < rows, slots[0], slots[1], wave, first);
+    base += step;
+    if (base >= rows) break;
+    ra = rc;
+  }
+}
+
+// Row tier for rows of any length from one vector up and any element alignment: the lanes' vectors start at the row's
+// first element, wherever it lies, and a vector that would pass the row's end is moved back to end with it. Its first
+// elements are then another lane's (the same bits, and the same results when they are stored twice), so the maximum takes
+// every loaded element and the sum leaves out the first `skip` of the vector; only the wave that holds the row's end
+// looks at that, and vectors that lie past the end for a whole wave are not worked on.
+// 8192 x 3001 bf16 55.5 us through the scalar kernel's three passes of 2-byte accesses, 16.9 us here.
+template <typename T, int WAVES, int NV>
+struct AnyRow {
+  static constexpr int G = WAVES * kWave, V = T::V;
+  int cols, t;
+  int first;  // the wave's first lane in the group: wave-uniform
+
+  __device__ __forceinline__ int start(int k) const { return (k * G + t) * V; }
+  __device__ __forceinline__ int offset(int k) const { return least(start(k), cols - V); }
+  __device__ __forceinline__ bool used(int k) const { return (k * G + first) * V < cols; }          // by some lane
+  __device__ __forceinline__ bool whole(int k) const { return (k * G + first + kWave) * V <= cols; }  // in every lane
+
+  __device__ __forceinline__ void load(Regs<NV>& r, const void* x, long long row) const {
+    const char* base = static_cast<const char*>(x) + row * cols * T::bytes;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) r.v[k] = load16_at<false>(base, (uint32_t)(offset(k) * T::bytes));
+  }
+
+  __device__ __forceinline__ void softmax(const Regs<NV>& r, void* y, long long row, bool active, float* slots0,
+                                          float* slots1, int wave, int first_wave) const {
+    float f[NV][V];
+    float m = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      unpack<T>(r.v[k], f[k]);
+#pragma unroll
+      for (int i = 0; i < V; ++i) m = fmaxf(m, f[k][i]);
+    }
+    m = group_reduce<WAVES>(m, OpMax{}, slots0, wave, first_wave);
+    float s[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      s[k] = 0.0f;
+      if (!used(k)) continue;
+#pragma unroll
+      for (int i = 0; i < V; ++i) f[k][i] = exp_below<T>(f[k][i] - m);
+      s[k] = whole(k) ? sum_vector<T>(f[k], 0) : sum_vector<T>(f[k], start(k) - offset(k));
+    }
+#pragma unroll
+    for (int d = 1; d < NV; d *= 2)  // in pairs, as within a vector: the error of a long chain of additions is kept out
+#pragma unroll
+      for (int k = 0; k < NV; k += 2 * d) s[k] += s[k + d];
+    const float sum = group_reduce<WAVES>(s[0], OpSum{}, slots1, wave, first_wave);
+    const float inv = 1.0f / sum;
+    char* base = static_cast<char*>(y) + row * cols * T::bytes;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      if (!active || start(k) >= cols) continue;
+#pragma unroll
+      for (int i = 0; i < V; ++i) f[k][i] = quotient<T>(f[k][i], sum, inv);
+      store16_at<true>(base, (uint32_t)(offset(k) * T::bytes), pack<T>(f[k]));
+    }
+  }
+};
+
+template <typename T, int WAVES, int NV>
+__global__ void __launch_bounds__((WAVES < 4 ? 4 : WAVES) * 64)
+    softmax_rows_any(const void* __restrict__ x, void* __restrict__ y, long long rows, int cols) {
+  constexpr int BW = WAVES < 4 ? 4 : WAVES;
+  constexpr int GROUPS = BW / WAVES;
+  __shared__ float slots[2][BW];
+  const int wave = __builtin_amdgcn_readfirstlane(wave_id());
+  const int first = (wave / WAVES) * WAVES;
+  const AnyRow<T, WAVES, NV> a{cols, (int)threadIdx.x - first * kWave, (wave - first) * kWave};
+  const long long step = (long long)gridDim.x * GROUPS;
+  long long base = (long long)blockIdx.x * GROUPS;
+  if (base >= rows) return;
+  const long long last = rows - 1;
+  long long ra = base + wave / WAVES;
+  Regs<NV> p, q;
+  a.load(p, x, ra < rows ? ra : last);
+  while (true) {
+    const long long rb = ra + step;
+    a.load(q, x, rb < rows ? rb : last);
+    a.softmax(p, y, ra, ra < rows, slots[0], slots[1], wave, first);
+    base += step;
+    if (base >= rows) break;
+    ra = rb;
+    const long long rc = ra + step;
+    a.load(p, x, rc < rows ? rc : last);
+    a.softmax(q, y, ra, ra < rows, slots[0], slots[1], wave, first);
     base += step;
     if (base >= rows) break;
     ra = rc;
@@ -266,10 +382,13 @@ __global__ void __launch_bounds__(256) softmax_coop_cell(int cell, unsigned iter
 
 // LOOP: some row group has more than one row (groups < rows); without it every workgroup takes one row, and the
 // kernel is compiled without the loop (which costs registers: fewer resident workgroups).
-template <typename T, int WAVES, int NV, bool NTL, bool NTS, bool LOOP>
+// ANY: rows of any length (nvec vectors, the last one partial) and element alignment. The row's last vector is moved
+// back to end with the row (AnyRow), its first `skip` elements being another lane's. fp32 chunks are held as x, and the
+// outputs are exp(x - M) / S with the division's remainder taken into account, as the row tier of such rows rounds them.
+template <typename T, int WAVES, int NV, bool NTL, bool NTS, bool LOOP, bool ANY>
 __global__ void __launch_bounds__(WAVES * 64)
-    softmax_coop(const void* __restrict__ x, void* __restrict__ y, long long rows, long long nvec, int chunks,
-                 int groups, unsigned tag0, int cell, unsigned wait_ticks) {
+    softmax_coop(const void* __restrict__ x, void* __restrict__ y, long long rows, long long nvec, long long cols,
+                 int chunks, int groups, unsigned tag0, int cell, unsigned wait_ticks) {
   constexpr int G = WAVES * kWave;
   // a captured launch (cell >= 0) reads its first tag from its cell, filled by the kernel node just before it
   if (cell >= 0) tag0 = __hip_atomic_load(&g_coop_cells[cell], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -282,10 +401,29 @@ __global__ void __launch_bounds__(WAVES * 64)
   const int first = c * (int)CH;  // < 2^31: at most kCoopMaxChunks chunks of CH vectors
   const int count = nvec - first < CH ? (int)(nvec - first) : (int)CH;
   const int t0 = (int)threadIdx.x;
+  const int wave0 = __builtin_amdgcn_readfirstlane(t0 & ~(kWave - 1));
   const int iters = (int)((rows - group + groups - 1) / groups);
   constexpr bool PREFETCH = LOOP && T::V == 8;
+  constexpr bool HOLD = !(ANY && T::bytes == 4);  // the chunk is held as exp(x - m)
   Regs<NV> next;  // PREFETCH: the next row's raw chunk, loaded during the wait
-  if constexpr (PREFETCH) load_vectors<G, NV, false, NTL>(next, x, group * nvec + first, count, t0);
+  // ANY: elements of the row from V before the chunk's first on; a vector past the row's last whole start is moved back to it
+  const int reach = (int)(cols - (long long)first * T::V);  // the chunk's first element to the row's end: >= 1
+  auto offset = [&](int k, int t) __attribute__((always_inline)) {
+    return (uint32_t)((least((k * G + t) * T::V, reach - T::V) + T::V) * T::bytes);
+  };
+  auto chunk_base = [&](long long row) __attribute__((always_inline)) {
+    return (row * cols + ((long long)first - 1) * T::V) * T::bytes;
+  };
+  auto load_chunk = [&](Regs<NV>& r, long long row, int t) __attribute__((always_inline)) {
+    if constexpr (ANY) {
+      const char* base = static_cast<const char*>(x) + chunk_base(row);
+#pragma unroll
+      for (int k = 0; k < NV; ++k) r.v[k] = load16_at<NTL>(base, offset(k, t));
+    } else {
+      load_vectors<G, NV, false, NTL>(r, x, row * nvec + first, count, t);
+    }
+  };
+  if constexpr (PREFETCH) load_chunk(next, group, t0);
   for (int it = 0; it < iters; ++it) {
     const long long row = group + (long long)it * groups;
     // the lane's offsets are formed anew each iteration (hoisted out of the loop they would hold NV 64-bit offsets in
@@ -293,10 +431,10 @@ __global__ void __launch_bounds__(WAVES * 64)
     int t = t0;
     if constexpr (LOOP) asm volatile("" : "+v"(t));
     const unsigned long long tag = (unsigned long long)coop_tag(tag0, it) << 32;
-    unsigned long long(*table)[2] = g_coop_pairs[it & 1] + (long long)group * chunks;
+    unsigned long long(*table)[2] = g_coop_pairs[it & 1] + group * chunks;
     Regs<NV> r;
     if constexpr (PREFETCH) r = next;
-    else load_vectors<G, NV, false, NTL>(r, x, row * nvec + first, count, t);
+    else load_chunk(r, row, t);
     float m = -INFINITY;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
@@ -308,24 +446,35 @@ __global__ void __launch_bounds__(WAVES * 64)
     }
     m = group_reduce<WAVES>(m, OpMax{}, slots[0], wave_id(), 0);
     // the registers take e = exp(x - m) (0 for an all -inf chunk) in place of x: one exp per element
-    float e[NV][T::V];
+    float e[HOLD ? NV : 1][T::V];
     float s = 0.0f;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
       float f[T::V];
       unpack<T>(r.v[k], f);
       const bool ok = k * G + t < count;
+      if constexpr (ANY) {
+        const int start = (k * G + t) * T::V;
 #pragma unroll
-      for (int i = 0; i < T::V; ++i) {
-        e[k][i] = ok && m != -INFINITY ? exp_to<T>(f[i] - m) : 0.0f;
-        s += e[k][i];
+        for (int i = 0; i < T::V; ++i) {
+          f[i] = m != -INFINITY ? exp_below<T>(f[i] - m) : 0.0f;
+          if constexpr (HOLD) e[k][i] = f[i];
+        }
+        s += (k * G + wave0 + kWave) * T::V <= reach ? sum_vector<T>(f, 0)
+                                                     : sum_vector<T>(f, start - least(start, reach - T::V));
+      } else {
+#pragma unroll
+        for (int i = 0; i < T::V; ++i) {
+          e[k][i] = ok && m != -INFINITY ? exp_to<T>(f[i] - m) : 0.0f;
+          s += e[k][i];
+        }
       }
     }
     s = group_reduce<WAVES>(s, OpSum{}, slots[1], wave_id(), 0);
     // x is now held as e: the next row's loads go out before the wait and the stores, into the freed registers (bf16,
     // whose raw chunk is half the size of e; for fp32 the two together would halve the resident workgroups)
     if constexpr (PREFETCH)
-      if (it + 1 < iters) load_vectors<G, NV, false, NTL>(next, x, (row + groups) * nvec + first, count, t);
+      if (it + 1 < iters) load_chunk(next, row + groups, t);
     if (t == 0) {  // an all -inf chunk publishes (-inf, 0) and contributes nothing to the merge
       __hip_atomic_store(&table[c][0], tag | __float_as_uint(m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __hip_atomic_store(&table[c][1], tag | __float_as_uint(s), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -385,10 +534,17 @@ __global__ void __launch_bounds__(WAVES * 64)
       float tm = -INFINITY, ts = 0.0f;
       for (long long i = t; i < nvec; i += G) {
         float f[T::V];
-        unpack<T>(load16<false>(x, row * nvec + i), f);
+        int skip = 0;
+        if constexpr (ANY) {
+          const int at = least((int)i * T::V, (int)cols - T::V);
+          unpack<T>(load16_at<false>(static_cast<const char*>(x) + row * cols * T::bytes, (uint32_t)(at * T::bytes)), f);
+          skip = (int)i * T::V - at;
+        } else {
+          unpack<T>(load16<false>(x, row * nvec + i), f);
+        }
 #pragma unroll
         for (int e = 0; e < T::V; ++e) {
-          if (f[e] == -INFINITY) continue;
+          if (e < skip || f[e] == -INFINITY) continue;
           if (f[e] > tm) {
             ts = ts * expf(tm - f[e]) + 1.0f;
             tm = f[e];
@@ -410,14 +566,22 @@ __global__ void __launch_bounds__(WAVES * 64)
     const float M = ms[0], S = ms[1];
     // y = e * exp(m - M) / S; an all -inf chunk (e = 0) gives 0, or NaN when the whole row is -inf (M = -inf)
     const float scale = m == -INFINITY ? (M == -INFINITY ? NAN : 0.0f) : expf(m - M) / S;
+    const float inv = 1.0f / S;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
       const int i = k * G + t;
       if (i < count) {
         float f[T::V];
+        if constexpr (HOLD) {
 #pragma unroll
-        for (int j = 0; j < T::V; ++j) f[j] = e[k][j] * scale;
-        store16<NTS>(y, row * nvec + first + i, pack<T>(f));
+          for (int j = 0; j < T::V; ++j) f[j] = e[k][j] * scale;
+        } else {
+          unpack<T>(r.v[k], f);
+#pragma unroll
+          for (int j = 0; j < T::V; ++j) f[j] = quotient<T>(exp_below<T>(f[j] - M), S, inv);
+        }
+        if constexpr (ANY) store16_at<NTS>(static_cast<char*>(y) + chunk_base(row), offset(k, t), pack<T>(f));
+        else store16<NTS>(y, row * nvec + first + i, pack<T>(f));
       }
     }
     if constexpr (!LOOP) break;
@@ -459,6 +623,8 @@ __global__ void __launch_bounds__(256)
 enum { kTuneWaves = 0, kTuneNv = 1, kTuneBlocksPerCu = 2, kTuneStreamWaves = 3, kTuneCoopGroups = 4, kTuneTier = 5,
        kTuneNtLoads = 6, kTuneWaitTicks = 7 };
 constexpr unsigned kCoopWaitTicks = 10000;  // 100 us: tens of times a row's arrival skew, a few launch lengths
+
+bool aligned_to(const void* p, int bytes) { return (reinterpret_cast<uintptr_t>(p) & (uintptr_t)(bytes - 1)) == 0; }
 
 int pow2_at_least(long long v) {
   int p = 1;
@@ -529,6 +695,49 @@ int launch_rows(int waves, int nv, const void* x, void* y, long long rows, long 
   }
 }
 
+// Rows of any length and element alignment (softmax_rows_any).
+template <typename T, int WAVES, int NV>
+int launch_any_k(const void* x, void* y, long long rows, int cols, hipStream_t stream) {
+  constexpr int BW = WAVES < 4 ? 4 : WAVES;
+  constexpr int GROUPS = BW / WAVES;
+  auto kern = softmax_rows_any<T, WAVES, NV>;
+  static int occ = 0;  // resident blocks per CU of this instantiation (idempotent cache)
+  if (occ <= 0) occ = blocks_per_cu(kern, BW * kWave);
+  int per_cu = rw_host::tune_get(kTuneBlocksPerCu);
+  // fp32 rows of four vectors a lane and more: the resident waves of launch_rows_k; otherwise about 24 waves per CU, whose
+  // loads are fewer or whose rows take more work per byte (8192 x 3001 fp32 as 4 waves x 4 vectors: 33.7 us with two
+  // blocks per CU, 34.8 with four; bf16 as 2 waves x 4 vectors: 17.3 with three, 16.9 with six; 65536 x 131 bf16: 23.5
+  // with two, 17.7 with six)
+  if (per_cu <= 0) per_cu = T::bytes == 4 && NV >= 4 ? (WAVES == 8 ? 2 : 8 / BW > 1 ? 8 / BW : 1) : (24 / BW > 1 ? 24 / BW : 1);
+  if (per_cu > occ) per_cu = occ;
+  const long long need = (rows + GROUPS - 1) / GROUPS;
+  long long grid = (long long)rw_host::device_cus() * per_cu;
+  if (grid > need) grid = need;
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(BW * kWave), 0, stream, x, y, rows, cols);
+  return (int)hipGetLastError();
+}
+
+template <typename T, int WAVES>
+int launch_any_w(int nv, const void* x, void* y, long long rows, int cols, hipStream_t stream) {
+  switch (nv) {
+    case 1: return launch_any_k<T, WAVES, 1>(x, y, rows, cols, stream);
+    case 2: return launch_any_k<T, WAVES, 2>(x, y, rows, cols, stream);
+    case 4: return launch_any_k<T, WAVES, 4>(x, y, rows, cols, stream);
+    default: return launch_any_k<T, WAVES, 8>(x, y, rows, cols, stream);
+  }
+}
+
+template <typename T>
+int launch_any(int waves, int nv, const void* x, void* y, long long rows, int cols, hipStream_t stream) {
+  switch (waves) {
+    case 1: return launch_any_w<T, 1>(nv, x, y, rows, cols, stream);
+    case 2: return launch_any_w<T, 2>(nv, x, y, rows, cols, stream);
+    case 4: return launch_any_w<T, 4>(nv, x, y, rows, cols, stream);
+    case 8: return launch_any_w<T, 8>(nv, x, y, rows, cols, stream);
+    default: return launch_any_w<T, 16>(nv, x, y, rows, cols, stream);
+  }
+}
+
 template <typename T, int WAVES>
 int launch_stream_w(const void* x, void* y, long long rows, long long nvec, hipStream_t stream) {
   long long grid = (long long)rw_host::device_cus() * (16 / WAVES > 1 ? 16 / WAVES : 1);
@@ -589,58 +798,67 @@ bool capturing(hipStream_t stream) {
   return status != hipStreamCaptureStatusNone;
 }
 
-// Co-resident tier: chunks of 4 waves x 64 lanes x 64 elements (16 fp32 or 8 bf16 vectors per lane), at most
-// kCoopMaxChunks per row; one row per workgroup when every row's chunks fit on the GPU at once, else row groups
-// walking several rows (a second instantiation: the loop costs registers). Returns 1, launching nothing, when one
-// row's chunks do not fit on the GPU at once.
-template <typename T, bool NTL>
-int launch_coop(const void* x, void* y, long long rows, long long nvec, hipStream_t stream) {
-  constexpr int WAVES = 4, NV1 = 64 / T::V, NVL = T::V == 4 ? 16 : 8;
-  constexpr long long CH1 = (long long)WAVES * kWave * NV1, CHL = (long long)WAVES * kWave * NVL;
-  auto one = softmax_coop<T, WAVES, NV1, NTL, true, false>;
-  auto loop = softmax_coop<T, WAVES, NVL, NTL, true, true>;
-  static int occ_one = 0, occ_loop = 0;  // resident blocks per CU of each instantiation (idempotent caches)
-  if (occ_one <= 0) occ_one = blocks_per_cu(one, WAVES * kWave);
-  if (occ_loop <= 0) occ_loop = blocks_per_cu(loop, WAVES * kWave);
-  const int want = rw_host::tune_get(kTuneCoopGroups);
-  const long long cus = rw_host::device_cus();
-  long long chunks = (nvec + CH1 - 1) / CH1;
-  long long slots = cus * occ_one;
-  if (slots > kCoopSlots) slots = kCoopSlots;
-  const bool single = chunks <= kCoopMaxChunks && rows * chunks <= slots && (want <= 0 || want >= rows);
-  if (!single) {
-    chunks = (nvec + CHL - 1) / CHL;
-    slots = cus * occ_loop;
-    if (slots > kCoopSlots) slots = kCoopSlots;
-    if (chunks > kCoopMaxChunks || chunks > slots) return 1;
-  }
-  long long groups = single ? rows : slots / chunks;
-  if (want > 0 && want < groups) groups = want;
-  if (groups > rows) groups = rows;
-  const long long iters = (rows + groups - 1) / groups;
+struct CoopLaunch {
+  const void* x;
+  void* y;
+  long long rows, nvec, cols;
+  hipStream_t stream;
+};
+constexpr int kCoopWaves = 4;
+
+// The launch of a co-resident kernel over `groups` row groups of `chunks` workgroups.
+template <typename Kernel>
+int launch_coop_k(Kernel kern, const CoopLaunch& a, long long chunks, long long groups) {
+  const long long iters = (a.rows + groups - 1) / groups;
   if (iters > 0x40000000LL) return 1;
   int dev = 0, err = (int)hipGetDevice(&dev);
   if (err != rw_host::kOk) return err;
   unsigned tag0 = 0;
   int cell = -1;
-  if (capturing(stream)) {
+  if (capturing(a.stream)) {
     // recorded into a graph: the tags are taken on the device at every replay, by a kernel node ahead of the launch
     cell = coop_cell(dev);
     if (cell < 0) return 1;
-    hipLaunchKernelGGL(softmax_coop_cell, dim3(1), dim3(256), 0, stream, cell, (unsigned)iters);
+    hipLaunchKernelGGL(softmax_coop_cell, dim3(1), dim3(256), 0, a.stream, cell, (unsigned)iters);
     err = (int)hipGetLastError();
   } else {
-    tag0 = coop_tags(dev, (unsigned)iters, stream, &err);
+    tag0 = coop_tags(dev, (unsigned)iters, a.stream, &err);
   }
   if (err != rw_host::kOk) return err;
   const int budget = rw_host::tune_get(kTuneWaitTicks);
   const unsigned ticks = budget > 0 ? (unsigned)budget : kCoopWaitTicks;
-  const dim3 grid((unsigned)(groups * chunks)), block(WAVES * kWave);
-  if (single)
-    hipLaunchKernelGGL(one, grid, block, 0, stream, x, y, rows, nvec, (int)chunks, (int)groups, tag0, cell, ticks);
-  else
-    hipLaunchKernelGGL(loop, grid, block, 0, stream, x, y, rows, nvec, (int)chunks, (int)groups, tag0, cell, ticks);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(groups * chunks)), dim3(kCoopWaves * kWave), 0, a.stream, a.x, a.y, a.rows,
+                     a.nvec, a.cols, (int)chunks, (int)groups, tag0, cell, ticks);
   return (int)hipGetLastError();
+}
+
+// Co-resident tier: chunks of 4 waves x 64 lanes x 64 elements (16 fp32 or 8 bf16 vectors per lane), at most
+// kCoopMaxChunks per row; one row per workgroup when every row's chunks fit on the GPU at once, else row groups
+// walking several rows (a second instantiation: the loop costs registers). Returns 1, launching nothing, when one
+// row's chunks do not fit on the GPU at once.
+template <typename T, bool NTL, bool ANY>
+int launch_coop(const CoopLaunch& a) {
+  constexpr int NV = 64 / T::V;
+  constexpr long long CH = (long long)kCoopWaves * kWave * NV;
+  auto one = softmax_coop<T, kCoopWaves, NV, NTL, true, false, ANY>;
+  auto loop = softmax_coop<T, kCoopWaves, NV, NTL, true, true, ANY>;
+  static int occ_one = 0, occ_loop = 0;  // resident blocks per CU of each instantiation (idempotent caches)
+  if (occ_one <= 0) occ_one = blocks_per_cu(one, kCoopWaves * kWave);
+  if (occ_loop <= 0) occ_loop = blocks_per_cu(loop, kCoopWaves * kWave);
+  const int want = rw_host::tune_get(kTuneCoopGroups);
+  const long long cus = rw_host::device_cus();
+  const long long chunks = (a.nvec + CH - 1) / CH;
+  long long slots = cus * occ_one;
+  if (slots > kCoopSlots) slots = kCoopSlots;
+  if (chunks > kCoopMaxChunks) return 1;
+  if (a.rows * chunks <= slots && (want <= 0 || want >= a.rows)) return launch_coop_k(one, a, chunks, a.rows);
+  slots = cus * occ_loop;
+  if (slots > kCoopSlots) slots = kCoopSlots;
+  if (chunks > slots) return 1;
+  long long groups = slots / chunks;
+  if (want > 0 && want < groups) groups = want;
+  if (groups > a.rows) groups = a.rows;
+  return launch_coop_k(loop, a, chunks, groups);
 }
 
 template <typename T>
@@ -655,9 +873,31 @@ template <typename T>
 int launch_typed(const void* x, void* y, long long rows, long long cols, hipStream_t stream) {
   const bool vec = cols % T::V == 0 && rw_host::aligned16(x) && rw_host::aligned16(y);
   const int tier = rw_host::tune_get(kTuneTier);
-  if (!vec || tier == 3) return launch_generic<T>(x, y, rows, cols, stream);
-  const long long nvec = cols / T::V;
+  const bool any = cols >= T::V && aligned_to(x, T::bytes) && aligned_to(y, T::bytes);
+  if (tier == 3 || !(vec || any)) return launch_generic<T>(x, y, rows, cols, stream);
+  const long long nvec = (cols + T::V - 1) / T::V;
+  if (!vec) {
+    const CoopLaunch coop{x, y, rows, nvec, cols, stream};
+    if (nvec > (long long)kMaxWaves * kWave * kMaxNv || tier == 4) {
+      const int rc = launch_coop<T, false, true>(coop);
+      return rc != 1 ? rc : launch_generic<T>(x, y, rows, cols, stream);
+    }
+    int waves = rw_host::tune_get(kTuneWaves), nv = rw_host::tune_get(kTuneNv);
+    auto pow2_to = [](int v, int most) { return v >= 1 && v <= most && (v & (v - 1)) == 0; };
+    if (!pow2_to(waves, kMaxWaves)) {
+      waves = pow2_at_least(((nvec + 3) / 4 + kWave - 1) / kWave);
+      // (fp32 rows for 16 waves of 4 vectors: 8 waves of 8 when there are rows for two such blocks per CU, 1024 x 16383
+      // 25.6 -> 24.3 us; bf16 600 x 32001 20.5 us as 16 x 4, 21.0 as 8 x 8)
+      if (T::bytes == 4 && waves == kMaxWaves && rows >= 2LL * rw_host::device_cus()) waves = kMaxWaves / 2;
+      waves = waves > kMaxWaves ? kMaxWaves : waves;
+    }
+    const int need = pow2_at_least((nvec + (long long)waves * kWave - 1) / ((long long)waves * kWave));
+    if (!pow2_to(nv, kMaxNv) || nv < need) nv = need;
+    if (nv > kMaxNv) return launch_generic<T>(x, y, rows, cols, stream);
+    return launch_any<T>(waves, nv, x, y, rows, (int)cols, stream);
+  }
   if (tier == 2) return launch_stream<T>(x, y, rows, nvec, stream);
+  const CoopLaunch coop{x, y, rows, nvec, cols, stream};
   const bool ntl = rw_host::tune_get(kTuneNtLoads) == 1;
   if (tier != 4 && nvec <= (long long)kMaxWaves * kWave * kMaxNv) {
     // Row tier: 4 vectors per lane as long as 16 waves suffice, then up to 8; except that rows of 513 to 1024
@@ -684,8 +924,7 @@ int launch_typed(const void* x, void* y, long long rows, long long cols, hipStre
                  : launch_rows<T, false>(waves, nv, x, y, rows, nvec, stream);
     }
   }
-  const int rc =
-      ntl ? launch_coop<T, true>(x, y, rows, nvec, stream) : launch_coop<T, false>(x, y, rows, nvec, stream);
+  const int rc = ntl ? launch_coop<T, true, false>(coop) : launch_coop<T, false, false>(coop);
   if (rc != 1) return rc;
   return launch_stream<T>(x, y, rows, nvec, stream);
 }

@@ -1,0 +1,133 @@
+"""Softmax rows of any length and element alignment on the vector tiers (softmax_rows_any and the co-resident tier's
+instantiation for such rows): the sizes where a row's last vector, a wave's share or a chunk begins to be used, base
+pointers off a 16-byte boundary, -inf elements and rows, against the oracle within the bounds of the softmax tests (fp32
+1e-5 relative, and 2^-147 below the normal range; bf16 1 ulp). The emulated cases run the kernels' source on the CPU
+between guard pages, so an access outside a row's tensor ends them; a stopped clock makes a wait end by its pairs only."""
+
+import ctypes
+import os
+
+import pytest
+import torch
+
+from _emu import build, run
+from _util import assert_rel, assert_ulp, bits16
+
+
+@pytest.fixture(scope="module")
+def emu_softmax(tmp_path_factory):
+    return build(tmp_path_factory.mktemp("emu_any_rows"), "softmax.hip", "emu_softmax.cpp")
+
+
+# cols around one vector, one wave's vectors, and the steps of the waves and of the vectors per lane
+EDGES = {0: [4, 5, 255, 257, 1023, 1025, 2047, 4097, 8191], 1: [8, 9, 511, 513, 2049, 3001, 4095, 8193]}
+
+
+@pytest.mark.parametrize("dtype,cols", [(d, c) for d in EDGES for c in EDGES[d]])
+def test_emulated_row_edges(emu_softmax, dtype, cols):
+    # offset 1: the buffers begin one element past a 16-byte boundary (and rows of a whole number of vectors are unaligned)
+    run(emu_softmax, [9, cols, dtype, 1, cols, 0, 0, 1, "special"])
+
+
+@pytest.mark.parametrize("dtype,waves,nv", [(0, 1, 8), (0, 2, 4), (0, 16, 1), (1, 1, 8), (1, 8, 2)])
+@pytest.mark.parametrize("env", [{}, {"EMU_WAVE_AHEAD": "1"}], ids=["lanes", "waves_ahead"])
+def test_emulated_row_shapes(emu_softmax, dtype, waves, nv, env):
+    run(emu_softmax, [21, 1999, dtype, 1, 5, waves, nv, 3, "randn"], env=dict(os.environ, **env))
+
+
+# rows, cols, dtype, row groups: chunks of 16384 elements and of a quarter of them (few rows), a last chunk of one vector
+COOP = [(2, 65539, 0, 0), (1, 4 * 4096 + 1, 0, 0), (3, 40001, 1, 0), (5, 16384 * 2 + 5, 0, 2), (5, 16384 * 3 - 1, 1, 3)]
+
+
+@pytest.mark.parametrize("rows,cols,dtype,groups", COOP)
+@pytest.mark.parametrize("pattern", ["randn", "special"])
+def test_emulated_coresident(emu_softmax, rows, cols, dtype, groups, pattern):
+    run(emu_softmax, [rows, cols, dtype, 4, 3, 0, groups, 1, pattern, 3], env=dict(os.environ, EMU_CLOCK_STOPPED="1"),
+        concurrent=True, weak=True, timeout=300)
+
+
+@pytest.mark.parametrize("rows,cols,dtype,groups", COOP)
+def test_emulated_coresident_fallback(emu_softmax, rows, cols, dtype, groups):
+    run(emu_softmax, [rows, cols, dtype, 4, 3, 0, groups, 1, "special", 2, 1])
+
+
+def _check(pkg, oracle, dev, rows, cols, dtype, offset=0, special=False):
+    print(f"[softmax any] {rows}x{cols} {dtype} offset {offset}", flush=True)
+    g = torch.Generator().manual_seed(rows * 131 + cols)
+    x = torch.randn(rows, cols, generator=g) * 3
+    if special:
+        x[0, ::3] = float("-inf")
+        x[-1] = float("-inf")
+    x = x.to(dtype)
+    n = rows * cols
+    # an in-place call at an offset: x and y are one buffer, whose other elements must stay as they were
+    buf = torch.full((n + 32,), 7.0, dtype=dtype)
+    buf[offset:offset + n] = x.view(-1)
+    d = buf.to(dev)
+    lib = pkg.candidate("softmax")._lib
+    at = d.data_ptr() + offset * d.element_size()
+    err = lib.launch(at, at, rows, cols, 0 if dtype == torch.float32 else 1, 256, 1024,
+                     ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert err == 0
+    out = d.cpu()
+    assert (out[:offset] == 7).all() and (out[offset + n:] == 7).all()
+    y = out[offset:offset + n].view(rows, cols)
+    if dtype == torch.float32:
+        assert_rel(y.numpy(), oracle.softmax(x.numpy(), "fp32"), 1e-5, f"{rows}x{cols}", 2.0 ** -147)
+    else:
+        assert_ulp(bits16(y), oracle.softmax(bits16(x), "bf16"), 1, f"{rows}x{cols}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("rows,cols", [(3, 8), (70, 9), (513, 255), (700, 513), (5, 2049), (300, 3001), (9, 8191),
+                                       (600, 16383), (3, 16384), (40, 20001), (2, 32767), (300, 20000), (5, 65535),
+                                       (3, 70001), (2, 262143), (70, 262143), (1, 1048576), (2, 1048577)])
+def test_gpu_rows(pkg, oracle, dev, dtype, rows, cols):
+    _check(pkg, oracle, dev, rows, cols, dtype, offset=1, special=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("offset", [0, 1, 2, 3, 5, 7, 8])
+def test_gpu_offsets(pkg, oracle, dev, dtype, offset):
+    for rows, cols in ((7, 1024), (7, 1027), (3, 40000)):
+        _check(pkg, oracle, dev, rows, cols, dtype, offset=offset)
+
+
+@pytest.mark.gpu
+def test_gpu_rows_on_two_streams(pkg, oracle, dev):
+    # long rows on two streams at once, over and over: each launch has pair slots of its own
+    g = torch.Generator().manual_seed(5)
+    xs = [torch.randn(24, 30000, generator=g) for _ in range(2)]
+    refs = [oracle.softmax(x.numpy(), "fp32") for x in xs]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    ds = [x.to(dev) for x in xs]
+    torch.cuda.synchronize()
+    ys = [[], []]
+    for _ in range(20):
+        for i in range(2):
+            with torch.cuda.stream(streams[i]):
+                ys[i].append(pkg.softmax(ds[i]))
+    torch.cuda.synchronize()
+    for i in range(2):
+        for y in ys[i]:
+            assert_rel(y.cpu().numpy(), refs[i], 1e-5, f"stream {i}", 2.0 ** -147)
+
+
+@pytest.mark.gpu
+def test_gpu_captured_rows_take_the_row_tier(pkg, oracle, dev):
+    # a captured launch of rows that an eager launch hands to the co-resident tier: replays on new values
+    x = torch.empty(8, 30000, device=dev)
+    pkg.softmax(x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = pkg.softmax(x)
+    for seed in range(3):
+        h = torch.randn(8, 30000, generator=torch.Generator().manual_seed(seed)) * 3
+        x.copy_(h)
+        pkg.softmax(x + 1)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_rel(y.cpu().numpy(), oracle.softmax(h.numpy(), "fp32"), 1e-5, f"replay {seed}", 2.0 ** -147)
