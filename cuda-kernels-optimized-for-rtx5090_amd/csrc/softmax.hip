@@ -388,7 +388,7 @@ __global__ void __launch_bounds__(256) softmax_coop_cell(int cell, unsigned iter
 template <typename T, int WAVES, int NV, bool NTL, bool NTS, bool LOOP, bool ANY>
 __global__ void __launch_bounds__(WAVES * 64)
     softmax_coop(const void* __restrict__ x, void* __restrict__ y, long long rows, long long nvec, long long cols,
-                 int chunks, int groups, unsigned tag0, int cell, unsigned wait_ticks) {
+                 int chunks, int groups, int slot0, unsigned tag0, int cell, unsigned wait_ticks) {
   constexpr int G = WAVES * kWave;
   // a captured launch (cell >= 0) reads its first tag from its cell, filled by the kernel node just before it
   if (cell >= 0) tag0 = __hip_atomic_load(&g_coop_cells[cell], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -431,7 +431,7 @@ __global__ void __launch_bounds__(WAVES * 64)
     int t = t0;
     if constexpr (LOOP) asm volatile("" : "+v"(t));
     const unsigned long long tag = (unsigned long long)coop_tag(tag0, it) << 32;
-    unsigned long long(*table)[2] = g_coop_pairs[it & 1] + group * chunks;
+    unsigned long long(*table)[2] = g_coop_pairs[it & 1] + slot0 + group * chunks;
     Regs<NV> r;
     if constexpr (PREFETCH) r = next;
     else load_chunk(r, row, t);
@@ -619,9 +619,9 @@ __global__ void __launch_bounds__(256)
 // resident blocks per CU, stream-tier waves, co-resident row groups (fewer forces more rows per workgroup), preferred
 // tier (1 row, 2 stream, 3 generic, 4 co-resident; a tier that cannot take the rows is passed over for the automatic
 // choice), non-temporal loads (1 on, 2 off), the co-resident tier's wait budget in 100 MHz ticks (tests force its
-// fallback with 1).
+// fallback with 1), the co-resident tier's vectors per lane (the longest chunks', half or a quarter of it).
 enum { kTuneWaves = 0, kTuneNv = 1, kTuneBlocksPerCu = 2, kTuneStreamWaves = 3, kTuneCoopGroups = 4, kTuneTier = 5,
-       kTuneNtLoads = 6, kTuneWaitTicks = 7 };
+       kTuneNtLoads = 6, kTuneWaitTicks = 7, kTuneCoopNv = 8 };
 constexpr unsigned kCoopWaitTicks = 10000;  // 100 us: tens of times a row's arrival skew, a few launch lengths
 
 bool aligned_to(const void* p, int bytes) { return (reinterpret_cast<uintptr_t>(p) & (uintptr_t)(bytes - 1)) == 0; }
@@ -775,6 +775,18 @@ unsigned coop_tags(int dev, unsigned n, hipStream_t stream, int* err) {
   return t;
 }
 
+// The first of a launch's n pair slots: launches take the table's slots in turn, so that launches that overlap on other
+// streams seldom meet in a slot (where their waits would fail).
+int coop_slots(int dev, int n) {
+  static std::mutex mu;
+  static int next[64];
+  std::lock_guard<std::mutex> lock(mu);
+  int& nx = next[dev & 63];
+  const int first = nx + n <= kCoopSlots ? nx : 0;
+  nx = first + n;
+  return first;
+}
+
 // A captured launch's tag cell: per device, cells are handed out once each, in capture order, and never reused (a
 // graph may be replayed at any time). Returns -1 when the device's cells are used up; such a launch takes the stream
 // tier, which keeps no state between launches.
@@ -798,6 +810,8 @@ bool capturing(hipStream_t stream) {
   return status != hipStreamCaptureStatusNone;
 }
 
+// Co-resident tier with one row per workgroup: chunks of 4 waves x 64 lanes x NV vectors, when every row's chunks fit on
+// the GPU at once. Returns 1, launching nothing, when they do not (or a row has more than kCoopMaxChunks of them).
 struct CoopLaunch {
   const void* x;
   void* y;
@@ -805,6 +819,8 @@ struct CoopLaunch {
   hipStream_t stream;
 };
 constexpr int kCoopWaves = 4;
+template <typename T> constexpr int kCoopFill = 4;
+template <> constexpr int kCoopFill<BF16> = 2;
 
 // The launch of a co-resident kernel over `groups` row groups of `chunks` workgroups.
 template <typename Kernel>
@@ -827,34 +843,56 @@ int launch_coop_k(Kernel kern, const CoopLaunch& a, long long chunks, long long 
   if (err != rw_host::kOk) return err;
   const int budget = rw_host::tune_get(kTuneWaitTicks);
   const unsigned ticks = budget > 0 ? (unsigned)budget : kCoopWaitTicks;
+  const int slot0 = coop_slots(dev, (int)(groups * chunks));
   hipLaunchKernelGGL(kern, dim3((unsigned)(groups * chunks)), dim3(kCoopWaves * kWave), 0, a.stream, a.x, a.y, a.rows,
-                     a.nvec, a.cols, (int)chunks, (int)groups, tag0, cell, ticks);
+                     a.nvec, a.cols, (int)chunks, (int)groups, slot0, tag0, cell, ticks);
   return (int)hipGetLastError();
 }
 
+template <typename T, int NV, bool NTL, bool ANY>
+int launch_coop_one(const CoopLaunch& a) {
+  auto one = softmax_coop<T, kCoopWaves, NV, NTL, true, false, ANY>;
+  static int occ = 0;  // resident blocks per CU (idempotent cache)
+  if (occ <= 0) occ = blocks_per_cu(one, kCoopWaves * kWave);
+  constexpr long long CH = (long long)kCoopWaves * kWave * NV;
+  const long long chunks = (a.nvec + CH - 1) / CH;
+  long long slots = (long long)rw_host::device_cus() * occ;
+  if (slots > kCoopSlots) slots = kCoopSlots;
+  if (chunks > kCoopMaxChunks || a.rows * chunks > slots) return 1;
+  return launch_coop_k(one, a, chunks, a.rows);
+}
+
 // Co-resident tier: chunks of 4 waves x 64 lanes x 64 elements (16 fp32 or 8 bf16 vectors per lane), at most
-// kCoopMaxChunks per row; one row per workgroup when every row's chunks fit on the GPU at once, else row groups
-// walking several rows (a second instantiation: the loop costs registers). Returns 1, launching nothing, when one
-// row's chunks do not fit on the GPU at once.
+// kCoopMaxChunks per row; shorter chunks (half or a quarter as long) when the rows are so few that the long ones would
+// leave CUs without a workgroup; row groups walking several rows (an instantiation of its own: the loop costs registers)
+// when the rows' chunks do not fit on the GPU at once. Returns 1, launching nothing, when one row's chunks do not fit.
 template <typename T, bool NTL, bool ANY>
-int launch_coop(const CoopLaunch& a) {
+int launch_coop(const CoopLaunch& a, bool single_only = false) {
   constexpr int NV = 64 / T::V;
   constexpr long long CH = (long long)kCoopWaves * kWave * NV;
-  auto one = softmax_coop<T, kCoopWaves, NV, NTL, true, false, ANY>;
-  auto loop = softmax_coop<T, kCoopWaves, NV, NTL, true, true, ANY>;
-  static int occ_one = 0, occ_loop = 0;  // resident blocks per CU of each instantiation (idempotent caches)
-  if (occ_one <= 0) occ_one = blocks_per_cu(one, kCoopWaves * kWave);
-  if (occ_loop <= 0) occ_loop = blocks_per_cu(loop, kCoopWaves * kWave);
   const int want = rw_host::tune_get(kTuneCoopGroups);
   const long long cus = rw_host::device_cus();
+  if (want <= 0 || want >= a.rows) {
+    int nv = rw_host::tune_get(kTuneCoopNv);
+    if (nv != NV && nv != NV / 2 && nv != NV / 4) {
+      nv = NV;
+      auto grid = [&](int n) { return a.rows * ((a.nvec + kCoopWaves * kWave * n - 1) / (kCoopWaves * kWave * n)); };
+      while (nv > NV / 4 && grid(nv) < kCoopFill<T> * cus) nv /= 2;
+    }
+    int rc = 1;  // a shape whose chunks are too many for the GPU or for a row takes the next longer chunks
+    if (nv == NV / 4) rc = launch_coop_one<T, NV / 4, NTL, ANY>(a);
+    if (rc == 1 && nv <= NV / 2) rc = launch_coop_one<T, NV / 2, NTL, ANY>(a);
+    if (rc == 1) rc = launch_coop_one<T, NV, NTL, ANY>(a);
+    if (rc != 1) return rc;
+  }
+  if (single_only) return 1;
+  auto loop = softmax_coop<T, kCoopWaves, NV, NTL, true, true, ANY>;
+  static int occ = 0;  // resident blocks per CU (idempotent cache)
+  if (occ <= 0) occ = blocks_per_cu(loop, kCoopWaves * kWave);
   const long long chunks = (a.nvec + CH - 1) / CH;
-  long long slots = cus * occ_one;
+  long long slots = cus * occ;
   if (slots > kCoopSlots) slots = kCoopSlots;
-  if (chunks > kCoopMaxChunks) return 1;
-  if (a.rows * chunks <= slots && (want <= 0 || want >= a.rows)) return launch_coop_k(one, a, chunks, a.rows);
-  slots = cus * occ_loop;
-  if (slots > kCoopSlots) slots = kCoopSlots;
-  if (chunks > slots) return 1;
+  if (chunks > kCoopMaxChunks || chunks > slots) return 1;
   long long groups = slots / chunks;
   if (want > 0 && want < groups) groups = want;
   if (groups > a.rows) groups = a.rows;
@@ -869,6 +907,21 @@ int launch_generic(const void* x, void* y, long long rows, long long cols, hipSt
   return (int)hipGetLastError();
 }
 
+// Rows that the row tier could hold but the co-resident tier takes faster: rows of more than 4096 vectors, which in the
+// row tier are 16 waves x 8 vectors with registers spilled (bf16 always: 600 x 40000 34 -> 19.5 us, 1024 x 50000 56 -> 46,
+// 1024 x 65536 51 -> 50; fp32 when every row's chunks are resident at once: 256 x 32768 15.0 -> 11.0, 512 x 20000
+// 19.0 -> 13.1, but 2048 x 32768 97 -> 103 in row groups), and rows of more than 2048 vectors when they are too few to
+// fill the GPU with one workgroup each (1 x 10000 fp32 4.5 -> 3.9, 16 x 32000 bf16 5.4 -> 4.2; 128 x 16384 fp32 6.0 either
+// way). A launch that is being captured stays in the row tier, which needs no second node and no tag cell.
+template <typename T>
+bool coop_instead_of_rows(long long rows, long long nvec, hipStream_t stream) {
+  const int w = rw_host::tune_get(kTuneWaves), n = rw_host::tune_get(kTuneNv);
+  auto pow2_to = [](int v, int most) { return v >= 0 && v <= most && (v & (v - 1)) == 0; };
+  const bool row_shape = (w || n) && pow2_to(w, kMaxWaves) && pow2_to(n, 16) && !(n == 16 && (w == 0 || w > 2));
+  if (rw_host::tune_get(kTuneTier) != 0 || row_shape) return false;  // a row-tier shape the kernels have is asked for
+  return (nvec > 4096 || (nvec > 2048 && rows <= 32)) && !capturing(stream);
+}
+
 template <typename T>
 int launch_typed(const void* x, void* y, long long rows, long long cols, hipStream_t stream) {
   const bool vec = cols % T::V == 0 && rw_host::aligned16(x) && rw_host::aligned16(y);
@@ -881,6 +934,10 @@ int launch_typed(const void* x, void* y, long long rows, long long cols, hipStre
     if (nvec > (long long)kMaxWaves * kWave * kMaxNv || tier == 4) {
       const int rc = launch_coop<T, false, true>(coop);
       return rc != 1 ? rc : launch_generic<T>(x, y, rows, cols, stream);
+    }
+    if (coop_instead_of_rows<T>(rows, nvec, stream)) {
+      const int rc = launch_coop<T, false, true>(coop, T::bytes == 4);
+      if (rc != 1) return rc;
     }
     int waves = rw_host::tune_get(kTuneWaves), nv = rw_host::tune_get(kTuneNv);
     auto pow2_to = [](int v, int most) { return v >= 1 && v <= most && (v & (v - 1)) == 0; };
@@ -898,6 +955,11 @@ int launch_typed(const void* x, void* y, long long rows, long long cols, hipStre
   }
   if (tier == 2) return launch_stream<T>(x, y, rows, nvec, stream);
   const CoopLaunch coop{x, y, rows, nvec, cols, stream};
+  if (nvec <= (long long)kMaxWaves * kWave * kMaxNv && coop_instead_of_rows<T>(rows, nvec, stream)) {
+    // fp32 rows keep the row tier's rounding (x held, the exponential taken again): the instantiation for any rows
+    const int rc = T::bytes == 4 ? launch_coop<T, false, true>(coop, true) : launch_coop<T, false, false>(coop);
+    if (rc != 1) return rc;
+  }
   const bool ntl = rw_host::tune_get(kTuneNtLoads) == 1;
   if (tier != 4 && nvec <= (long long)kMaxWaves * kWave * kMaxNv) {
     // Row tier: 4 vectors per lane as long as 16 waves suffice, then up to 8; except that rows of 513 to 1024
