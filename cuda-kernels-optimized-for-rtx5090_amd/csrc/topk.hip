@@ -2517,6 +2517,133 @@ __global__ void __launch_bounds__(kWave)
   if (lane_id() == 0) out[row] = drawn;
 }
 
+// ---- short rows ------------------------------------------------------------------------------------------------------
+
+// Rows of at most kShortCols columns (a router's experts, a reranker's candidates): topk_tile gives each a workgroup of
+// 256 lanes with 64 element registers apiece, nearly all of them padding. Here L lanes hold a row (16: four rows per
+// wave, reductions inside a DPP row; 64: one), E elements each, as words whose order is the composites' order:
+// fp32 (key << 32) | ~index, bf16 (the key's upper half << 16) | ~index in 32 bits, which makes an exchange of the lane's
+// sorting network one maximum and one minimum. A lane sorts its E words once; the row's next largest is then the
+// largest of the lanes' heads, k times over, and its lane steps on to its next word. The row's k words go through LDS,
+// from which the wave stores its rows' values and indices as one contiguous piece each. Bound by instruction issue (at
+// 16384 x 128 fp32, k = 8: 1.6 us of memory traffic).
+// 16384 x 128 fp32, k = 8: 69.2 us with topk_tile, 6.0 us here.
+constexpr int kShortCols = 1024;
+constexpr int kShortK = 64;
+
+template <typename T> struct ShortWord;
+template <> struct ShortWord<float> {
+  typedef u64 type;
+  static __device__ __forceinline__ u64 make(uint32_t u, int i) { return composite(u, (uint32_t)i); }
+  static __device__ __forceinline__ uint32_t value(u64 w) { return composite_bits(w); }
+  static __device__ __forceinline__ long long index(u64 w) { return composite_index(w); }
+};
+template <> struct ShortWord<uint16_t> {
+  typedef uint32_t type;
+  // (the index is below kShortCols, so that its complement's 16 bits are not 0 and no element is the empty word 0)
+  static __device__ __forceinline__ uint32_t make(uint32_t u, int i) {
+    const uint32_t key = key_of(u << 16);  // the lower half is 0 or, for a set sign, all ones
+    return (key & 0xffff0000u) | (0xffffu ^ (uint32_t)i);
+  }
+  static __device__ __forceinline__ uint32_t value(uint32_t w) { return bits_of(w | 0xffffu) >> 16 & 0xffffu; }
+  static __device__ __forceinline__ long long index(uint32_t w) { return (long long)(0xffffu ^ (w & 0xffffu)); }
+};
+
+// The largest of v over the L lanes of a row (16: a DPP row; 64: the wave); every lane returns its row's.
+template <int L>
+__device__ __forceinline__ uint32_t lanes_max(uint32_t v) {
+  if constexpr (L == kWave) return wave_ext32<true>(v);
+  auto step = [](uint32_t a, int b) { return a > (uint32_t)b ? a : (uint32_t)b; };
+  v = step(v, __builtin_amdgcn_update_dpp(0, (int)v, kDppXor1, 0xF, 0xF, false));
+  v = step(v, __builtin_amdgcn_update_dpp(0, (int)v, kDppXor2, 0xF, 0xF, false));
+  v = step(v, __builtin_amdgcn_update_dpp(0, (int)v, kDppHalfMirror, 0xF, 0xF, false));
+  return step(v, __builtin_amdgcn_update_dpp(0, (int)v, kDppMirror, 0xF, 0xF, false));
+}
+// Whether word w is the largest of its row's L lanes' (the words of a row are distinct, but for empty ones).
+template <int L>
+__device__ __forceinline__ bool leads(uint32_t w) { return w == lanes_max<L>(w); }
+template <int L>
+__device__ __forceinline__ bool leads(u64 w) {
+  const uint32_t hi = (uint32_t)(w >> 32), lo = (uint32_t)w;
+  const bool top = hi == lanes_max<L>(hi);
+  const uint32_t low = lanes_max<L>(top ? lo : 0u);  // (by every lane: a reduction takes no branch)
+  return top && lo == low;
+}
+
+template <typename T, bool VEC, int L, int E>
+__global__ void __launch_bounds__(kThreads)
+    topk_short(const T* __restrict__ x, void* __restrict__ values, long long* __restrict__ indices, long long rows,
+               int cols, int k) {
+  typedef ShortWord<T> Wd;
+  typedef typename Wd::type Word;
+  constexpr int R = kWave / L;  // rows per wave
+  constexpr int W = Fmt<T>::W;
+  __shared__ Word top[kWaves][R * kShortK];
+  const int wave = wave_id(), lane = lane_id(), l = lane & (L - 1), r = lane / L;
+  const long long row0 = ((long long)blockIdx.x * kWaves + wave) * R;
+  if (row0 >= rows) return;  // (no block barrier below: the waves are on their own)
+  const long long row = row0 + r < rows ? row0 + r : rows - 1;
+  const T* xr = x + row * cols;
+  Word c[E];
+  if constexpr (VEC) {
+    u32x4 v[E / W];
+#pragma unroll
+    for (int j = 0; j < E / W; ++j) {
+      const int e = (j * L + l) * W;
+      v[j] = load16<true>(e < cols ? (const void*)(xr + e) : (const void*)xr, 0);
+    }
+#pragma unroll
+    for (int j = 0; j < E / W; ++j)
+#pragma unroll
+      for (int i = 0; i < W; ++i) {
+        const int e = (j * L + l) * W + i;
+        const uint32_t u = sizeof(T) == 4 ? v[j][i * sizeof(T) / 4] : (v[j][i * sizeof(T) / 4] >> (16 * (i & 1))) & 0xffffu;
+        c[j * W + i] = e < cols ? Wd::make(u, e) : 0;
+      }
+  } else {
+    uint32_t u[E];
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+      const int e = j * L + l < cols ? j * L + l : 0;
+      if constexpr (sizeof(T) == 4) u[j] = reinterpret_cast<const uint32_t*>(xr)[e];
+      else u[j] = reinterpret_cast<const uint16_t*>(xr)[e];
+    }
+#pragma unroll
+    for (int j = 0; j < E; ++j) c[j] = j * L + l < cols ? Wd::make(u[j], j * L + l) : 0;
+  }
+  // Batcher's odd-even merge sort, the largest first
+#pragma unroll
+  for (int p = 1; p < E; p *= 2)
+#pragma unroll
+    for (int q = p; q >= 1; q /= 2)
+#pragma unroll
+      for (int j = q % p; j + q < E; j += 2 * q)
+#pragma unroll
+        for (int i = 0; i < q; ++i)
+          if (i + j + q < E && (i + j) / (2 * p) == (i + j + q) / (2 * p)) {
+            const Word a = c[i + j], b = c[i + j + q];
+            c[i + j] = a > b ? a : b;
+            c[i + j + q] = a > b ? b : a;
+          }
+  Word* out = top[wave];
+  for (int i = 0; i < k; ++i) {
+    if (leads<L>(c[0])) {
+      out[r * k + i] = c[0];
+#pragma unroll
+      for (int j = 0; j + 1 < E; ++j) c[j] = c[j + 1];
+      c[E - 1] = 0;
+    }
+  }
+  wave_lds_sync();  // the lanes' words before the wave's reads of other lanes' entries
+  const int n = (int)(rows - row0 < R ? rows - row0 : R) * k;
+  for (int j = lane; j < n; j += kWave) {
+    const Word w = out[j];
+    if constexpr (sizeof(T) == 4) static_cast<uint32_t*>(values)[row0 * k + j] = Wd::value(w);
+    else static_cast<uint16_t*>(values)[row0 * k + j] = (uint16_t)Wd::value(w);
+    indices[row0 * k + j] = Wd::index(w);
+  }
+}
+
 // ---- the naive tier ------------------------------------------------------------------------------------------------
 
 // The naive tier (the harness's "seed" column; launch() takes it when tuning slot 1 is 1): one workgroup per row
@@ -2557,8 +2684,9 @@ __global__ void __launch_bounds__(kThreads)
 
 // ---- host side ------------------------------------------------------------------------------------------------------
 
-// Tuning slots (0 = automatic): 0 resident workgroups per CU assumed by plan(); 1 the naive tier for launch() (1).
-enum { kTuneBlocksPerCu = 0, kTuneSeed = 1 };
+// Tuning slots (0 = automatic): 0 resident workgroups per CU assumed by plan(); 1 the naive tier for launch() (1); 2 the
+// short rows' kernel for every row it can hold (1) or for none (2).
+enum { kTuneBlocksPerCu = 0, kTuneSeed = 1, kTuneShort = 2 };
 
 // The chunking a launch of the caller's nchunks chunks of `chunk` columns actually runs, and the u64 slots of the
 // caller's work it uses (0 for unsplit rows). The result does not depend on the chunking, so the launch may join
@@ -2666,6 +2794,38 @@ int launch_chunks(const void* x, void* values, void* indices, void* work, void* 
   return (int)hipGetLastError();
 }
 
+// The short rows' launch: the fewest lanes and elements per lane that hold the row.
+template <typename T, bool VEC>
+int launch_short(const void* x, void* values, void* indices, long long rows, int cols, int k, hipStream_t stream) {
+  auto go = [&](auto kern, int per_wave) {
+    const long long per_block = (long long)kWaves * per_wave;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((rows + per_block - 1) / per_block)), dim3(kThreads), 0, stream,
+                       (const T*)x, values, (long long*)indices, rows, cols, k);
+    return (int)hipGetLastError();
+  };
+  if constexpr (sizeof(T) == 4)
+    if (cols <= 64) return go(topk_short<T, VEC, 16, 4>, 4);
+  if (cols <= 128) return go(topk_short<T, VEC, 16, 8>, 4);
+  if (cols <= 256) return go(topk_short<T, VEC, 16, 16>, 4);
+  if (cols <= 512) return go(topk_short<T, VEC, 64, 8>, 1);
+  return go(topk_short<T, VEC, 64, 16>, 1);
+}
+
+// Whether a plain launch takes the short rows' kernel: its time grows with k (a row's k steps are a serial chain of
+// about 0.1 us each, half of that for bf16's 32-bit words), so that for many columns and a large k the tile kernel is the
+// faster one until there are rows enough to hide the chain. Kernel times in us, tile kernel / this one:
+//   64 rows fp32: 128 columns k = 8 5.4 / 3.3, k = 64 10.2 / 8.9; 512 columns k = 32 5.6 / 7.4; 1024 columns k = 16
+//   5.5 / 6.4; bf16 512 columns k = 64 17.6 / 8.2, 1024 columns k = 32 6.0 / 6.6;
+//   16384 rows fp32: 128 columns k = 8 74.4 / 5.3; 512 columns k = 64 89 / 64; 1024 columns k = 32 77 / 50, k = 64 87 / 85.
+bool takes_short(long long rows, long long cols, int k, int dtype) {
+  const int want = rw_host::tune_get(kTuneShort);
+  if (cols > kShortCols || k > kShortK || want == 2) return false;
+  if (cols <= 128 || want == 1) return true;
+  if (rows >= 2048) return cols <= 512 || k <= 32;
+  if (dtype == 1) return cols <= 512 || k <= 16;
+  return cols <= 512 ? k <= 16 : k <= 8;
+}
+
 // Zeroes counters[0, n).
 __global__ void __launch_bounds__(kThreads) topk_zero(unsigned* __restrict__ counters, long long n) {
   for (long long i = (long long)blockIdx.x * kThreads + threadIdx.x; i < n; i += (long long)gridDim.x * kThreads)
@@ -2739,6 +2899,14 @@ int launch_impl(const void* x, void* values, void* indices, void* work, void* co
     return (int)hipGetLastError();
   }
   const int n = (int)nchunks;
+  if (!sa.out && takes_short(rows, cols, k, dtype)) {
+    const bool vec = cols % (dtype == 0 ? 4 : 8) == 0 && rw_host::aligned16(x);
+    if (dtype == 0)
+      return vec ? launch_short<float, true>(x, values, indices, rows, (int)cols, k, stream)
+                 : launch_short<float, false>(x, values, indices, rows, (int)cols, k, stream);
+    return vec ? launch_short<uint16_t, true>(x, values, indices, rows, (int)cols, k, stream)
+               : launch_short<uint16_t, false>(x, values, indices, rows, (int)cols, k, stream);
+  }
   if (dtype == 0) {
     if (cols % 4 == 0 && rw_host::aligned16(x))
       return launch_chunks<float, true>(x, values, indices, work, counters, rows, cols, chunk, n, k, sa, stream);
