@@ -17,7 +17,8 @@
 // Rows whose length is a multiple of 8 with 16-byte aligned x, y (and w) run the row kernel: a group of WAVES waves
 // holds one row in registers as NV 16-byte vectors per lane, reduces the sum over the group (DPP within a wave, LDS
 // slots across waves) and writes y from the registers; each lane holds the weight vectors of its columns once for all
-// rows. Workgroups are persistent and load their next row while they reduce and store the current one. Other rows use
+// rows. Workgroups are persistent and load their next row while they reduce and store the current one. Rows of at most 32
+// vectors share waves, four at a time (rmsnorm_short). Other rows use
 // a generic kernel (one workgroup per row, scalar accesses, two passes).
 #include <climits>
 #include <cmath>
@@ -161,6 +162,112 @@ __global__ void __launch_bounds__((WAVES < 4 ? 4 : WAVES) * 64)
   }
 }
 
+// Short rows (at most 32 vectors: the norm of each query or key head): 16 lanes hold a row, NV vectors per lane, and a
+// wave takes kShortSets sets of four rows at once, so that every lane holds data, and the row factor's chain (fp64 square
+// root and divisions, about 100 instructions) runs once per wave for all sixteen rows: the reduction over a row's lanes
+// first trades the four sets within each quad of lanes (two steps that halve the values a lane holds), which leaves set
+// q's sum in the lanes with lane % 4 == q, and every lane reads its sets' factors back from its quad. Waves are
+// persistent and load their next sixteen rows while they work on these; no LDS and no barrier. Bound by memory at 128
+// columns, by instruction issue below.
+// 163840 x 128 bf16 with a weight: 62.9 us as a wave per row with 16 of 64 lanes holding data, 16 us here.
+constexpr int kShortLanes = 16, kShortSets = 4;
+constexpr int kShortRows = kShortSets * (kWave / kShortLanes);  // a wave's rows per step
+constexpr int kDppRor4 = 0x124, kDppRor8 = 0x128;               // row_ror: rotation within a 16-lane row
+
+// The sum over each 16-lane row of every set's value, for the set lane % 4.
+__device__ __forceinline__ double short_sums(const double (&a)[kShortSets], int lane) {
+  static_assert(kShortSets == 4, "two trading steps");
+  const bool odd = lane & 1, upper = lane & 2;
+  const double e = (odd ? a[1] : a[0]) + dpp<kDppXor1>(odd ? a[0] : a[1]);
+  const double f = (odd ? a[3] : a[2]) + dpp<kDppXor1>(odd ? a[2] : a[3]);
+  double s = (upper ? f : e) + dpp<kDppXor2>(upper ? e : f);
+  s += dpp<kDppRor4>(s);
+  return s + dpp<kDppRor8>(s);
+}
+
+template <typename T, int NV, bool HAS_W>
+__global__ void __launch_bounds__(256)
+    rmsnorm_short(const void* x, const void* __restrict__ w, void* y, long long rows, int nvec, int cols, float eps) {
+  const int lane = lane_id(), l = lane & (kShortLanes - 1), sub = lane / kShortLanes;
+  const int per_block = (int)blockDim.x / kWave;
+  const long long wave = (long long)blockIdx.x * per_block + __builtin_amdgcn_readfirstlane(wave_id());
+  const long long step = (long long)gridDim.x * per_block * kShortRows;
+  u32x4 wr[HAS_W ? NV : 1];
+  if constexpr (HAS_W) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) wr[k] = load16<false>(w, least(k * kShortLanes + l, nvec - 1));
+  }
+  struct Step {
+    u32x4 v[kShortSets][NV];
+  };
+  // vector k of the lane's row of set u, of the sixteen rows from `first` on; a row past the last and a vector past the
+  // row's end are clamped (and not stored)
+  auto at = [&](long long first, int u, int k) __attribute__((always_inline)) {
+    const long long left = rows - 1 - first;
+    const int r = u * (kWave / kShortLanes) + sub;
+    return (uint32_t)((left < r ? (int)left : r) * nvec + least(k * kShortLanes + l, nvec - 1));
+  };
+  auto load = [&](Step& s, long long first) __attribute__((always_inline)) {
+    if (first >= rows) first = rows - 1;
+#pragma unroll
+    for (int u = 0; u < kShortSets; ++u)
+#pragma unroll
+      for (int k = 0; k < NV; ++k)
+        s.v[u][k] = load16<true>(static_cast<const char*>(x) + first * nvec * 16, at(first, u, k));
+  };
+  auto work = [&](const Step& s, long long first) __attribute__((always_inline)) {
+    double acc[kShortSets];
+#pragma unroll
+    for (int u = 0; u < kShortSets; ++u) {
+      acc[u] = 0.0;
+#pragma unroll
+      for (int k = 0; k < NV; ++k) {
+        float f[T::V];
+        unpack<T>(s.v[u][k], f);
+        double a = 0.0;
+#pragma unroll
+        for (int i = 0; i < T::V; ++i) a += (double)(f[i] * f[i]);
+        acc[u] += k * kShortLanes + l < nvec ? a : 0.0;
+      }
+    }
+    const float mine = row_inv<T>(short_sums(acc, lane), cols, eps);  // the factor of set lane % 4
+    const float inv[kShortSets] = {dpp<0x00>(mine), dpp<0x55>(mine), dpp<0xAA>(mine), dpp<0xFF>(mine)};
+#pragma unroll
+    for (int u = 0; u < kShortSets; ++u) {
+      const bool in = first + u * (kWave / kShortLanes) + sub < rows;
+#pragma unroll
+      for (int k = 0; k < NV; ++k) {
+        if (!in || k * kShortLanes + l >= nvec) continue;
+        float f[T::V];
+        unpack<T>(s.v[u][k], f);
+#pragma unroll
+        for (int e = 0; e < T::V; ++e) f[e] = f[e] * inv[u];
+        if constexpr (HAS_W) {
+          float g[T::V];
+          unpack<T>(wr[k], g);
+#pragma unroll
+          for (int e = 0; e < T::V; ++e) f[e] = g[e] * round_to<T>(f[e]);
+        }
+        store16<true>(static_cast<char*>(y) + first * nvec * 16, at(first, u, k), pack<T>(f));
+      }
+    }
+  };
+  long long first = wave * kShortRows;
+  if (first >= rows) return;
+  Step a, b;
+  load(a, first);
+  while (true) {
+    load(b, first + step);
+    work(a, first);
+    first += step;
+    if (first >= rows) break;
+    load(a, first + step);
+    work(b, first);
+    first += step;
+    if (first >= rows) break;
+  }
+}
+
 // Generic kernel: any row length and alignment, one 256-thread block per row (grid-strided), two scalar passes.
 // With RES, pass 1 writes h = T(x + residual) to res_out and pass 2 reads h back (the thread's own elements).
 template <typename T, bool HAS_W, bool RES>
@@ -234,8 +341,11 @@ int launch_k(const Args& a) {
   auto kern = rmsnorm_rows<T, WAVES, NV, FULL, HAS_W, RES, NTL, true>;
   static int occ = 0;
   if (occ <= 0) occ = blocks_per_cu(kern, BW * kWave);
-  // about 8 resident waves per CU by default (more waves only contend for the memory queues; measured on MI355X)
+  // about 8 resident waves per CU by default (more waves only contend for the memory queues; measured on MI355X); 32 for
+  // rows of at most 96 vectors, whose waves hold too little in flight (65536 rows bf16: 264 columns 28.4 -> 20.5 us, 512
+  // columns 31.0 -> 24.4, 640 columns 38.1 -> 31.9, but 1024 columns 44.9 -> 47.0)
   int per_cu = rw_host::tune_get(kTuneBlocksPerCu);
+  if (per_cu <= 0 && WAVES == 1 && a.nvec <= 96) per_cu = 8;
   if (per_cu <= 0) per_cu = 8 / BW > 1 ? 8 / BW : 1;
   if (per_cu > occ) per_cu = occ;
   const long long need = (a.rows + GROUPS - 1) / GROUPS;
@@ -275,6 +385,22 @@ int launch_rows(int waves, int nv, const Args& a) {
   }
 }
 
+template <typename T, int NV, bool HAS_W>
+int launch_short(const Args& a) {
+  auto kern = rmsnorm_short<T, NV, HAS_W>;
+  const long long cus = rw_host::device_cus();
+  const long long waves = (a.rows + kShortRows - 1) / kShortRows;
+  int per_cu = rw_host::tune_get(kTuneBlocksPerCu);
+  if (per_cu <= 0) per_cu = 6;  // 24 waves per CU (163840 x 128 bf16: 8 waves 17.0 us, 16 17.4, 24 15.8, 32 16.4)
+  // one wave per block until every CU has four: few rows then spread over the GPU
+  const int per_block = waves >= 4 * cus ? 4 : 1;
+  long long grid = (waves + per_block - 1) / per_block;
+  if (grid > cus * per_cu * 4 / per_block) grid = cus * per_cu * 4 / per_block;
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(per_block * kWave), 0, a.stream, a.x, a.w, a.y, a.rows,
+                     (int)a.nvec, a.cols, a.eps);
+  return (int)hipGetLastError();
+}
+
 template <typename T, bool HAS_W, bool RES = false>
 int launch_typed(const void* x, const void* w, void* y, long long rows, int cols, float eps, hipStream_t stream,
                  const void* res = nullptr, void* res_out = nullptr) {
@@ -291,6 +417,12 @@ int launch_typed(const void* x, const void* w, void* y, long long rows, int cols
     };
     auto auto_nv = [&](int w) { return pow2_at_least((nvec + (long long)w * kWave - 1) / ((long long)w * kWave)); };
     int waves = rw_host::tune_get(kTuneWaves), nv = rw_host::tune_get(kTuneNv);
+    if constexpr (!RES) {
+      if (nvec <= 2 * kShortLanes && waves <= 0 && nv <= 0) {  // 65536 x 256 bf16 28.0 -> 14.4 us, 65536 x 8 23.7 -> 4.6
+        const Args a{x, w, y, res, res_out, rows, nvec, cols, eps, stream};
+        return nvec <= kShortLanes ? launch_short<T, 1, HAS_W>(a) : launch_short<T, 2, HAS_W>(a);
+      }
+    }
     if (waves <= 0) waves = auto_waves();
     if (nv <= 0) nv = auto_nv(waves);
     // a tuned shape the row kernel does not have (launch_rows below) is ignored: the automatic choice runs

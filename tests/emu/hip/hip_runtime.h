@@ -305,6 +305,8 @@ inline int readfirstlane(int v, int line) {
 // the lane that lane l reads under DPP control ctrl, or -1 where the source is out of range
 inline int dpp_src(int l, int ctrl, int line) {
   if (ctrl > 0x110 && ctrl < 0x120) return (l & 15) >= ctrl - 0x110 ? l - (ctrl - 0x110) : -1;  // row_shr:n
+  if (ctrl >= 0 && ctrl < 0x100) return (l & ~3) | ((ctrl >> (2 * (l & 3))) & 3);             // quad_perm
+  if (ctrl > 0x120 && ctrl < 0x130) return (l & ~15) | ((l - (ctrl - 0x120)) & 15);           // row_ror:n
   switch (ctrl) {
     case 0xB1: return l ^ 1;
     case 0x4E: return l ^ 2;
