@@ -2745,6 +2745,12 @@ enum { kTuneBlocksPerCu = 0, kTuneSeed = 1, kTuneShort = 2 };
 //    16.8 -> 10.3 us, 32 x 128256 19.6 -> 12.2 us, 16 x 32000 11.5 -> 9.9 us; at k = 1: 32 x 128256 10.2 -> 6.9 us,
 //    4 x 128256 6.3 -> 5.4 us, 16 x 32000 6.4 -> 4.8 us; at k = 300, from chunks of 16 k = 4800 columns: 8 x 128256
 //    26.8 -> 13.1 us, 32 x 128256 33.6 -> 15.2 us.
+//  - the chunks of a row are then made equal: full chunks and a remainder leave a last chunk whose few lanes with
+//    elements give it no bound (k <= 64: the exact re-push path; k > 64: it admits nearly everything). bf16: 64 x 50000
+//    k = 50 37.5 -> 10.4 us, 16 x 132352 k = 50 48 -> 10.8, 92 x 70753 k = 1024 64 -> 24; fp32: 143 x 33536 k = 50
+//    25.2 -> 11.5 us, 128 x 128256 unchanged. Not when that makes more register tiles in all (300 x 167148 fp32 in
+//    chunks of four tiles, k = 1024: 70.5 -> 75.5), nor when the last chunk is nearly as long as the others, nor for k > 64 below 10 k columns (a chunk's bound needs the group
+//    maxima of that many: 276 x 17664 fp32, k = 1024 as two chunks of 8832: 24 -> 50).
 //  - 1 < k <= 64: a row of two chunks within two register tiles is taken whole by one workgroup, tile after tile,
 //    when there are at least as many rows as CUs (512 x 32000 fp32 at k = 50: 19.2 -> 17.6 us on MI355X; the chunks'
 //    hand-off and merge cost more than the second tile's wait, while one workgroup per row still fills the GPU).
@@ -2759,6 +2765,22 @@ struct Chunking {
   long long slots;
 };
 constexpr long long kShortChunk = 8192;
+
+// A split row's chunks made equal (but for rounding to whole vectors) when the last one is under three quarters of the
+// others, no more of them than before and with no more register tiles in all, unless they would be shorter than
+// `least_chunk`.
+void even_chunks(long long cols, long long& chunk, int& nchunks, long long least_chunk) {
+  if (nchunks <= 1 || 4 * (cols - (nchunks - 1) * chunk) >= 3 * chunk) return;
+  const long long tile = (long long)kThreads * kTileE;
+  auto tiles = [&](long long len) { return (len + tile - 1) / tile; };
+  const long long even = ((cols + nchunks - 1) / nchunks + 7) / 8 * 8;
+  const int n = (int)((cols + even - 1) / even);
+  const long long before = (nchunks - 1) * tiles(chunk) + tiles(cols - (nchunks - 1) * chunk);
+  const long long after = (n - 1) * tiles(even) + tiles(cols - (n - 1) * even);
+  if (even < least_chunk || after > before) return;
+  chunk = even;
+  nchunks = n;
+}
 
 Chunking chunking(long long rows, long long cols, long long chunk, int nchunks, int k, int width) {
   const long long tile = (long long)kThreads * kTileE;
@@ -2776,6 +2798,7 @@ Chunking chunking(long long rows, long long cols, long long chunk, int nchunks, 
     }
     const long long tail = cols - (long long)(nchunks - 1) * chunk;
     if (nchunks > 1 && tail < (long long)kThreads * width && chunk + tail <= (long long)kThreads * kTileE) --nchunks;
+    even_chunks(cols, chunk, nchunks, 0);
     if (k > 1 && nchunks == 2 && cols <= 2LL * kThreads * kTileE && rows >= rw_host::device_cus()) {
       chunk = cols;
       nchunks = 1;
@@ -2789,6 +2812,7 @@ Chunking chunking(long long rows, long long cols, long long chunk, int nchunks, 
       chunk = want < cols ? (want + 7) / 8 * 8 : cols;
       nchunks = (int)((cols + chunk - 1) / chunk);
     }
+    even_chunks(cols, chunk, nchunks, 10LL * k);
   }
   return Chunking{chunk, nchunks, nchunks > 1 ? rows * nchunks * (k == 1 ? 1LL : (long long)k) : 0LL};
 }

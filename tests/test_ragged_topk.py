@@ -74,3 +74,22 @@ def test_gpu_rows_off_a_vector_boundary(pkg, oracle, dev, dtype):
         v, i = pkg.topk(at, 50)
         assert np.array_equal(i.cpu().numpy(), ri)
         assert np.array_equal(v.cpu().numpy() if name == "fp32" else bits16(v), rv)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("rows,cols", [(64, 50000), (39, 17920), (16, 132352), (143, 33536), (300, 17152), (2, 41984),
+                                       (4, 17152), (90, 37070), (300, 49160)])
+def test_gpu_rows_whose_last_chunk_would_be_short(pkg, oracle, dev, dtype, rows, cols):
+    # full chunks of 16384 (or 8192) columns would leave a short one at the end; the launch makes the chunks equal
+    g = torch.Generator().manual_seed(rows + cols)
+    x = (torch.randn(rows, cols, generator=g) * 2).to(dtype)
+    x[:, -1] = 11.0
+    raw = x.numpy() if dtype == torch.float32 else bits16(x)
+    name = "fp32" if dtype == torch.float32 else "bf16"
+    for k in (1, 8, 64, 100, 1024):
+        print(f"[topk chunks] {rows}x{cols} {name} k={k}", flush=True)
+        v, i = pkg.topk(x.to(dev), k)
+        rv, ri = oracle.topk(raw, k, name)
+        got, ref = (v.cpu().numpy().view(np.uint32), rv.view(np.uint32)) if name == "fp32" else (bits16(v), rv)
+        assert np.array_equal(i.cpu().numpy(), ri) and np.array_equal(got, ref)
