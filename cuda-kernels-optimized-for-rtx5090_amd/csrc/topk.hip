@@ -816,14 +816,6 @@ struct Tile {
     b0 = t0;
     b1 = end - t0 > NT * EPL ? t0 + NT * EPL : end;
     lane0 = b0 + (int)threadIdx.x * W;
-    auto vector = [&](int e0) __attribute__((always_inline)) {
-      if constexpr (VEC) {
-        return load16<true>(e0 < b1 ? (const void*)(row + e0) : (const void*)&g_sentinel_vec, 0);
-      } else {
-        const int at = least(e0, b1 - W);
-        return load16_at<true>(e0 < b1 ? (const void*)(row + at) : (const void*)&g_sentinel_vec, 0);
-      }
-    };
     if constexpr (!VEC) {
       if (b1 < W) {  // a row shorter than a vector
         load_few(row);
@@ -838,13 +830,19 @@ struct Tile {
         if constexpr (VEC) r[v] = load16<true>(at, 0);
         else r[v] = load16_at<true>(at, 0);
       }
-      r[NV - 1] = vector(first(NV - 1));
+      r[NV - 1] = load_vector(row, first(NV - 1));
     } else {
 #pragma unroll
-      for (int v = 0; v < NV; ++v) r[v] = vector(first(v));
+      for (int v = 0; v < NV; ++v) r[v] = load_vector(row, first(v));
     }
     if constexpr (!VEC) set_tail();
     asm volatile("" ::: "memory");  // issue the loads here: the scheduler must not sink them past later work
+  }
+
+  // The vector of elements from e0 on, or the sentinel past the tile's end.
+  __device__ __forceinline__ u32x4 load_vector(const T* row, int e0) const {
+    if constexpr (VEC) return load16<true>(e0 < b1 ? (const void*)(row + e0) : (const void*)&g_sentinel_vec, 0);
+    else return load16_at<true>(e0 < b1 ? (const void*)(row + least(e0, b1 - W)) : (const void*)&g_sentinel_vec, 0);
   }
 
   // The row's b1 < W elements, in vector 0 of lane 0.
