@@ -17,11 +17,13 @@
 // Rows whose length is a multiple of 8 with 16-byte aligned x, y (and w) run the row kernel: a group of WAVES waves
 // holds one row in registers as NV 16-byte vectors per lane, reduces the sum over the group (DPP within a wave, LDS
 // slots across waves) and writes y from the registers; each lane holds the weight vectors of its columns once for all
-// rows. Workgroups are persistent and load their next row while they reduce and store the current one. Rows of at most 32
-// vectors share waves, four at a time (rmsnorm_short). Other rows use
-// a generic kernel (one workgroup per row, scalar accesses, two passes).
+// rows. Workgroups are persistent and load their next row while they reduce and store the current one. Rows of any other
+// length from 8 columns up, or otherwise aligned, run the same kernel with element-aligned vectors (Form kAny); aligned
+// rows of at most 32 vectors share waves, four at a time (rmsnorm_short). What is left (rows of fewer than 8 columns, or
+// longer than 16 waves hold) takes a generic kernel (one workgroup per row, scalar accesses, two passes).
 #include <climits>
 #include <cmath>
+#include <type_traits>
 
 #include "host.hpp"
 #include "rowwise.hpp"
@@ -38,14 +40,47 @@ struct Regs {
   u32x4 v[NV];
 };
 
-template <int G, int NV, bool FULL, bool NTL>
-__device__ __forceinline__ void load_vectors(Regs<NV>& r, const void* base, long long first, long long count, int t) {
-#pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    long long i = (long long)k * G + t;
-    if constexpr (!FULL) i = i < count ? i : count - 1;
-    r.v[k] = load16<NTL>(base, first + i);
+// How rows lie under a group's vectors: kFull, as many aligned vectors as the group holds; kPart, fewer; kAny, rows of any
+// length (at least a vector) at any element alignment: the row's last vector is moved back to end with the row, its first
+// elements being another lane's (the same bits, and the same results when they are stored twice).
+enum Form { kPart = 0, kFull = 1, kAny = 2 };
+
+// The lane's place in its rows. Lane t of the group's G holds vectors t, t + G, ..., clamped into the row.
+template <int FORM, int G>
+struct Place {
+  static constexpr int V = 8;
+  long long nvec;
+  int cols, t;
+  int wave0;  // the wave's first lane in the group: wave-uniform
+  // whether vector k holds elements of the row in some lane of the wave, and (kAny) whole vectors of them in every lane
+  __device__ __forceinline__ bool used(int k) const { return FORM == kFull || (long long)k * G + wave0 < nvec; }
+  __device__ __forceinline__ bool whole(int k) const { return (k * G + wave0 + kWave) * V <= cols; }
+  __device__ __forceinline__ int start(int k) const { return (k * G + t) * V; }  // vector k's first element
+  __device__ __forceinline__ bool in(int k) const { return FORM == kFull || (FORM == kAny ? start(k) < cols : (long long)k * G + t < nvec); }
+  __device__ __forceinline__ uint32_t any_at(int k) const { return (uint32_t)least(start(k), cols - V) * 2u; }  // bytes
+  __device__ __forceinline__ int skip(int k) const { return start(k) - least(start(k), cols - V); }  // another lane's elements
+
+  template <bool NTL>
+  __device__ __forceinline__ u32x4 load(const void* base, long long row, int k) const {
+    if constexpr (FORM == kAny) {
+      return load16_at<NTL>(static_cast<const char*>(base) + row * cols * 2, any_at(k));
+    } else {
+      long long i = (long long)k * G + t;
+      if constexpr (FORM == kPart) i = i < nvec ? i : nvec - 1;
+      return load16<NTL>(base, row * nvec + i);
+    }
   }
+  template <bool NTS>
+  __device__ __forceinline__ void store(void* base, long long row, int k, const u32x4& v) const {
+    if constexpr (FORM == kAny) store16_at<NTS>(static_cast<char*>(base) + row * cols * 2, any_at(k), v);
+    else store16<NTS>(base, row * nvec + (long long)k * G + t, v);
+  }
+};
+
+template <int FORM, int G, int NV, bool NTL>
+__device__ __forceinline__ void load_vectors(Regs<NV>& r, const void* base, long long row, const Place<FORM, G>& at) {
+#pragma unroll
+  for (int k = 0; k < NV; ++k) r.v[k] = at.template load<NTL>(base, row, k);
 }
 
 // inv from the exact sum of squares: fp32 mean and eps as the reference, rsqrt correctly rounded to fp32, then to T.
@@ -57,56 +92,78 @@ __device__ __forceinline__ float row_inv(double sum, int cols, float eps) {
   return round_to<T>(inv32);
 }
 
-template <typename T, int WAVES, int NV, bool FULL, bool HAS_W, bool NTS>
-__device__ __forceinline__ void norm_row(const Regs<NV>& r, const Regs<NV>& w, void* y, long long row,
-                                         long long nvec, int cols, float eps, int t, bool active, double* slots,
+// Keeps a product apart from its rounding to fp16 (fused into one mixed-precision multiply-add with +0, a product of -0
+// comes out as +0).
+template <typename T>
+__device__ __forceinline__ void apart(float& v) {
+  if constexpr (std::is_same<T, F16>::value) asm volatile("" : "+v"(v));
+}
+
+template <typename T, int WAVES, int NV, int FORM, bool HAS_W, bool RES, bool NTS>
+__device__ __forceinline__ void norm_row(const Regs<NV>& r, const Regs<NV>& w, void* y, void* res_out, long long row,
+                                         const Place<FORM, WAVES * kWave>& at, float eps, bool active, double* slots,
                                          int wave, int first) {
-  constexpr int G = WAVES * kWave;
   double acc = 0.0;
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
+    // (kPart with a residual measured 1% slower with the skip at 16384 x 5120; without one 64.2 -> 62.3 us)
+    if (!(FORM == kPart && RES) && !at.used(k)) continue;
     float f[T::V];
     unpack<T>(r.v[k], f);
-    const bool ok = FULL || (long long)k * G + t < nvec;
+    if (FORM == kAny && !at.whole(k)) {
+      const int skip = at.skip(k);
 #pragma unroll
-    for (int i = 0; i < T::V; ++i) acc += ok ? (double)(f[i] * f[i]) : 0.0;
+      for (int i = 0; i < T::V; ++i) acc += i >= skip ? (double)(f[i] * f[i]) : 0.0;
+    } else {
+      const bool ok = FORM == kAny || at.in(k);
+#pragma unroll
+      for (int i = 0; i < T::V; ++i) acc += ok ? (double)(f[i] * f[i]) : 0.0;
+    }
   }
   acc = group_reduce<WAVES>(acc, OpSum{}, slots, wave, first);
-  const float inv = row_inv<T>(acc, cols, eps);
+  const float inv = row_inv<T>(acc, at.cols, eps);
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
-    const long long i = (long long)k * G + t;
-    if (active && (FULL || i < nvec)) {
+    if (active && at.in(k)) {
+      // (kAny: h is stored only here, behind the reduction, which every wave reaches with its vectors loaded: in place, a
+      // vector moved back at the row's end reads elements that another wave writes)
+      if constexpr (RES && FORM == kAny) at.template store<NTS>(res_out, row, k, r.v[k]);
       float f[T::V];
       unpack<T>(r.v[k], f);
 #pragma unroll
-      for (int e = 0; e < T::V; ++e) f[e] = f[e] * inv;
+      for (int e = 0; e < T::V; ++e) {
+        f[e] = f[e] * inv;
+        if constexpr (FORM == kAny) apart<T>(f[e]);
+      }
       if constexpr (HAS_W) {
         float g[T::V];
         unpack<T>(w.v[k], g);
 #pragma unroll
-        for (int e = 0; e < T::V; ++e) f[e] = g[e] * round_to<T>(f[e]);
+        for (int e = 0; e < T::V; ++e) {
+          f[e] = g[e] * round_to<T>(f[e]);
+          if constexpr (FORM == kAny) apart<T>(f[e]);
+        }
       }
-      store16<NTS>(y, row * nvec + i, pack<T>(f));
+      at.template store<NTS>(y, row, k, pack<T>(f));
     }
   }
 }
 
 // Fused residual: r becomes h = T(x + residual), which is written to res_out (the lane's own vectors: res_out may be
-// residual, and y may be x).
-template <typename T, int G, int NV, bool FULL, bool NTS>
+// residual, and y may be x; kAny rows are written by norm_row).
+template <typename T, int FORM, int G, int NV, bool NTS>
 __device__ __forceinline__ void add_residual(Regs<NV>& r, const Regs<NV>& res, void* res_out, long long row,
-                                             long long nvec, int t, bool active) {
+                                             const Place<FORM, G>& at, bool active) {
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
+    if (FORM == kAny && !at.used(k)) continue;
     float a[T::V], b[T::V];
     unpack<T>(r.v[k], a);
     unpack<T>(res.v[k], b);
 #pragma unroll
     for (int e = 0; e < T::V; ++e) a[e] = a[e] + b[e];
     r.v[k] = pack<T>(a);
-    const long long i = (long long)k * G + t;
-    if (active && (FULL || i < nvec)) store16<NTS>(res_out, row * nvec + i, r.v[k]);
+    if (FORM != kAny && active && at.in(k)) at.template store<NTS>(res_out, row, k, r.v[k]);
   }
 }
 
@@ -116,7 +173,7 @@ __device__ __forceinline__ void add_residual(Regs<NV>& r, const Regs<NV>& res, v
 // With RES the group also loads the residual rows, forms h = T(x + residual) and writes it to res_out before the
 // normalisation (x and y, and residual and res_out, may be the same buffers: a lane reads its vectors before it
 // writes them).
-template <typename T, int WAVES, int NV, bool FULL, bool HAS_W, bool RES, bool NTL, bool NTS>
+template <typename T, int WAVES, int NV, int FORM, bool HAS_W, bool RES, bool NTL, bool NTS>
 __global__ void __launch_bounds__((WAVES < 4 ? 4 : WAVES) * 64)
     rmsnorm_rows(const void* x, const void* res, const void* __restrict__ w, void* y, void* res_out, long long rows,
                  long long nvec, int cols, float eps) {
@@ -124,38 +181,38 @@ __global__ void __launch_bounds__((WAVES < 4 ? 4 : WAVES) * 64)
   constexpr int GROUPS = BW / WAVES;
   constexpr int G = WAVES * kWave;
   __shared__ double slots[2][BW];
-  const int wave = wave_id();
+  const int wave = FORM == kAny || (FORM == kPart && !RES) ? __builtin_amdgcn_readfirstlane(wave_id()) : wave_id();
   const int first = (wave / WAVES) * WAVES;
-  const int t = (int)threadIdx.x - first * kWave;
+  const Place<FORM, G> at{nvec, cols, (int)threadIdx.x - first * kWave, (wave - first) * kWave};
   const long long step = (long long)gridDim.x * GROUPS;
   long long base = (long long)blockIdx.x * GROUPS;
   if (base >= rows) return;
   const long long last = rows - 1;
   Regs<NV> wr;
-  if constexpr (HAS_W) load_vectors<G, NV, FULL, false>(wr, w, 0, nvec, t);
+  if constexpr (HAS_W) load_vectors<FORM, G, NV, false>(wr, w, 0, at);
   long long ra = base + wave / WAVES;
   Regs<NV> a, b;
   Regs<RES ? NV : 1> ea, eb;  // residual rows
-  load_vectors<G, NV, FULL, NTL>(a, x, (ra < rows ? ra : last) * nvec, nvec, t);
-  if constexpr (RES) load_vectors<G, NV, FULL, NTL>(ea, res, (ra < rows ? ra : last) * nvec, nvec, t);
+  load_vectors<FORM, G, NV, NTL>(a, x, ra < rows ? ra : last, at);
+  if constexpr (RES) load_vectors<FORM, G, NV, NTL>(ea, res, ra < rows ? ra : last, at);
   while (true) {
     const long long rb = ra + step;
-    load_vectors<G, NV, FULL, NTL>(b, x, (rb < rows ? rb : last) * nvec, nvec, t);
+    load_vectors<FORM, G, NV, NTL>(b, x, rb < rows ? rb : last, at);
     if constexpr (RES) {
-      load_vectors<G, NV, FULL, NTL>(eb, res, (rb < rows ? rb : last) * nvec, nvec, t);
-      add_residual<T, G, NV, FULL, NTS>(a, ea, res_out, ra, nvec, t, ra < rows);
+      load_vectors<FORM, G, NV, NTL>(eb, res, rb < rows ? rb : last, at);
+      add_residual<T, FORM, G, NV, NTS>(a, ea, res_out, ra, at, ra < rows);
     }
-    norm_row<T, WAVES, NV, FULL, HAS_W, NTS>(a, wr, y, ra, nvec, cols, eps, t, ra < rows, slots[0], wave, first);
+    norm_row<T, WAVES, NV, FORM, HAS_W, RES, NTS>(a, wr, y, res_out, ra, at, eps, ra < rows, slots[0], wave, first);
     base += step;
     if (base >= rows) break;
     ra = rb;
     const long long rc = ra + step;
-    load_vectors<G, NV, FULL, NTL>(a, x, (rc < rows ? rc : last) * nvec, nvec, t);
+    load_vectors<FORM, G, NV, NTL>(a, x, rc < rows ? rc : last, at);
     if constexpr (RES) {
-      load_vectors<G, NV, FULL, NTL>(ea, res, (rc < rows ? rc : last) * nvec, nvec, t);
-      add_residual<T, G, NV, FULL, NTS>(b, eb, res_out, ra, nvec, t, ra < rows);
+      load_vectors<FORM, G, NV, NTL>(ea, res, rc < rows ? rc : last, at);
+      add_residual<T, FORM, G, NV, NTS>(b, eb, res_out, ra, at, ra < rows);
     }
-    norm_row<T, WAVES, NV, FULL, HAS_W, NTS>(b, wr, y, ra, nvec, cols, eps, t, ra < rows, slots[1], wave, first);
+    norm_row<T, WAVES, NV, FORM, HAS_W, RES, NTS>(b, wr, y, res_out, ra, at, eps, ra < rows, slots[1], wave, first);
     base += step;
     if (base >= rows) break;
     ra = rc;
@@ -332,13 +389,14 @@ struct Args {
   int cols;
   float eps;
   hipStream_t stream;
+  bool any;  // rows of any length and alignment
 };
 
-template <typename T, int WAVES, int NV, bool FULL, bool HAS_W, bool RES, bool NTL>
+template <typename T, int WAVES, int NV, int FORM, bool HAS_W, bool RES, bool NTL>
 int launch_k(const Args& a) {
   constexpr int BW = WAVES < 4 ? 4 : WAVES;
   constexpr int GROUPS = BW / WAVES;
-  auto kern = rmsnorm_rows<T, WAVES, NV, FULL, HAS_W, RES, NTL, true>;
+  auto kern = rmsnorm_rows<T, WAVES, NV, FORM, HAS_W, RES, NTL, true>;
   static int occ = 0;
   if (occ <= 0) occ = blocks_per_cu(kern, BW * kWave);
   // about 8 resident waves per CU by default (more waves only contend for the memory queues; measured on MI355X); 32 for
@@ -358,8 +416,10 @@ int launch_k(const Args& a) {
 
 template <typename T, int WAVES, int NV, bool HAS_W, bool RES, bool NTL>
 int launch_nv(const Args& a) {
-  if (a.nvec == (long long)WAVES * kWave * NV) return launch_k<T, WAVES, NV, true, HAS_W, RES, NTL>(a);
-  return launch_k<T, WAVES, NV, false, HAS_W, RES, NTL>(a);
+  if constexpr (NTL)  // (the tuning slot that switches it off is for aligned rows)
+    if (a.any) return launch_k<T, WAVES, NV, kAny, HAS_W, RES, true>(a);
+  if (a.nvec == (long long)WAVES * kWave * NV) return launch_k<T, WAVES, NV, kFull, HAS_W, RES, NTL>(a);
+  return launch_k<T, WAVES, NV, kPart, HAS_W, RES, NTL>(a);
 }
 
 template <typename T, int WAVES, bool HAS_W, bool RES, bool NTL>
@@ -407,8 +467,10 @@ int launch_typed(const void* x, const void* w, void* y, long long rows, int cols
   const bool vec = cols % T::V == 0 && rw_host::aligned16(x) && rw_host::aligned16(y) &&
                    (!HAS_W || rw_host::aligned16(w)) &&
                    (!RES || (rw_host::aligned16(res) && rw_host::aligned16(res_out)));
-  const long long nvec = cols / T::V;
-  if (vec && rw_host::tune_get(kTuneGeneric) != 1 && nvec <= (long long)kMaxWaves * kWave * kMaxNv) {
+  const long long nvec = ((long long)cols + T::V - 1) / T::V;
+  auto even = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 1u) == 0; };
+  const bool any = !vec && cols >= T::V && even(x) && even(y) && even(w) && even(res) && even(res_out);
+  if ((vec || any) && rw_host::tune_get(kTuneGeneric) != 1 && nvec <= (long long)kMaxWaves * kWave * kMaxNv) {
     // One wave per row up to 4 vectors per lane (2048 two-byte columns), then more waves at 4 vectors per lane (and 8
     // per lane once 16 waves are not enough).
     auto auto_waves = [&] {
@@ -418,8 +480,8 @@ int launch_typed(const void* x, const void* w, void* y, long long rows, int cols
     auto auto_nv = [&](int w) { return pow2_at_least((nvec + (long long)w * kWave - 1) / ((long long)w * kWave)); };
     int waves = rw_host::tune_get(kTuneWaves), nv = rw_host::tune_get(kTuneNv);
     if constexpr (!RES) {
-      if (nvec <= 2 * kShortLanes && waves <= 0 && nv <= 0) {  // 65536 x 256 bf16 28.0 -> 14.4 us, 65536 x 8 23.7 -> 4.6
-        const Args a{x, w, y, res, res_out, rows, nvec, cols, eps, stream};
+      if (vec && nvec <= 2 * kShortLanes && waves <= 0 && nv <= 0) {  // 65536 x 256 bf16 28.0 -> 14.4 us, 65536 x 8 23.7 -> 4.6
+        const Args a{x, w, y, res, res_out, rows, nvec, cols, eps, stream, any};
         return nvec <= kShortLanes ? launch_short<T, 1, HAS_W>(a) : launch_short<T, 2, HAS_W>(a);
       }
     }
@@ -433,9 +495,9 @@ int launch_typed(const void* x, const void* w, void* y, long long rows, int cols
       nv = auto_nv(waves);
     }
     if ((long long)waves * kWave * nv >= nvec) {
-      const Args a{x, w, y, res, res_out, rows, nvec, cols, eps, stream};
+      const Args a{x, w, y, res, res_out, rows, nvec, cols, eps, stream, any};
       // non-temporal loads unless switched off (2): x is read once
-      return rw_host::tune_get(kTuneNtLoads) != 2 ? launch_rows<T, HAS_W, RES, true>(waves, nv, a)
+      return any || rw_host::tune_get(kTuneNtLoads) != 2 ? launch_rows<T, HAS_W, RES, true>(waves, nv, a)
                                                   : launch_rows<T, HAS_W, RES, false>(waves, nv, a);
     }
   }
