@@ -415,7 +415,13 @@ struct Ptrs {
 template <typename T, typename C, bool FREQ, bool KV, int IPT>
 int launch_vec_k(const Ptrs& p, const Shape& s, int threads, hipStream_t stream) {
   auto kern = threads > 256 ? rope_vec<T, C, FREQ, KV, IPT, true> : rope_vec<T, C, FREQ, KV, IPT, false>;
-  int occ = blocks_per_cu(kern, threads);
+  // resident blocks per CU by the block's waves, of the kernel that this instantiation takes for them (idempotent cache)
+  static std::atomic<int> resident[1024 / kWave + 1];
+  int occ = resident[threads / kWave].load(std::memory_order_relaxed);
+  if (occ <= 0) {
+    occ = blocks_per_cu(kern, threads);
+    resident[threads / kWave].store(occ, std::memory_order_relaxed);
+  }
   int per_cu = rw_host::tune_get(kTuneBlocksPerCu);
   if (per_cu <= 0) per_cu = 8;  // 8 resident token blocks per CU by default (measured on MI355X)
   if (per_cu > occ) per_cu = occ;

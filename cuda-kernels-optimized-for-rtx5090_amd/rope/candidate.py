@@ -64,8 +64,36 @@ _lib.rope_kv_launch.argtypes = [ctypes.c_void_p] * 9 + [ctypes.c_longlong] + [ct
 _lib.rope_kv_launch.restype = ctypes.c_int
 
 
+# The device's current stream as an integer, without a Stream object where torch has the accessor (0.1 us against 1.9).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def _stream(device):
+    return _raw_stream(device.index) if _raw_stream else torch.cuda.current_stream(device).cuda_stream
+
+
+def _plain(q, k, ids, inv_freq, inplace):
+    """Whether these tensors are the usual accepted case of the rotation on the fly, each property read once: the checks
+    of _reject one by one took 2.6 us, more than the launch of a decode step; these 1.4."""
+    dtype, device, qs, ks = q.dtype, q.device, q.shape, k.shape
+    return dtype in _QK and k.dtype is dtype and ids.dtype is torch.int64 and len(qs) == 4 == len(ks) and \
+        qs[:2] == ks[:2] == ids.shape and qs[3] == ks[3] and inv_freq.dtype is torch.float32 and \
+        inv_freq.dim() == 1 and 2 * inv_freq.shape[0] == qs[3] and device.type == "cuda" and k.device == device and \
+        ids.device == device and inv_freq.device == device and not inplace
+
+
+def _plain_kv(q, k, v, ids, kc, vc, slots):
+    """The same for the cache write's further tensors (q, k and ids being accepted)."""
+    dtype, device, cs, ks = q.dtype, q.device, kc.shape, k.shape
+    return v.dtype is dtype and v.shape == ks and kc.dtype is dtype and vc.dtype is dtype and cs == vc.shape and \
+        len(cs) == 3 and cs[1:] == ks[2:] and kc.is_contiguous() and vc.is_contiguous() and kc.device == device and \
+        vc.device == device and slots.dtype is torch.int64 and slots.shape == ids.shape and slots.device == device
+
+
 def _reject(q, k, cos, sin, ids, inv_freq, inplace):
     """A short reason when these tensors cannot go to the kernels, else None."""
+    if inv_freq is not None and _plain(q, k, ids, inv_freq, inplace):
+        return None
     if q.dtype not in _QK or k.dtype != q.dtype:
         return f"dtypes q {q.dtype}, k {k.dtype}"
     if ids.dtype != torch.int64 or q.dim() != 4 or k.dim() != 4 or ids.dim() != 2:
@@ -94,7 +122,7 @@ def _run_kv(inputs):
     kc, vc, slots, inv_freq = inputs["k_cache"], inputs["v_cache"], inputs["slot_mapping"], inputs.get("inv_freq")
     inplace = bool(inputs.get("inplace", False))
     reason = _reject(q, k, None, None, ids, inv_freq, inplace) if inv_freq is not None else "inv_freq missing"
-    if reason is None:
+    if reason is None and not _plain_kv(q, k, v, ids, kc, vc, slots):
         Hk, D = k.shape[2], k.shape[3]
         if v.dtype != q.dtype or tuple(v.shape) != tuple(k.shape):
             reason = f"v {v.dtype} {tuple(v.shape)}"
@@ -111,7 +139,7 @@ def _run_kv(inputs):
     inv_freq = inv_freq.contiguous()
     err = _lib.rope_kv_launch(q.data_ptr(), k.data_ptr(), v.data_ptr(), ids.data_ptr(), inv_freq.data_ptr(),
                               q_out.data_ptr(), kc.data_ptr(), vc.data_ptr(), slots.data_ptr(), batch * seq, q_heads,
-                              k.shape[2], head_dim, _QK[q.dtype], torch.cuda.current_stream(q.device).cuda_stream)
+                              k.shape[2], head_dim, _QK[q.dtype], _stream(q.device))
     if err:
         raise RuntimeError(f"kernel launch failed: HIP error {err}")
     return {"q_out": q_out, "k_cache": kc, "v_cache": vc}
@@ -129,7 +157,7 @@ def run(inputs):
     q, k, ids = q.contiguous(), k.contiguous(), ids.contiguous()
     q_out, k_out = (q, k) if inplace else (torch.empty_like(q), torch.empty_like(k))
     batch, seq, q_heads, head_dim = q.shape
-    stream = torch.cuda.current_stream(q.device).cuda_stream
+    stream = _stream(q.device)
     if inv_freq is None:
         cos, sin = cos.contiguous(), sin.contiguous()
         err = _lib.launch(q.data_ptr(), k.data_ptr(), cos.data_ptr(), sin.data_ptr(), ids.data_ptr(),
