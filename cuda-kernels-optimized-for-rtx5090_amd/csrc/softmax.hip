@@ -5,6 +5,7 @@
 // Tiers, chosen by row length in 16-byte vectors (4 fp32 or 8 bf16 elements). The first two have an instantiation for rows
 // whose length is a multiple of the vector width and whose x and y are 16-byte aligned, and one for any other rows of
 // at least one vector (AnyRow):
+//  - short rows (at most 64 vectors): four rows side by side in a wave; see softmax_short.
 //  - row tier (rows up to 16 waves x 64 lanes x 8 vectors = 32768 fp32 / 65536 bf16 columns): a group of WAVES waves
 //    holds one row in registers, NV 16-byte vectors per lane. A max and a sum of exp(x - max) are reduced over the
 //    group (DPP inside each wave, one LDS slot per wave across waves) and y = exp(x - max) / sum is written from the
@@ -257,6 +258,101 @@ __global__ void __launch_bounds__((WAVES < 4 ? 4 : WAVES) * 64)
     base += step;
     if (base >= rows) break;
     ra = rc;
+  }
+}
+
+// Short rows (at most 64 vectors: attention over a short context, a router's experts), of any length from one vector up and
+// any element alignment: 16 lanes hold a row, NV vectors per lane (placed as AnyRow's), four rows side by side in a wave,
+// and a wave takes SETS times four rows per step, so that lanes hold data and several loads are in flight where a wave
+// per row would have one, mostly empty. The reductions stay inside a 16-lane DPP row; no LDS and no barrier. Waves are
+// persistent and load their next rows while they work on these.
+// 65536 rows, us as a wave per row / here: fp32 8 columns 20.8 / 4.7, 64 22.5 / 6.5, 128 23.0 / 11.0, 256 23.6 / 20.3; bf16 64
+// 24.5 / 5.9, 131 17.9 / 9.0 (56 in the scalar kernel), 512 24.0 / 21.5.
+constexpr int kShortLanes = 16;
+
+template <typename Op>
+__device__ __forceinline__ float short_reduce(float v, Op op) {
+  v = op(v, dpp<kDppXor1>(v));
+  v = op(v, dpp<kDppXor2>(v));
+  v = op(v, dpp<kDppHalfMirror>(v));
+  return op(v, dpp<kDppMirror>(v));
+}
+
+template <typename T, int NV>
+__global__ void __launch_bounds__(256)
+    softmax_short(const void* __restrict__ x, void* __restrict__ y, long long rows, int cols) {
+  constexpr int V = T::V, SIDE = kWave / kShortLanes, SETS = NV == 1 ? 4 : 2;
+  constexpr int ROWS = SETS * SIDE;  // a wave's rows per step
+  const int lane = lane_id(), l = lane & (kShortLanes - 1), sub = lane / kShortLanes;
+  const int per_block = (int)blockDim.x / kWave;
+  const long long step = (long long)gridDim.x * per_block * ROWS;
+  struct Step {
+    u32x4 v[SETS][NV];
+  };
+  auto start = [&](int k) { return (k * kShortLanes + l) * V; };
+  // the byte of vector k of the lane's row of set u, from the wave's first row on; a row past the last is the last
+  auto at = [&](long long first, int u, int k) __attribute__((always_inline)) {
+    const long long left = rows - 1 - first;
+    const int r = u * SIDE + sub;
+    return (uint32_t)(((left < r ? (int)left : r) * cols + least(start(k), cols - V)) * T::bytes);
+  };
+  auto load = [&](Step& s, long long first) __attribute__((always_inline)) {
+    if (first >= rows) first = rows - 1;
+    const char* base = static_cast<const char*>(x) + first * cols * T::bytes;
+#pragma unroll
+    for (int u = 0; u < SETS; ++u)
+#pragma unroll
+      for (int k = 0; k < NV; ++k) s.v[u][k] = load16_at<false>(base, at(first, u, k));
+  };
+  auto work = [&](const Step& s, long long first) __attribute__((always_inline)) {
+    char* base = static_cast<char*>(y) + first * cols * T::bytes;
+#pragma unroll
+    for (int u = 0; u < SETS; ++u) {
+      float f[NV][V];
+      float m = -INFINITY;
+#pragma unroll
+      for (int k = 0; k < NV; ++k) {
+        unpack<T>(s.v[u][k], f[k]);
+#pragma unroll
+        for (int i = 0; i < V; ++i) m = fmaxf(m, f[k][i]);
+      }
+      m = short_reduce(m, OpMax{});
+      float p[NV];
+#pragma unroll
+      for (int k = 0; k < NV; ++k) {
+#pragma unroll
+        for (int i = 0; i < V; ++i) f[k][i] = exp_below<T>(f[k][i] - m);
+        p[k] = sum_vector<T>(f[k], start(k) - least(start(k), cols - V));
+      }
+#pragma unroll
+      for (int d = 1; d < NV; d *= 2)
+#pragma unroll
+        for (int k = 0; k < NV; k += 2 * d) p[k] += p[k + d];
+      const float sum = short_reduce(p[0], OpSum{});
+      const float inv = 1.0f / sum;
+      const bool in = first + u * SIDE + sub < rows;
+#pragma unroll
+      for (int k = 0; k < NV; ++k) {
+        if (!in || start(k) >= cols) continue;
+#pragma unroll
+        for (int i = 0; i < V; ++i) f[k][i] = quotient<T>(f[k][i], sum, inv);
+        store16_at<true>(base, at(first, u, k), pack<T>(f[k]));
+      }
+    }
+  };
+  long long first = ((long long)blockIdx.x * per_block + __builtin_amdgcn_readfirstlane(wave_id())) * ROWS;
+  if (first >= rows) return;
+  Step a, b;
+  load(a, first);
+  while (true) {
+    load(b, first + step);
+    work(a, first);
+    first += step;
+    if (first >= rows) break;
+    load(a, first + step);
+    work(b, first);
+    first += step;
+    if (first >= rows) break;
   }
 }
 
@@ -738,6 +834,27 @@ int launch_any(int waves, int nv, const void* x, void* y, long long rows, int co
   }
 }
 
+template <typename T, int NV>
+int launch_short_nv(const void* x, void* y, long long rows, int cols, hipStream_t stream) {
+  constexpr int ROWS = (NV == 1 ? 4 : 2) * (kWave / kShortLanes);
+  const long long cus = rw_host::device_cus(), waves = (rows + ROWS - 1) / ROWS;
+  int per_cu = rw_host::tune_get(kTuneBlocksPerCu);
+  if (per_cu <= 0) per_cu = 6;
+  const int per_block = waves >= 4 * cus ? 4 : 1;  // one wave per block until every CU has four: few rows spread over the GPU
+  long long grid = (waves + per_block - 1) / per_block;
+  if (grid > cus * per_cu * 4 / per_block) grid = cus * per_cu * 4 / per_block;
+  hipLaunchKernelGGL((softmax_short<T, NV>), dim3((unsigned)grid), dim3(per_block * kWave), 0, stream, x, y, rows, cols);
+  return (int)hipGetLastError();
+}
+
+template <typename T>
+int launch_short(const void* x, void* y, long long rows, long long cols, hipStream_t stream) {
+  const long long nvec = (cols + T::V - 1) / T::V;
+  if (nvec <= kShortLanes) return launch_short_nv<T, 1>(x, y, rows, (int)cols, stream);
+  if (nvec <= 2 * kShortLanes) return launch_short_nv<T, 2>(x, y, rows, (int)cols, stream);
+  return launch_short_nv<T, 4>(x, y, rows, (int)cols, stream);
+}
+
 template <typename T, int WAVES>
 int launch_stream_w(const void* x, void* y, long long rows, long long nvec, hipStream_t stream) {
   long long grid = (long long)rw_host::device_cus() * (16 / WAVES > 1 ? 16 / WAVES : 1);
@@ -907,6 +1024,13 @@ int launch_generic(const void* x, void* y, long long rows, long long cols, hipSt
   return (int)hipGetLastError();
 }
 
+// Whether the tuning slots ask for a row-tier shape that the kernels have.
+bool row_shape_tuned() {
+  const int w = rw_host::tune_get(kTuneWaves), n = rw_host::tune_get(kTuneNv);
+  auto pow2_to = [](int v, int most) { return v >= 0 && v <= most && (v & (v - 1)) == 0; };
+  return (w || n) && pow2_to(w, kMaxWaves) && pow2_to(n, 16) && !(n == 16 && (w == 0 || w > 2));
+}
+
 // Rows that the row tier could hold but the co-resident tier takes faster: rows of more than 4096 vectors, which in the
 // row tier are 16 waves x 8 vectors with registers spilled (bf16 always: 600 x 40000 34 -> 19.5 us, 1024 x 50000 56 -> 46,
 // 1024 x 65536 51 -> 50; fp32 when every row's chunks are resident at once: 256 x 32768 15.0 -> 11.0, 512 x 20000
@@ -915,10 +1039,7 @@ int launch_generic(const void* x, void* y, long long rows, long long cols, hipSt
 // way). A launch that is being captured stays in the row tier, which needs no second node and no tag cell.
 template <typename T>
 bool coop_instead_of_rows(long long rows, long long nvec, hipStream_t stream) {
-  const int w = rw_host::tune_get(kTuneWaves), n = rw_host::tune_get(kTuneNv);
-  auto pow2_to = [](int v, int most) { return v >= 0 && v <= most && (v & (v - 1)) == 0; };
-  const bool row_shape = (w || n) && pow2_to(w, kMaxWaves) && pow2_to(n, 16) && !(n == 16 && (w == 0 || w > 2));
-  if (rw_host::tune_get(kTuneTier) != 0 || row_shape) return false;  // a row-tier shape the kernels have is asked for
+  if (rw_host::tune_get(kTuneTier) != 0 || row_shape_tuned()) return false;
   return (nvec > 4096 || (nvec > 2048 && rows <= 32)) && !capturing(stream);
 }
 
@@ -929,6 +1050,10 @@ int launch_typed(const void* x, void* y, long long rows, long long cols, hipStre
   const bool any = cols >= T::V && aligned_to(x, T::bytes) && aligned_to(y, T::bytes);
   if (tier == 3 || !(vec || any)) return launch_generic<T>(x, y, rows, cols, stream);
   const long long nvec = (cols + T::V - 1) / T::V;
+  // (four vectors per lane: only with rows enough to keep the GPU full at eight to a wave; 4096 x 257 bf16 3.7 us as a
+  // wave per row, 4.3 as short rows; 65536 x 257 19.1 and 17.5)
+  if (any && nvec <= (rows >= 8192 ? 4 : 2) * kShortLanes && tier == 0 && !row_shape_tuned())
+    return launch_short<T>(x, y, rows, cols, stream);
   if (!vec) {
     const CoopLaunch coop{x, y, rows, nvec, cols, stream};
     if (nvec > (long long)kMaxWaves * kWave * kMaxNv || tier == 4) {

@@ -1,5 +1,5 @@
-"""Softmax rows of any length and element alignment on the vector tiers (softmax_rows_any and the co-resident tier's
-instantiation for such rows): the sizes where a row's last vector, a wave's share or a chunk begins to be used, base
+"""Softmax rows of any length and element alignment on the vector tiers (softmax_short, softmax_rows_any and the
+co-resident tier's instantiation for such rows): the sizes where a row's last vector, a wave's share or a chunk begins to be used, base
 pointers off a 16-byte boundary, -inf elements and rows, against the oracle within the bounds of the softmax tests (fp32
 1e-5 relative, and 2^-147 below the normal range; bf16 1 ulp). The emulated cases run the kernels' source on the CPU
 between guard pages, so an access outside a row's tensor ends them; a stopped clock makes a wait end by its pairs only."""
@@ -27,6 +27,18 @@ EDGES = {0: [4, 5, 255, 257, 1023, 1025, 2047, 4097, 8191], 1: [8, 9, 511, 513, 
 def test_emulated_row_edges(emu_softmax, dtype, cols):
     # offset 1: the buffers begin one element past a 16-byte boundary (and rows of a whole number of vectors are unaligned)
     run(emu_softmax, [9, cols, dtype, 1, cols, 0, 0, 1, "special"])
+
+
+# rows of one vector to 64 of them (fp32 4 to 256 columns, bf16 8 to 512) in softmax_short, numbers of rows that leave a
+# wave's sets empty or take several steps
+SHORT = [(1, 4, 0), (3, 5, 0), (17, 63, 0), (16, 64, 0), (9, 65, 0), (33, 127, 0), (8200, 130, 0), (1, 8, 1), (70, 9, 1),
+         (15, 127, 1), (40, 129, 1), (8, 256, 1), (8193, 257, 1)]
+
+
+@pytest.mark.parametrize("pattern", ["randn", "special"])
+@pytest.mark.parametrize("rows,cols,dtype", SHORT)
+def test_emulated_short_rows(emu_softmax, rows, cols, dtype, pattern):
+    run(emu_softmax, [rows, cols, dtype, 0, cols, 0, 0, cols % 4, pattern])
 
 
 @pytest.mark.parametrize("dtype,waves,nv", [(0, 1, 8), (0, 2, 4), (0, 16, 1), (1, 1, 8), (1, 8, 2)])
@@ -80,7 +92,8 @@ def _check(pkg, oracle, dev, rows, cols, dtype, offset=0, special=False):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
-@pytest.mark.parametrize("rows,cols", [(3, 8), (70, 9), (513, 255), (700, 513), (5, 2049), (300, 3001), (9, 8191),
+@pytest.mark.parametrize("rows,cols", [(3, 8), (70, 9), (40000, 8), (5000, 63), (70001, 64), (16385, 131), (9000, 255),
+                                       (8191, 256), (8192, 257), (9001, 511), (20000, 512), (513, 255), (700, 513), (5, 2049), (300, 3001), (9, 8191),
                                        (600, 16383), (3, 16384), (40, 20001), (2, 32767), (300, 20000), (5, 65535),
                                        (3, 70001), (2, 262143), (70, 262143), (1, 1048576), (2, 1048577)])
 def test_gpu_rows(pkg, oracle, dev, dtype, rows, cols):
