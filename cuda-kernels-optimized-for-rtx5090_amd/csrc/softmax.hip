@@ -560,10 +560,8 @@ __global__ void __launch_bounds__(WAVES * 64)
                                                      : sum_vector<T>(f, start - least(start, reach - T::V));
       } else {
 #pragma unroll
-        for (int i = 0; i < T::V; ++i) {
-          e[k][i] = ok && m != -INFINITY ? exp_to<T>(f[i] - m) : 0.0f;
-          s += e[k][i];
-        }
+        for (int i = 0; i < T::V; ++i) e[k][i] = ok && m != -INFINITY ? exp_to<T>(f[i] - m) : 0.0f;
+        s += sum_vector<T>(e[k], 0);
       }
     }
     s = group_reduce<WAVES>(s, OpSum{}, slots[1], wave_id(), 0);
