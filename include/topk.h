@@ -70,7 +70,8 @@ int topk_launch_sample(const void* x, void* values, void* indices, void* work, v
 
 /* No counterpart in the reference: tuning override for parameter sweeps. Slot 0: resident workgroups per CU assumed by
  * plan(); slot 1: 1 makes launch() take the naive tier (one workgroup per row, one scan of the row per output
- * position: the harness's seed column). Returns 0 or -1. */
+ * position: the harness's seed column); slot 2: the short rows' kernel for every row it can hold (1) or none (2).
+ * Returns 0 or -1. */
 int topk_tune(int slot, int value);
 
 #ifdef __cplusplus

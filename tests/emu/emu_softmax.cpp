@@ -8,7 +8,7 @@
 //   tier: 1 row, 2 stream, 3 generic, 4 co-resident (preferred through softmax_tune); waves / nv: the row tier's
 //   shape (tier 1), the stream tier's waves (tier 2), the co-resident tier's row groups in nv (tier 4; fewer groups
 //   than rows make each workgroup walk several rows), 0 automatic; offset shifts x and y by that many elements from a
-//   16-byte boundary (a misaligned row takes the generic tier); pattern: randn (N(0, 4)) or special (-inf elements,
+//   16-byte boundary; pattern: randn (N(0, 4)) or special (-inf elements,
 //   an all -inf row, a row of one huge value); reps: launches on the same buffers, each checked (the co-resident
 //   tier's pair table is reused by the next launch, under fresh tags); wait_ticks bounds the co-resident tier's wait
 //   (1 makes its workgroups stop waiting and take the row's statistics from x).

@@ -1,8 +1,9 @@
 """Softmax rows of any length and element alignment on the vector tiers (softmax_short, softmax_rows_any and the
-co-resident tier's instantiation for such rows): the sizes where a row's last vector, a wave's share or a chunk begins to be used, base
-pointers off a 16-byte boundary, -inf elements and rows, against the oracle within the bounds of the softmax tests (fp32
-1e-5 relative, and 2^-147 below the normal range; bf16 1 ulp). The emulated cases run the kernels' source on the CPU
-between guard pages, so an access outside a row's tensor ends them; a stopped clock makes a wait end by its pairs only."""
+co-resident tier's instantiation for such rows): the sizes where a row's last vector, a wave's share or a chunk begins
+to be used, base pointers off a 16-byte boundary, -inf elements and rows, against the oracle within the bounds of the
+softmax tests (fp32 1e-5 relative, and 2^-147 below the normal range; bf16 1 ulp). The emulated cases run the kernels'
+source on the CPU between guard pages, so an access outside a row's tensor ends them; a stopped clock makes a wait end
+by its pairs only."""
 
 import ctypes
 import os

@@ -8,8 +8,8 @@ to 33 ulps from the oracle on rows whose outputs reach that range (checked in te
 normal magnitude keep the relative bound alone.
 Shapes cover every tier: wave-per-row and workgroup-per-row rows (full and ragged), the single-pass co-resident tier
 for long rows (one row per workgroup, and row groups walking several rows when the rows' chunks do not all fit at
-once), the two-pass stream tier for rows beyond it, and the generic tier for lengths that are not a multiple of the
-vector width and for misaligned pointers.
+once), the two-pass stream tier for rows beyond it, and lengths that are not a multiple of the vector width and
+misaligned pointers.
 """
 
 import ctypes
@@ -80,7 +80,7 @@ def test_many_rows_persistent(pkg, oracle, dev):
 def test_misaligned_and_special_values(pkg, oracle, dev):
     g = torch.Generator().manual_seed(6)
     base = torch.randn(4 * 1024 + 1, generator=g).to(dev)
-    x = base[1:].view(4, 1024)  # data pointer 4 bytes past a 16-byte boundary: the generic tier
+    x = base[1:].view(4, 1024)  # data pointer 4 bytes past a 16-byte boundary
     y = torch.empty_like(x)
     lib = pkg.candidate("softmax")._lib
     assert lib.launch(x.data_ptr(), y.data_ptr(), 4, 1024, 0, 256, 1024, torch.cuda.current_stream().cuda_stream) == 0
