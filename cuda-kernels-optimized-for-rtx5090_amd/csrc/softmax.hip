@@ -1034,7 +1034,8 @@ bool row_shape_tuned() {
 // 1024 x 65536 51 -> 50; fp32 when every row's chunks are resident at once: 256 x 32768 15.0 -> 11.0, 512 x 20000
 // 19.0 -> 13.1, but 2048 x 32768 97 -> 103 in row groups), and rows of more than 2048 vectors when they are too few to
 // fill the GPU with one workgroup each (1 x 10000 fp32 4.5 -> 3.9, 16 x 32000 bf16 5.4 -> 4.2; 128 x 16384 fp32 6.0 either
-// way). A launch that is being captured stays in the row tier, which needs no second node and no tag cell.
+// way). A launch that is being captured stays in the row tier, which needs no second node and no tag cell, and so does
+// one in place (its callers look), where a timed-out wait's second read of the row would meet outputs.
 template <typename T>
 bool coop_instead_of_rows(long long rows, long long nvec, hipStream_t stream) {
   if (rw_host::tune_get(kTuneTier) != 0 || row_shape_tuned()) return false;
@@ -1055,10 +1056,11 @@ int launch_typed(const void* x, void* y, long long rows, long long cols, hipStre
   if (!vec) {
     const CoopLaunch coop{x, y, rows, nvec, cols, stream};
     if (nvec > (long long)kMaxWaves * kWave * kMaxNv || tier == 4) {
-      const int rc = launch_coop<T, false, true>(coop);
+      // (in place, a workgroup whose wait timed out would read a row that others have begun to overwrite)
+      const int rc = x != y ? launch_coop<T, false, true>(coop) : 1;
       return rc != 1 ? rc : launch_generic<T>(x, y, rows, cols, stream);
     }
-    if (coop_instead_of_rows<T>(rows, nvec, stream)) {
+    if (x != y && coop_instead_of_rows<T>(rows, nvec, stream)) {
       const int rc = launch_coop<T, false, true>(coop, T::bytes == 4);
       if (rc != 1) return rc;
     }
@@ -1078,7 +1080,7 @@ int launch_typed(const void* x, void* y, long long rows, long long cols, hipStre
   }
   if (tier == 2) return launch_stream<T>(x, y, rows, nvec, stream);
   const CoopLaunch coop{x, y, rows, nvec, cols, stream};
-  if (nvec <= (long long)kMaxWaves * kWave * kMaxNv && coop_instead_of_rows<T>(rows, nvec, stream)) {
+  if (x != y && nvec <= (long long)kMaxWaves * kWave * kMaxNv && coop_instead_of_rows<T>(rows, nvec, stream)) {
     // fp32 rows keep the row tier's rounding (x held, the exponential taken again): the instantiation for any rows
     const int rc = T::bytes == 4 ? launch_coop<T, false, true>(coop, true) : launch_coop<T, false, false>(coop);
     if (rc != 1) return rc;

@@ -2,7 +2,7 @@
  * Library: build/softmax/libkernel.so. Replaces the reference's softmax/kernel.cu:520-527 (and the same ABI of
  * softmax/seed.cu:68-81). x and y are device pointers to row-major contiguous [rows, cols] data; the call is
  * asynchronous on `stream` and allocates nothing; rows may have any length and x and y any element alignment. Rows longer
- * than 32768 fp32 / 65536 bf16 elements whose chunks fit on the GPU at once (and, outside a capture, some shorter ones:
+ * than 32768 fp32 / 65536 bf16 elements whose chunks fit on the GPU at once (and, outside a capture and not in place, some shorter ones:
  * more than 16384 fp32 / 32768 bf16 elements, or more than half of that in at most 32 rows) are done in one pass by
  * co-resident workgroups that exchange their chunk statistics through a static device table of the library (entries tagged per launch, nothing to clear); launches on one stream are ordered
  * by it, and a launch overlapping another on a second stream stays exact (at worst its workgroups stop waiting after

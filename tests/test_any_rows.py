@@ -73,22 +73,25 @@ def _check(pkg, oracle, dev, rows, cols, dtype, offset=0, special=False):
         x[-1] = float("-inf")
     x = x.to(dtype)
     n = rows * cols
-    # an in-place call at an offset: x and y are one buffer, whose other elements must stay as they were
+    # at an offset into a buffer whose other elements must stay as they were: into another buffer, and in place
     buf = torch.full((n + 32,), 7.0, dtype=dtype)
     buf[offset:offset + n] = x.view(-1)
-    d = buf.to(dev)
     lib = pkg.candidate("softmax")._lib
-    at = d.data_ptr() + offset * d.element_size()
-    err = lib.launch(at, at, rows, cols, 0 if dtype == torch.float32 else 1, 256, 1024,
-                     ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
-    assert err == 0
-    out = d.cpu()
-    assert (out[:offset] == 7).all() and (out[offset + n:] == 7).all()
-    y = out[offset:offset + n].view(rows, cols)
-    if dtype == torch.float32:
-        assert_rel(y.numpy(), oracle.softmax(x.numpy(), "fp32"), 1e-5, f"{rows}x{cols}", 2.0 ** -147)
-    else:
-        assert_ulp(bits16(y), oracle.softmax(bits16(x), "bf16"), 1, f"{rows}x{cols}")
+    for inplace in (False, True):
+        src = buf.to(dev)
+        dst = src if inplace else torch.full_like(src, 7.0)
+        at = offset * src.element_size()
+        err = lib.launch(src.data_ptr() + at, dst.data_ptr() + at, rows, cols, 0 if dtype == torch.float32 else 1, 256,
+                         1024, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        assert err == 0
+        out = dst.cpu()
+        assert (out[:offset] == 7).all() and (out[offset + n:] == 7).all()
+        y = out[offset:offset + n].view(rows, cols)
+        what = f"{rows}x{cols} in place {inplace}"
+        if dtype == torch.float32:
+            assert_rel(y.numpy(), oracle.softmax(x.numpy(), "fp32"), 1e-5, what, 2.0 ** -147)
+        else:
+            assert_ulp(bits16(y), oracle.softmax(bits16(x), "bf16"), 1, what)
 
 
 @pytest.mark.gpu
@@ -145,3 +148,26 @@ def test_gpu_captured_rows_take_the_row_tier(pkg, oracle, dev):
         graph.replay()
         torch.cuda.synchronize()
         assert_rel(y.cpu().numpy(), oracle.softmax(h.numpy(), "fp32"), 1e-5, f"replay {seed}", 2.0 ** -147)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_gpu_captured_unaligned_long_rows(pkg, oracle, dev, dtype):
+    # unaligned rows beyond the row tier, recorded into a graph: fresh tags at every replay, eager launches in between
+    x = torch.empty(3, 70001, device=dev, dtype=dtype)
+    pkg.softmax(x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = pkg.softmax(x)
+    for seed in range(4):
+        h = (torch.randn(3, 70001, generator=torch.Generator().manual_seed(seed)) * 3).to(dtype)
+        x.copy_(h)
+        if seed % 2:
+            pkg.softmax(x + 1)
+        graph.replay()
+        torch.cuda.synchronize()
+        if dtype == torch.float32:
+            assert_rel(y.cpu().numpy(), oracle.softmax(h.numpy(), "fp32"), 1e-5, f"replay {seed}", 2.0 ** -147)
+        else:
+            assert_ulp(bits16(y), oracle.softmax(bits16(h), "bf16"), 1, f"replay {seed}")
