@@ -17,10 +17,10 @@
 // Rows whose length is a multiple of 8 with 16-byte aligned x, y (and w) run the row kernel: a group of WAVES waves
 // holds one row in registers as NV 16-byte vectors per lane, reduces the sum over the group (DPP within a wave, LDS
 // slots across waves) and writes y from the registers; each lane holds the weight vectors of its columns once for all
-// rows. Workgroups are persistent and load their next row while they reduce and store the current one. Rows of any other
-// length from 8 columns up, or otherwise aligned, run the same kernel with element-aligned vectors (Form kAny); aligned
-// rows of at most 32 vectors share waves, four at a time (rmsnorm_short). What is left (rows of fewer than 8 columns, or
-// longer than 16 waves hold) takes a generic kernel (one workgroup per row, scalar accesses, two passes).
+// rows. Workgroups are persistent and load their next row while they reduce and store the current one. Rows of any
+// other length from 8 columns up, or otherwise aligned, run the same kernel with element-aligned vectors (Form kAny);
+// aligned rows of at most 32 vectors share waves, four at a time (rmsnorm_short). What is left (rows of fewer than 8
+// columns, or longer than 16 waves hold) takes a generic kernel (one workgroup per row, scalar accesses, two passes).
 #include <climits>
 #include <cmath>
 #include <type_traits>
@@ -40,9 +40,9 @@ struct Regs {
   u32x4 v[NV];
 };
 
-// How rows lie under a group's vectors: kFull, as many aligned vectors as the group holds; kPart, fewer; kAny, rows of any
-// length (at least a vector) at any element alignment: the row's last vector is moved back to end with the row, its first
-// elements being another lane's (the same bits, and the same results when they are stored twice).
+// How rows lie under a group's vectors: kFull, as many aligned vectors as the group holds; kPart, fewer; kAny, rows of
+// any length (at least a vector) at any element alignment: the row's last vector is moved back to end with the row, its
+// first elements being another lane's (the same bits, and the same results when they are stored twice).
 enum Form { kPart = 0, kFull = 1, kAny = 2 };
 
 // The lane's place in its rows. Lane t of the group's G holds vectors t, t + G, ..., clamped into the row.
@@ -56,9 +56,12 @@ struct Place {
   __device__ __forceinline__ bool used(int k) const { return FORM == kFull || (long long)k * G + wave0 < nvec; }
   __device__ __forceinline__ bool whole(int k) const { return (k * G + wave0 + kWave) * V <= cols; }
   __device__ __forceinline__ int start(int k) const { return (k * G + t) * V; }  // vector k's first element
-  __device__ __forceinline__ bool in(int k) const { return FORM == kFull || (FORM == kAny ? start(k) < cols : (long long)k * G + t < nvec); }
+  __device__ __forceinline__ bool in(int k) const {
+    return FORM == kFull || (FORM == kAny ? start(k) < cols : (long long)k * G + t < nvec);
+  }
   __device__ __forceinline__ uint32_t any_at(int k) const { return (uint32_t)least(start(k), cols - V) * 2u; }  // bytes
-  __device__ __forceinline__ int skip(int k) const { return start(k) - least(start(k), cols - V); }  // another lane's elements
+  // the first elements of vector k that are another lane's
+  __device__ __forceinline__ int skip(int k) const { return start(k) - least(start(k), cols - V); }
 
   template <bool NTL>
   __device__ __forceinline__ u32x4 load(const void* base, long long row, int k) const {
@@ -125,8 +128,8 @@ __device__ __forceinline__ void norm_row(const Regs<NV>& r, const Regs<NV>& w, v
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
     if (active && at.in(k)) {
-      // (kAny: h is stored only here, behind the reduction, which every wave reaches with its vectors loaded: in place, a
-      // vector moved back at the row's end reads elements that another wave writes)
+      // (kAny: h is stored only here, behind the reduction, which every wave reaches with its vectors loaded: in place,
+      // a vector moved back at the row's end reads elements that another wave writes)
       if constexpr (RES && FORM == kAny) at.template store<NTS>(res_out, row, k, r.v[k]);
       float f[T::V];
       unpack<T>(r.v[k], f);
@@ -220,12 +223,12 @@ __global__ void __launch_bounds__((WAVES < 4 ? 4 : WAVES) * 64)
 }
 
 // Short rows (at most 32 vectors: the norm of each query or key head): 16 lanes hold a row, NV vectors per lane, and a
-// wave takes kShortSets sets of four rows at once, so that every lane holds data, and the row factor's chain (fp64 square
-// root and divisions, about 100 instructions) runs once per wave for all sixteen rows: the reduction over a row's lanes
-// first trades the four sets within each quad of lanes (two steps that halve the values a lane holds), which leaves set
-// q's sum in the lanes with lane % 4 == q, and every lane reads its sets' factors back from its quad. Waves are
-// persistent and load their next sixteen rows while they work on these; no LDS and no barrier. Bound by memory at 128
-// columns, by instruction issue below.
+// wave takes kShortSets sets of four rows at once, so that every lane holds data, and the row factor's chain (fp64
+// square root and divisions, about 100 instructions) runs once per wave for all sixteen rows: the reduction over a
+// row's lanes first trades the four sets within each quad of lanes (two steps that halve the values a lane holds),
+// which leaves set q's sum in the lanes with lane % 4 == q, and every lane reads its sets' factors back from its quad.
+// Waves are persistent and load their next sixteen rows while they work on these; no LDS and no barrier. Bound by
+// memory at 128 columns, by instruction issue below.
 // 163840 x 128 bf16 with a weight: 62.9 us as a wave per row with 16 of 64 lanes holding data, 16 us here.
 constexpr int kShortLanes = 16, kShortSets = 4;
 constexpr int kShortRows = kShortSets * (kWave / kShortLanes);  // a wave's rows per step
@@ -399,9 +402,9 @@ int launch_k(const Args& a) {
   auto kern = rmsnorm_rows<T, WAVES, NV, FORM, HAS_W, RES, NTL, true>;
   static int occ = 0;
   if (occ <= 0) occ = blocks_per_cu(kern, BW * kWave);
-  // about 8 resident waves per CU by default (more waves only contend for the memory queues; measured on MI355X); 32 for
-  // rows of at most 96 vectors, whose waves hold too little in flight (65536 rows bf16: 264 columns 28.4 -> 20.5 us, 512
-  // columns 31.0 -> 24.4, 640 columns 38.1 -> 31.9, but 1024 columns 44.9 -> 47.0)
+  // about 8 resident waves per CU by default (more waves only contend for the memory queues; measured on MI355X); 32
+  // for rows of at most 96 vectors, whose waves hold too little in flight (65536 rows bf16: 264 columns 28.4 -> 20.5
+  // us, 512 columns 31.0 -> 24.4, 640 columns 38.1 -> 31.9, but 1024 columns 44.9 -> 47.0)
   int per_cu = rw_host::tune_get(kTuneBlocksPerCu);
   if (per_cu <= 0 && WAVES == 1 && a.nvec <= 96) per_cu = 8;
   if (per_cu <= 0) per_cu = 8 / BW > 1 ? 8 / BW : 1;
@@ -480,7 +483,8 @@ int launch_typed(const void* x, const void* w, void* y, long long rows, int cols
     auto auto_nv = [&](int w) { return pow2_at_least((nvec + (long long)w * kWave - 1) / ((long long)w * kWave)); };
     int waves = rw_host::tune_get(kTuneWaves), nv = rw_host::tune_get(kTuneNv);
     if constexpr (!RES) {
-      if (vec && nvec <= 2 * kShortLanes && waves <= 0 && nv <= 0) {  // 65536 x 256 bf16 28.0 -> 14.4 us, 65536 x 8 23.7 -> 4.6
+      if (vec && nvec <= 2 * kShortLanes && waves <= 0 && nv <= 0) {
+        // 65536 x 256 bf16 28.0 -> 14.4 us, 65536 x 8 23.7 -> 4.6
         const Args a{x, w, y, res, res_out, rows, nvec, cols, eps, stream, any};
         return nvec <= kShortLanes ? launch_short<T, 1, HAS_W>(a) : launch_short<T, 2, HAS_W>(a);
       }

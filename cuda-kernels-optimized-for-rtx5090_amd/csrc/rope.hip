@@ -415,7 +415,8 @@ struct Ptrs {
 template <typename T, typename C, bool FREQ, bool KV, int IPT>
 int launch_vec_k(const Ptrs& p, const Shape& s, int threads, hipStream_t stream) {
   auto kern = threads > 256 ? rope_vec<T, C, FREQ, KV, IPT, true> : rope_vec<T, C, FREQ, KV, IPT, false>;
-  // resident blocks per CU by the block's waves, of the kernel that this instantiation takes for them (idempotent cache)
+  // resident blocks per CU by the block's waves, of the kernel that this instantiation takes for them (idempotent
+  // cache)
   static std::atomic<int> resident[1024 / kWave + 1];
   int occ = resident[threads / kWave].load(std::memory_order_relaxed);
   if (occ <= 0) {

@@ -109,10 +109,10 @@ __device__ __forceinline__ float exp_narrow(float d) {
 template <typename T> __device__ __forceinline__ float exp_to(float d) { return exp_narrow(d); }
 template <> __device__ __forceinline__ float exp_to<F32>(float d) { return expf(d); }
 
-// expf's accuracy (about an ulp) in half its instructions, for d <= 0: d log2 e is split into an integer n and a fraction
-// of at most a half by fused multiply-adds, the hardware's exp2 takes the fraction and v_ldexp_f32 applies n (results
-// below the normal range stay subnormal). n is bounded from below, so that d = -inf gives 0; NaN stays NaN. 1024 x 16383
-// fp32 softmax 25.9 us with expf, 23.7 us with this, at the same distance from the fp64 softmax.
+// expf's accuracy (about an ulp) in half its instructions, for d <= 0: d log2 e is split into an integer n and a
+// fraction of at most a half by fused multiply-adds, the hardware's exp2 takes the fraction and v_ldexp_f32 applies n
+// (results below the normal range stay subnormal). n is bounded from below, so that d = -inf gives 0; NaN stays NaN.
+// 1024 x 16383 fp32 softmax 25.9 us with expf, 23.7 us with this, at the same distance from the fp64 softmax.
 __device__ __forceinline__ float exp_nonpositive(float d) {
   const float n = fmaxf(__builtin_rintf(d * 1.44269504088896341f), -300.0f);
   const float f = __builtin_fmaf(d, 1.92596298909109e-8f, __builtin_fmaf(d, 1.4426950216293335f, -n));
@@ -160,10 +160,10 @@ __device__ __forceinline__ void store16(void* p, long long v, const u32x4& r) {
   else *q = r;
 }
 
-// The same at any element boundary: 16 bytes from byte `at` of the region, aligned to 2 bytes (a wave-uniform base and a
-// 32-bit offset per lane, which one instruction takes). The hardware takes 16-byte
-// global accesses at any address; a 48 MiB copy measured 18.1 us aligned, 19.2 us 4 bytes off and 20.6 us 2 bytes off, a
-// read 8.4, 8.5 and 10.9 us.
+// The same at any element boundary: 16 bytes from byte `at` of the region, aligned to 2 bytes (a wave-uniform base and
+// a 32-bit offset per lane, which one instruction takes). The hardware takes 16-byte
+// global accesses at any address; a 48 MiB copy measured 18.1 us aligned, 19.2 us 4 bytes off and 20.6 us 2 bytes off,
+// a read 8.4, 8.5 and 10.9 us.
 typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
 template <bool NT>
 __device__ __forceinline__ u32x4 load16_at(const void* p, uint32_t at) {

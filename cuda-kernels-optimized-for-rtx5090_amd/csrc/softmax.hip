@@ -2,9 +2,9 @@
 // accumulated in fp32 and each output rounded once (round to nearest even for bf16), behind the reference's C-ABI
 // `launch` (softmax/kernel.cu:520-527, softmax/seed.cu:68-81).
 //
-// Tiers, chosen by row length in 16-byte vectors (4 fp32 or 8 bf16 elements). The first two have an instantiation for rows
-// whose length is a multiple of the vector width and whose x and y are 16-byte aligned, and one for any other rows of
-// at least one vector (AnyRow):
+// Tiers, chosen by row length in 16-byte vectors (4 fp32 or 8 bf16 elements). The first two have an instantiation for
+// rows whose length is a multiple of the vector width and whose x and y are 16-byte aligned, and one for any other rows
+// of at least one vector (AnyRow):
 //  - short rows (at most 64 vectors): four rows side by side in a wave; see softmax_short.
 //  - row tier (rows up to 16 waves x 64 lanes x 8 vectors = 32768 fp32 / 65536 bf16 columns): a group of WAVES waves
 //    holds one row in registers, NV 16-byte vectors per lane. A max and a sum of exp(x - max) are reduced over the
@@ -171,9 +171,9 @@ __global__ void __launch_bounds__((WAVES < 4 ? 4 : WAVES) * 64)
 
 // Row tier for rows of any length from one vector up and any element alignment: the lanes' vectors start at the row's
 // first element, wherever it lies, and a vector that would pass the row's end is moved back to end with it. Its first
-// elements are then another lane's (the same bits, and the same results when they are stored twice), so the maximum takes
-// every loaded element and the sum leaves out the first `skip` of the vector; only the wave that holds the row's end
-// looks at that, and vectors that lie past the end for a whole wave are not worked on.
+// elements are then another lane's (the same bits, and the same results when they are stored twice), so the maximum
+// takes every loaded element and the sum leaves out the first `skip` of the vector; only the wave that holds the row's
+// end looks at that, and vectors that lie past the end for a whole wave are not worked on.
 // 8192 x 3001 bf16 55.5 us through the scalar kernel's three passes of 2-byte accesses, 16.9 us here.
 template <typename T, int WAVES, int NV>
 struct AnyRow {
@@ -261,13 +261,13 @@ __global__ void __launch_bounds__((WAVES < 4 ? 4 : WAVES) * 64)
   }
 }
 
-// Short rows (at most 64 vectors: attention over a short context, a router's experts), of any length from one vector up and
-// any element alignment: 16 lanes hold a row, NV vectors per lane (placed as AnyRow's), four rows side by side in a wave,
-// and a wave takes SETS times four rows per step, so that lanes hold data and several loads are in flight where a wave
-// per row would have one, mostly empty. The reductions stay inside a 16-lane DPP row; no LDS and no barrier. Waves are
-// persistent and load their next rows while they work on these.
-// 65536 rows, us as a wave per row / here: fp32 8 columns 20.8 / 4.7, 64 22.5 / 6.5, 128 23.0 / 11.0, 256 23.6 / 20.3; bf16 64
-// 24.5 / 5.9, 131 17.9 / 9.0 (56 in the scalar kernel), 512 24.0 / 21.5.
+// Short rows (at most 64 vectors: attention over a short context, a router's experts), of any length from one vector up
+// and any element alignment: 16 lanes hold a row, NV vectors per lane (placed as AnyRow's), four rows side by side in a
+// wave, and a wave takes SETS times four rows per step, so that lanes hold data and several loads are in flight where a
+// wave per row would have one, mostly empty. The reductions stay inside a 16-lane DPP row; no LDS and no barrier. Waves
+// are persistent and load their next rows while they work on these.
+// 65536 rows, us as a wave per row / here: fp32 8 columns 20.8 / 4.7, 64 22.5 / 6.5, 128 23.0 / 11.0, 256 23.6 / 20.3;
+// bf16 64 24.5 / 5.9, 131 17.9 / 9.0 (56 in the scalar kernel), 512 24.0 / 21.5.
 constexpr int kShortLanes = 16;
 
 template <typename Op>
@@ -480,7 +480,8 @@ __global__ void __launch_bounds__(256) softmax_coop_cell(int cell, unsigned iter
 // kernel is compiled without the loop (which costs registers: fewer resident workgroups).
 // ANY: rows of any length (nvec vectors, the last one partial) and element alignment. The row's last vector is moved
 // back to end with the row (AnyRow), its first `skip` elements being another lane's. fp32 chunks are held as x, and the
-// outputs are exp(x - M) / S with the division's remainder taken into account, as the row tier of such rows rounds them.
+// outputs are exp(x - M) / S with the division's remainder taken into account, as the row tier of such rows rounds
+// them.
 template <typename T, int WAVES, int NV, bool NTL, bool NTS, bool LOOP, bool ANY>
 __global__ void __launch_bounds__(WAVES * 64)
     softmax_coop(const void* __restrict__ x, void* __restrict__ y, long long rows, long long nvec, long long cols,
@@ -502,7 +503,8 @@ __global__ void __launch_bounds__(WAVES * 64)
   constexpr bool PREFETCH = LOOP && T::V == 8;
   constexpr bool HOLD = !(ANY && T::bytes == 4);  // the chunk is held as exp(x - m)
   Regs<NV> next;  // PREFETCH: the next row's raw chunk, loaded during the wait
-  // ANY: elements of the row from V before the chunk's first on; a vector past the row's last whole start is moved back to it
+  // ANY: elements of the row from V before the chunk's first on; a vector past the row's last whole start is moved back
+  // to it
   const int reach = (int)(cols - (long long)first * T::V);  // the chunk's first element to the row's end: >= 1
   auto offset = [&](int k, int t) __attribute__((always_inline)) {
     return (uint32_t)((least((k * G + t) * T::V, reach - T::V) + T::V) * T::bytes);
@@ -631,7 +633,8 @@ __global__ void __launch_bounds__(WAVES * 64)
         int skip = 0;
         if constexpr (ANY) {
           const int at = least((int)i * T::V, (int)cols - T::V);
-          unpack<T>(load16_at<false>(static_cast<const char*>(x) + row * cols * T::bytes, (uint32_t)(at * T::bytes)), f);
+          const char* base = static_cast<const char*>(x) + row * cols * T::bytes;
+          unpack<T>(load16_at<false>(base, (uint32_t)(at * T::bytes)), f);
           skip = (int)i * T::V - at;
         } else {
           unpack<T>(load16<false>(x, row * nvec + i), f);
@@ -798,11 +801,14 @@ int launch_any_k(const void* x, void* y, long long rows, int cols, hipStream_t s
   static int occ = 0;  // resident blocks per CU of this instantiation (idempotent cache)
   if (occ <= 0) occ = blocks_per_cu(kern, BW * kWave);
   int per_cu = rw_host::tune_get(kTuneBlocksPerCu);
-  // fp32 rows of four vectors a lane and more: the resident waves of launch_rows_k; otherwise about 24 waves per CU, whose
-  // loads are fewer or whose rows take more work per byte (8192 x 3001 fp32 as 4 waves x 4 vectors: 33.7 us with two
-  // blocks per CU, 34.8 with four; bf16 as 2 waves x 4 vectors: 17.3 with three, 16.9 with six; 65536 x 131 bf16: 23.5
-  // with two, 17.7 with six)
-  if (per_cu <= 0) per_cu = T::bytes == 4 && NV >= 4 ? (WAVES == 8 ? 2 : 8 / BW > 1 ? 8 / BW : 1) : (24 / BW > 1 ? 24 / BW : 1);
+  // fp32 rows of four vectors a lane and more: the resident waves of launch_rows_k; otherwise about 24 waves per CU,
+  // whose loads are fewer or whose rows take more work per byte (8192 x 3001 fp32 as 4 waves x 4 vectors: 33.7 us with
+  // two blocks per CU, 34.8 with four; bf16 as 2 waves x 4 vectors: 17.3 with three, 16.9 with six; 65536 x 131 bf16:
+  // 23.5 with two, 17.7 with six)
+  if (per_cu <= 0) {
+    const int resident = T::bytes == 4 && NV >= 4 ? (WAVES == 8 ? 16 : 8) : 24;
+    per_cu = resident / BW > 1 ? resident / BW : 1;
+  }
   if (per_cu > occ) per_cu = occ;
   const long long need = (rows + GROUPS - 1) / GROUPS;
   long long grid = (long long)rw_host::device_cus() * per_cu;
@@ -838,10 +844,12 @@ int launch_short_nv(const void* x, void* y, long long rows, int cols, hipStream_
   const long long cus = rw_host::device_cus(), waves = (rows + ROWS - 1) / ROWS;
   int per_cu = rw_host::tune_get(kTuneBlocksPerCu);
   if (per_cu <= 0) per_cu = 6;
-  const int per_block = waves >= 4 * cus ? 4 : 1;  // one wave per block until every CU has four: few rows spread over the GPU
+  // one wave per block until every CU has four: few rows then spread over the GPU
+  const int per_block = waves >= 4 * cus ? 4 : 1;
   long long grid = (waves + per_block - 1) / per_block;
   if (grid > cus * per_cu * 4 / per_block) grid = cus * per_cu * 4 / per_block;
-  hipLaunchKernelGGL((softmax_short<T, NV>), dim3((unsigned)grid), dim3(per_block * kWave), 0, stream, x, y, rows, cols);
+  hipLaunchKernelGGL((softmax_short<T, NV>), dim3((unsigned)grid), dim3(per_block * kWave), 0, stream, x, y, rows,
+                     cols);
   return (int)hipGetLastError();
 }
 
@@ -925,8 +933,8 @@ bool capturing(hipStream_t stream) {
   return status != hipStreamCaptureStatusNone;
 }
 
-// Co-resident tier with one row per workgroup: chunks of 4 waves x 64 lanes x NV vectors, when every row's chunks fit on
-// the GPU at once. Returns 1, launching nothing, when they do not (or a row has more than kCoopMaxChunks of them).
+// Co-resident tier with one row per workgroup: chunks of 4 waves x 64 lanes x NV vectors, when every row's chunks fit
+// on the GPU at once. Returns 1, launching nothing, when they do not (or a row has more than kCoopMaxChunks of them).
 struct CoopLaunch {
   const void* x;
   void* y;
@@ -979,8 +987,9 @@ int launch_coop_one(const CoopLaunch& a) {
 
 // Co-resident tier: chunks of 4 waves x 64 lanes x 64 elements (16 fp32 or 8 bf16 vectors per lane), at most
 // kCoopMaxChunks per row; shorter chunks (half or a quarter as long) when the rows are so few that the long ones would
-// leave CUs without a workgroup; row groups walking several rows (an instantiation of its own: the loop costs registers)
-// when the rows' chunks do not fit on the GPU at once. Returns 1, launching nothing, when one row's chunks do not fit.
+// leave CUs without a workgroup; row groups walking several rows (an instantiation of its own: the loop costs
+// registers) when the rows' chunks do not fit on the GPU at once. Returns 1, launching nothing, when one row's chunks
+// do not fit.
 template <typename T, bool NTL, bool ANY>
 int launch_coop(const CoopLaunch& a, bool single_only = false) {
   constexpr int NV = 64 / T::V;
@@ -1030,12 +1039,12 @@ bool row_shape_tuned() {
 }
 
 // Rows that the row tier could hold but the co-resident tier takes faster: rows of more than 4096 vectors, which in the
-// row tier are 16 waves x 8 vectors with registers spilled (bf16 always: 600 x 40000 34 -> 19.5 us, 1024 x 50000 56 -> 46,
-// 1024 x 65536 51 -> 50; fp32 when every row's chunks are resident at once: 256 x 32768 15.0 -> 11.0, 512 x 20000
+// row tier are 16 waves x 8 vectors with registers spilled (bf16 always: 600 x 40000 34 -> 19.5 us, 1024 x 50000 56 ->
+// 46, 1024 x 65536 51 -> 50; fp32 when every row's chunks are resident at once: 256 x 32768 15.0 -> 11.0, 512 x 20000
 // 19.0 -> 13.1, but 2048 x 32768 97 -> 103 in row groups), and rows of more than 2048 vectors when they are too few to
-// fill the GPU with one workgroup each (1 x 10000 fp32 4.5 -> 3.9, 16 x 32000 bf16 5.4 -> 4.2; 128 x 16384 fp32 6.0 either
-// way). A launch that is being captured stays in the row tier, which needs no second node and no tag cell, and so does
-// one in place (its callers look), where a timed-out wait's second read of the row would meet outputs.
+// fill the GPU with one workgroup each (1 x 10000 fp32 4.5 -> 3.9, 16 x 32000 bf16 5.4 -> 4.2; 128 x 16384 fp32 6.0
+// either way). A launch that is being captured stays in the row tier, which needs no second node and no tag cell, and
+// so does one in place (its callers look), where a timed-out wait's second read of the row would meet outputs.
 template <typename T>
 bool coop_instead_of_rows(long long rows, long long nvec, hipStream_t stream) {
   if (rw_host::tune_get(kTuneTier) != 0 || row_shape_tuned()) return false;

@@ -959,10 +959,10 @@ struct Tile {
     }
   }
 
-  // max_key() of an fp32 tile by way of the signed maxima gm of its groups of 8 elements, which filter_groups takes: the
-  // minima are looked at only when some lane of the wave holds no element from 0 up. About 60 of a wave's 590 vector
-  // instructions fewer (k = 50: 128 x 128256 18.34 -> 18.2 us, 64 x 151936 15.9 -> 15.65, 8 x 128256 9.6 -> 9.4). (The wide
-  // kernel's group keys without the minima measured 0.1 to 0.3 us slower.)
+  // max_key() of an fp32 tile by way of the signed maxima gm of its groups of 8 elements, which filter_groups takes:
+  // the minima are looked at only when some lane of the wave holds no element from 0 up. About 60 of a wave's 590
+  // vector instructions fewer (k = 50: 128 x 128256 18.34 -> 18.2 us, 64 x 151936 15.9 -> 15.65, 8 x 128256 9.6 ->
+  // 9.4). (The wide kernel's group keys without the minima measured 0.1 to 0.3 us slower.)
   __device__ __forceinline__ uint32_t max_key_groups(int (&gm)[NV / 2]) const {
     group_maxima(gm);
     int mx = INT_MIN;
@@ -2599,8 +2599,8 @@ __global__ void __launch_bounds__(kWave)
 // Rows of at most kShortCols columns (a router's experts, a reranker's candidates): topk_tile gives each a workgroup of
 // 256 lanes with 64 element registers apiece, nearly all of them padding. Here L lanes hold a row (16: four rows per
 // wave, reductions inside a DPP row; 64: one), E elements each, as words whose order is the composites' order:
-// fp32 (key << 32) | ~index, bf16 (the key's upper half << 16) | ~index in 32 bits, which makes an exchange of the lane's
-// sorting network one maximum and one minimum. A lane sorts its E words once; the row's next largest is then the
+// fp32 (key << 32) | ~index, bf16 (the key's upper half << 16) | ~index in 32 bits, which makes an exchange of the
+// lane's sorting network one maximum and one minimum. A lane sorts its E words once; the row's next largest is then the
 // largest of the lanes' heads, k times over, and its lane steps on to its next word. The row's k words go through LDS,
 // from which the wave stores its rows' values and indices as one contiguous piece each. Bound by instruction issue (at
 // 16384 x 128 fp32, k = 8: 1.6 us of memory traffic).
@@ -2674,7 +2674,8 @@ __global__ void __launch_bounds__(kThreads)
 #pragma unroll
       for (int i = 0; i < W; ++i) {
         const int e = (j * L + l) * W + i;
-        const uint32_t u = sizeof(T) == 4 ? v[j][i * sizeof(T) / 4] : (v[j][i * sizeof(T) / 4] >> (16 * (i & 1))) & 0xffffu;
+        const uint32_t word = v[j][i * sizeof(T) / 4];
+        const uint32_t u = sizeof(T) == 4 ? word : (word >> (16 * (i & 1))) & 0xffffu;
         c[j * W + i] = e < cols ? Wd::make(u, e) : 0;
       }
   } else {
@@ -2761,8 +2762,8 @@ __global__ void __launch_bounds__(kThreads)
 
 // ---- host side ------------------------------------------------------------------------------------------------------
 
-// Tuning slots (0 = automatic): 0 resident workgroups per CU assumed by plan(); 1 the naive tier for launch() (1); 2 the
-// short rows' kernel for every row it can hold (1) or for none (2).
+// Tuning slots (0 = automatic): 0 resident workgroups per CU assumed by plan(); 1 the naive tier for launch() (1); 2
+// the short rows' kernel for every row it can hold (1) or for none (2).
 enum { kTuneBlocksPerCu = 0, kTuneSeed = 1, kTuneShort = 2 };
 
 // The chunking a launch of the caller's nchunks chunks of `chunk` columns actually runs, and the u64 slots of the
@@ -2782,8 +2783,9 @@ enum { kTuneBlocksPerCu = 0, kTuneSeed = 1, kTuneShort = 2 };
 //    elements give it no bound (k <= 64: the exact re-push path; k > 64: it admits nearly everything). bf16: 64 x 50000
 //    k = 50 37.5 -> 10.4 us, 16 x 132352 k = 50 48 -> 10.8, 92 x 70753 k = 1024 64 -> 24; fp32: 143 x 33536 k = 50
 //    25.2 -> 11.5 us, 128 x 128256 unchanged. Not when that makes more register tiles in all (300 x 167148 fp32 in
-//    chunks of four tiles, k = 1024: 70.5 -> 75.5), nor when the last chunk is nearly as long as the others, nor for k > 64 below 10 k columns (a chunk's bound needs the group
-//    maxima of that many: 276 x 17664 fp32, k = 1024 as two chunks of 8832: 24 -> 50).
+//    chunks of four tiles, k = 1024: 70.5 -> 75.5), nor when the last chunk is nearly as long as the others, nor for k
+//    > 64 below 10 k columns (a chunk's bound needs the group maxima of that many: 276 x 17664 fp32, k = 1024 as two
+//    chunks of 8832: 24 -> 50).
 //  - 1 < k <= 64: a row of two chunks within two register tiles is taken whole by one workgroup, tile after tile,
 //    when there are at least as many rows as CUs (512 x 32000 fp32 at k = 50: 19.2 -> 17.6 us on MI355X; the chunks'
 //    hand-off and merge cost more than the second tile's wait, while one workgroup per row still fills the GPU).
@@ -2913,11 +2915,12 @@ int launch_short(const void* x, void* values, void* indices, long long rows, int
 }
 
 // Whether a plain launch takes the short rows' kernel: its time grows with k (a row's k steps are a serial chain of
-// about 0.1 us each, half of that for bf16's 32-bit words), so that for many columns and a large k the tile kernel is the
-// faster one until there are rows enough to hide the chain. Kernel times in us, tile kernel / this one:
+// about 0.1 us each, half of that for bf16's 32-bit words), so that for many columns and a large k the tile kernel is
+// the faster one until there are rows enough to hide the chain. Kernel times in us, tile kernel / this one:
 //   64 rows fp32: 128 columns k = 8 5.4 / 3.3, k = 64 10.2 / 8.9; 512 columns k = 32 5.6 / 7.4; 1024 columns k = 16
 //   5.5 / 6.4; bf16 512 columns k = 64 17.6 / 8.2, 1024 columns k = 32 6.0 / 6.6;
-//   16384 rows fp32: 128 columns k = 8 74.4 / 5.3; 512 columns k = 64 89 / 64; 1024 columns k = 32 77 / 50, k = 64 87 / 85.
+//   16384 rows fp32: 128 columns k = 8 74.4 / 5.3; 512 columns k = 64 89 / 64; 1024 columns k = 32 77 / 50, k = 64 87 /
+//   85.
 bool takes_short(long long rows, long long cols, int k, int dtype) {
   const int want = rw_host::tune_get(kTuneShort);
   if (cols > kShortCols || k > kShortK || want == 2) return false;

@@ -97,9 +97,10 @@ def _check(pkg, oracle, dev, rows, cols, dtype, offset=0, special=False):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("rows,cols", [(3, 8), (70, 9), (40000, 8), (5000, 63), (70001, 64), (16385, 131), (9000, 255),
-                                       (8191, 256), (8192, 257), (9001, 511), (20000, 512), (513, 255), (700, 513), (5, 2049), (300, 3001), (9, 8191),
-                                       (600, 16383), (3, 16384), (40, 20001), (2, 32767), (300, 20000), (5, 65535),
-                                       (3, 70001), (2, 262143), (70, 262143), (1, 1048576), (2, 1048577)])
+                                       (8191, 256), (8192, 257), (9001, 511), (20000, 512), (513, 255), (700, 513),
+                                       (5, 2049), (300, 3001), (9, 8191), (600, 16383), (3, 16384), (40, 20001), (2, 32767),
+                                       (300, 20000), (5, 65535), (3, 70001), (2, 262143), (70, 262143), (1, 1048576),
+                                       (2, 1048577)])
 def test_gpu_rows(pkg, oracle, dev, dtype, rows, cols):
     _check(pkg, oracle, dev, rows, cols, dtype, offset=1, special=True)
 

@@ -79,7 +79,8 @@ def test_gpu_any_rows(pkg, oracle, dev, dtype, rows, cols):
 def test_gpu_short_rows(pkg, oracle, dev, dtype, rows, cols):
     print(f"[rmsnorm short] {rows}x{cols} {dtype}", flush=True)
     g = torch.Generator().manual_seed(rows + cols)
-    x = (torch.randn(rows, cols, generator=g) * torch.rand(rows, 1, generator=g) * 3).to(dtype) + 0  # no -0: the weighted fp16 product of -0 comes out as +0 on the GPU
+    # (+ 0: no -0, whose weighted fp16 product comes out as +0 on the GPU)
+    x = (torch.randn(rows, cols, generator=g) * torch.rand(rows, 1, generator=g) * 3).to(dtype) + 0
     x[rows // 2, cols // 2] = float("nan")
     x[0] = 0
     w = (torch.rand(cols, generator=g) + 0.5).to(dtype)
