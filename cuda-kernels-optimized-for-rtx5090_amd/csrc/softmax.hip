@@ -543,7 +543,10 @@ __global__ void __launch_bounds__(WAVES * 64)
       for (int i = 0; i < T::V; ++i) m = ok ? fmaxf(m, f[i]) : m;
     }
     m = group_reduce<WAVES>(m, OpMax{}, slots[0], wave_id(), 0);
-    // the registers take e = exp(x - m) (0 for an all -inf chunk) in place of x: one exp per element
+    // the registers take e = exp(x - m) in place of x: one exp per element. A chunk of only -inf and NaN has m = -inf
+    // (fmaxf takes the other operand of a NaN); its elements are taken from 0 instead, -inf to 0 and NaN to NaN, so that
+    // a NaN reaches s, the row's S, and through it every output of the row
+    const float from = m == -INFINITY ? 0.0f : m;
     float e[HOLD ? NV : 1][T::V];
     float s = 0.0f;
 #pragma unroll
@@ -555,14 +558,14 @@ __global__ void __launch_bounds__(WAVES * 64)
         const int start = (k * G + t) * T::V;
 #pragma unroll
         for (int i = 0; i < T::V; ++i) {
-          f[i] = m != -INFINITY ? exp_below<T>(f[i] - m) : 0.0f;
+          f[i] = exp_below<T>(f[i] - from);
           if constexpr (HOLD) e[k][i] = f[i];
         }
         s += (k * G + wave0 + kWave) * T::V <= reach ? sum_vector<T>(f, 0)
                                                      : sum_vector<T>(f, start - least(start, reach - T::V));
       } else {
 #pragma unroll
-        for (int i = 0; i < T::V; ++i) e[k][i] = ok && m != -INFINITY ? exp_to<T>(f[i] - m) : 0.0f;
+        for (int i = 0; i < T::V; ++i) e[k][i] = ok ? exp_to<T>(f[i] - from) : 0.0f;
         s += sum_vector<T>(e[k], 0);
       }
     }
@@ -571,7 +574,7 @@ __global__ void __launch_bounds__(WAVES * 64)
     // whose raw chunk is half the size of e; for fp32 the two together would halve the resident workgroups)
     if constexpr (PREFETCH)
       if (it + 1 < iters) load_chunk(next, row + groups, t);
-    if (t == 0) {  // an all -inf chunk publishes (-inf, 0) and contributes nothing to the merge
+    if (t == 0) {  // an all -inf chunk publishes (-inf, 0), which adds nothing to the merge; with a NaN in it, (-inf, NaN)
       __hip_atomic_store(&table[c][0], tag | __float_as_uint(m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __hip_atomic_store(&table[c][1], tag | __float_as_uint(s), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -608,15 +611,13 @@ __global__ void __launch_bounds__(WAVES * 64)
       for (int i = 0; i < PER; ++i) {
         if (i * kWave + lane < chunks) {
           const float qm = __uint_as_float((unsigned)wm[i]), qs = __uint_as_float((unsigned)ws[i]);
-          const float mm = fmaxf(pm, qm);
-          if (mm != -INFINITY) {
-            ps = ps * expf(pm - mm) + qs * expf(qm - mm);
-            pm = mm;
-          }
+          const float mm = fmaxf(pm, qm), base = mm == -INFINITY ? 0.0f : mm;
+          ps = ps * expf(pm - base) + qs * expf(qm - base);
+          pm = mm;
         }
       }
       const float M = wave_max(pm);
-      const float S = wave_sum(M == -INFINITY ? ps : ps * expf(pm - M));
+      const float S = wave_sum(ps * expf(pm - (M == -INFINITY ? 0.0f : M)));  // (-inf, s): 0, or NaN where s is
       if (lane == 0) {
         ms[0] = M;
         ms[1] = S;
@@ -651,8 +652,7 @@ __global__ void __launch_bounds__(WAVES * 64)
         }
       }
       const float RM = group_reduce<WAVES>(tm, OpMax{}, slots[0], wave_id(), 0);
-      const float RS =
-          group_reduce<WAVES>(tm == -INFINITY ? 0.0f : ts * expf(tm - RM), OpSum{}, slots[1], wave_id(), 0);
+      const float RS = group_reduce<WAVES>(ts * expf(tm - (RM == -INFINITY ? 0.0f : RM)), OpSum{}, slots[1], wave_id(), 0);
       __syncthreads();  // every wave has read ms and the slots before they are written
       if (t == 0) {
         ms[0] = RM;
@@ -661,8 +661,8 @@ __global__ void __launch_bounds__(WAVES * 64)
       __syncthreads();
     }
     const float M = ms[0], S = ms[1];
-    // y = e * exp(m - M) / S; an all -inf chunk (e = 0) gives 0, or NaN when the whole row is -inf (M = -inf)
-    const float scale = m == -INFINITY ? (M == -INFINITY ? NAN : 0.0f) : expf(m - M) / S;
+    // y = e * exp(m - M) / S; an all -inf chunk (e = 0) gives 0, or NaN when the whole row is -inf (S = 0) or S is NaN
+    const float scale = (m == -INFINITY ? 0.0f : expf(m - M)) / S;
     const float inv = 1.0f / S;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {

@@ -8,8 +8,9 @@
 //   tier: 1 row, 2 stream, 3 generic, 4 co-resident (preferred through softmax_tune); waves / nv: the row tier's
 //   shape (tier 1), the stream tier's waves (tier 2), the co-resident tier's row groups in nv (tier 4; fewer groups
 //   than rows make each workgroup walk several rows), 0 automatic; offset shifts x and y by that many elements from a
-//   16-byte boundary; pattern: randn (N(0, 4)) or special (-inf elements,
-//   an all -inf row, a row of one huge value); reps: launches on the same buffers, each checked (the co-resident
+//   16-byte boundary; pattern: randn (N(0, 4)), special (-inf elements,
+//   an all -inf row, a row of one huge value) or nan (the middle half of every row masked: -inf with one NaN in it, all
+//   NaN, -inf with a NaN or a +inf elsewhere in the row, and only -inf); reps: launches on the same buffers, each checked (the co-resident
 //   tier's pair table is reused by the next launch, under fresh tags); wait_ticks bounds the co-resident tier's wait
 //   (1 makes its workgroups stop waiting and take the row's statistics from x).
 // EMU_GRAPH set: after an eager launch, the launch is recorded as a graph (the emulation's capture) and every rep
@@ -64,7 +65,7 @@ int main(int argc, char** argv) {
   }
   const size_t esz = dtype == 0 ? 4 : 2, n = (size_t)rows * cols;
   const bool graph = std::getenv("EMU_GRAPH") != nullptr;
-  if (pattern != "randn" && pattern != "special") {
+  if (pattern != "randn" && pattern != "special" && pattern != "nan") {
     std::fprintf(stderr, "unknown pattern %s\n", pattern.c_str());
     return 2;
   }
@@ -80,6 +81,12 @@ int main(int argc, char** argv) {
         if (r % 4 == 0 && c % 5 == 1) v = -INFINITY;
         if (r % 4 == 1) v = -INFINITY;
         if (r % 4 == 2 && c == cols / 2) v = 80.0f;
+      }
+      if (pattern == "nan") {
+        if (c >= cols / 4 && c < cols - cols / 4) v = r % 5 == 1 ? NAN : -INFINITY;
+        if (r % 5 == 0 && c == cols / 2) v = NAN;
+        if (r % 5 == 2 && c == cols - 1) v = NAN;
+        if (r % 5 == 3 && c == 0) v = INFINITY;
       }
       if (dtype == 0) std::memcpy(&host[i * 4], &v, 4);
       else {

@@ -64,6 +64,22 @@ def test_emulated_coresident_fallback(emu_softmax, rows, cols, dtype, groups):
     run(emu_softmax, [rows, cols, dtype, 4, 3, 0, groups, 1, "special", 2, 1])
 
 
+# rows whose middle half is masked, NaN among the masked elements or elsewhere: whole chunks of -inf and NaN. tier 0 is
+# the automatic choice (rows of the row tier's lengths that an eager launch hands to the co-resident tier), 4 the
+# co-resident tier; rows, cols, dtype, tier, row groups
+NAN_ROWS = [(2, 30000, 0, 0, 0), (2, 49999, 0, 0, 0), (2, 49152, 1, 0, 0), (2, 60001, 1, 0, 0), (5, 70000, 0, 4, 0),
+            (5, 70001, 0, 4, 0), (5, 49152, 1, 4, 0), (5, 49153, 1, 4, 0), (5, 70000, 0, 4, 2), (5, 70001, 0, 4, 2),
+            (5, 70000, 1, 4, 2), (5, 70001, 1, 4, 2)]
+
+
+@pytest.mark.parametrize("rows,cols,dtype,tier,groups", NAN_ROWS)
+@pytest.mark.parametrize("ticks", [0, 1], ids=["pairs", "fallback"])
+def test_emulated_coresident_nan(emu_softmax, rows, cols, dtype, tier, groups, ticks):
+    env = dict(os.environ) if ticks else dict(os.environ, EMU_CLOCK_STOPPED="1")
+    run(emu_softmax, [rows, cols, dtype, tier, 3, 0, groups, 0, "nan", 1, ticks], env=env, concurrent=not ticks,
+        timeout=300)
+
+
 def _check(pkg, oracle, dev, rows, cols, dtype, offset=0, special=False):
     print(f"[softmax any] {rows}x{cols} {dtype} offset {offset}", flush=True)
     g = torch.Generator().manual_seed(rows * 131 + cols)
@@ -111,6 +127,33 @@ def test_gpu_rows(pkg, oracle, dev, dtype, rows, cols):
 def test_gpu_offsets(pkg, oracle, dev, dtype, offset):
     for rows, cols in ((7, 1024), (7, 1027), (3, 40000)):
         _check(pkg, oracle, dev, rows, cols, dtype, offset=offset)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("rows,cols", [(5, 3001), (5, 4096), (5, 30000), (5, 49152), (5, 49999), (40, 70000), (5, 70001),
+                                       (300, 70000), (300, 70001)])
+@pytest.mark.parametrize("ticks", [0, 1])
+def test_gpu_nan_among_masked(pkg, oracle, dev, dtype, rows, cols, ticks):
+    # as test_emulated_coresident_nan: the row's middle half masked, in the row tiers and in the co-resident tier
+    print(f"[softmax nan] {rows}x{cols} {dtype} ticks {ticks}", flush=True)
+    x = torch.randn(rows, cols, generator=torch.Generator().manual_seed(cols)) * 3
+    x[:, cols // 4:cols - cols // 4] = float("-inf")
+    x[1::5, cols // 4:cols - cols // 4] = float("nan")
+    x[0::5, cols // 2] = float("nan")
+    x[2::5, cols - 1] = float("nan")
+    x[3::5, 0] = float("inf")
+    x = x.to(dtype)
+    lib = pkg.candidate("softmax")._lib
+    try:
+        lib.softmax_tune(7, ticks)
+        y = pkg.softmax(x.to(dev)).cpu()
+    finally:
+        lib.softmax_tune(7, 0)
+    if dtype == torch.float32:
+        assert_rel(y.numpy(), oracle.softmax(x.numpy(), "fp32"), 1e-5, "nan", 2.0 ** -147)
+    else:
+        assert_ulp(bits16(y), oracle.softmax(bits16(x), "bf16"), 1, "nan")
 
 
 @pytest.mark.gpu
