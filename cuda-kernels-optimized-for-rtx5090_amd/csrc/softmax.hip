@@ -387,20 +387,21 @@ __global__ void __launch_bounds__(WAVES * 64)
         for (int e = 0; e < T::V; ++e) cm = ok ? fmaxf(cm, f[u][e]) : cm;
       }
       if (cm > m) {  // rescale the running sum to the new maximum (-inf elements never raise it)
-        s = m == -INFINITY ? 0.0f : s * expf(m - cm);
+        s = s * expf(m - cm);
         m = cm;
       }
-      if (m != -INFINITY) {
+      // while there is no maximum, elements are taken from 0: -inf adds nothing, a NaN makes the sum NaN
+      const float from = m == -INFINITY ? 0.0f : m;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const bool ok = i0 + (long long)u * G + t < nvec;
+      for (int u = 0; u < U; ++u) {
+        const bool ok = i0 + (long long)u * G + t < nvec;
 #pragma unroll
-          for (int e = 0; e < T::V; ++e) s += ok ? exp_to<T>(f[u][e] - m) : 0.0f;
-        }
+        for (int e = 0; e < T::V; ++e) s += ok ? exp_to<T>(f[u][e] - from) : 0.0f;
       }
     }
     const float M = group_reduce<WAVES>(m, OpMax{}, slots[0], wave_id(), 0);
-    const float S = group_reduce<WAVES>(m == -INFINITY ? 0.0f : s * expf(m - M), OpSum{}, slots[1], wave_id(), 0);
+    const float S =
+        group_reduce<WAVES>(s * expf(m - (M == -INFINITY ? 0.0f : M)), OpSum{}, slots[1], wave_id(), 0);
     const float inv = 1.0f / S;  // an all -inf row: M = -inf, S = 0, and every output NaN (as the fp64 reference)
     for (long long i = t; i < nvec; i += G) {
       float f[T::V];

@@ -80,6 +80,12 @@ def test_emulated_coresident_nan(emu_softmax, rows, cols, dtype, tier, groups, t
         timeout=300)
 
 
+@pytest.mark.parametrize("rows,cols,dtype,waves", [(5, 4096, 0, 16), (5, 20000, 0, 4), (5, 8192, 1, 16), (5, 2048, 1, 4)])
+def test_emulated_stream_nan(emu_softmax, rows, cols, dtype, waves):
+    # with a vector or two per lane, some lanes hold masked elements only
+    run(emu_softmax, [rows, cols, dtype, 2, 3, waves, 0, 0, "nan"])
+
+
 def _check(pkg, oracle, dev, rows, cols, dtype, offset=0, special=False):
     print(f"[softmax any] {rows}x{cols} {dtype} offset {offset}", flush=True)
     g = torch.Generator().manual_seed(rows * 131 + cols)
@@ -132,7 +138,7 @@ def test_gpu_offsets(pkg, oracle, dev, dtype, offset):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("rows,cols", [(5, 3001), (5, 4096), (5, 30000), (5, 49152), (5, 49999), (40, 70000), (5, 70001),
-                                       (300, 70000), (300, 70001)])
+                                       (300, 70000), (300, 70001), (5, 1200000)])
 @pytest.mark.parametrize("ticks", [0, 1])
 def test_gpu_nan_among_masked(pkg, oracle, dev, dtype, rows, cols, ticks):
     # as test_emulated_coresident_nan: the row's middle half masked, in the row tiers and in the co-resident tier
