@@ -109,18 +109,19 @@ __device__ __forceinline__ float exp_narrow(float d) {
 template <typename T> __device__ __forceinline__ float exp_to(float d) { return exp_narrow(d); }
 template <> __device__ __forceinline__ float exp_to<F32>(float d) { return expf(d); }
 
-// expf's accuracy (about an ulp) in half its instructions, for d <= 0: d log2 e is split into an integer n and a
-// fraction of at most a half by fused multiply-adds, the hardware's exp2 takes the fraction and v_ldexp_f32 applies n
-// (results below the normal range stay subnormal). n is bounded from below, so that d = -inf gives 0; NaN stays NaN.
+// expf's accuracy (about an ulp) in half its instructions, for d <= 0: Cody and Waite's reduction of the argument in two
+// parts (Software Manual for the Elementary Functions, 1980). d log2 e = n + f with n the nearest integer, so that f is
+// at most a half; f is formed by fused multiply-adds from log2 e as fl32(log2 e) + (log2 e - fl32(log2 e)), whose first
+// product is exact; the hardware's exp2 takes f and v_ldexp_f32 applies n (results below the normal range stay
+// subnormal). n is bounded from below, so that d = -inf gives 0; NaN stays NaN.
 // 1024 x 16383 fp32 softmax 25.9 us with expf, 23.7 us with this, at the same distance from the fp64 softmax.
 __device__ __forceinline__ float exp_nonpositive(float d) {
-  const float n = fmaxf(__builtin_rintf(d * 1.44269504088896341f), -300.0f);
-  const float f = __builtin_fmaf(d, 1.92596298909109e-8f, __builtin_fmaf(d, 1.4426950216293335f, -n));
+  constexpr double kLog2E = 1.4426950408889634;
+  constexpr float kHigh = (float)kLog2E, kLow = (float)(kLog2E - (double)kHigh);
+  const float n = fmaxf(__builtin_rintf(d * kHigh), -300.0f);
+  const float f = __builtin_fmaf(d, kLow, __builtin_fmaf(d, kHigh, -n));
   return __builtin_ldexpf(__builtin_amdgcn_exp2f(f), (int)n);
 }
-// The exponential of d <= 0 for outputs of format T.
-template <typename T> __device__ __forceinline__ float exp_below(float d) { return exp_narrow(d); }
-template <> __device__ __forceinline__ float exp_below<F32>(float d) { return exp_nonpositive(d); }
 
 // Scalar element access (unaligned / ragged paths).
 template <typename T> __device__ __forceinline__ float load_elem(const void* p, long long i);

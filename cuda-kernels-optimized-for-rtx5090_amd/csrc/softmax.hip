@@ -19,8 +19,10 @@
 // The library allocates no device memory: the co-resident tier exchanges its chunk pairs through a static device
 // table whose entries carry a per-launch tag, so nothing has to be cleared between launches; launches recorded into a
 // HIP graph take fresh tags at every replay (see softmax_coop).
-// The normalisation multiplies by the fp32 reciprocal of the row sum (the reference divides, softmax/kernel.cu:240;
-// the two differ by at most 1.5 ulp in fp32 and are within the 1e-5 relative tolerance of the fp64 oracle).
+// Aligned rows of the row tier and the stream tier multiply by the fp32 reciprocal of the row sum (the reference divides,
+// softmax/kernel.cu:240; the two differ by at most 1.5 ulp in fp32 and are within the 1e-5 relative tolerance of the
+// fp64 oracle); rows of other lengths and alignments, short fp32 rows and the fp32 chunks held as x take the quotient
+// (quotient below), the generic tier the division.
 #include <climits>
 #include <cmath>
 #include <mutex>
@@ -112,13 +114,11 @@ __device__ __forceinline__ float sum_vector(const float (&f)[T::V], int skip) {
   return a[0];
 }
 
-// e / s within a correctly rounded division's last bit, from inv = 1 / s: the product and one step of its remainder for
-// fp32 results; for 16-bit results the product alone, whose fp32 ulp their rounding does not see.
-template <typename T>
+// e / s within a correctly rounded division's last bit, from inv = 1 / s: the product, corrected by its remainder (one
+// Newton step of the quotient).
 __device__ __forceinline__ float quotient(float e, float s, float inv) {
   const float q = e * inv;
-  if constexpr (T::bytes == 2) return q;
-  else return __builtin_fmaf(__builtin_fmaf(-q, s, e), inv, q);
+  return __builtin_fmaf(__builtin_fmaf(-q, s, e), inv, q);
 }
 
 template <typename T, int WAVES, int NV, bool FULL, bool NTS>
@@ -174,7 +174,9 @@ __global__ void __launch_bounds__((WAVES < 4 ? 4 : WAVES) * 64)
 // elements are then another lane's (the same bits, and the same results when they are stored twice), so the maximum
 // takes every loaded element and the sum leaves out the first `skip` of the vector; only the wave that holds the row's
 // end looks at that, and vectors that lie past the end for a whole wave are not worked on.
-// 8192 x 3001 bf16 55.5 us through the scalar kernel's three passes of 2-byte accesses, 16.9 us here.
+// 8192 x 3001 bf16 62.1 us through the scalar kernel's three passes of 2-byte accesses, 18.3 us here (17.0 with
+// exp_narrow and the reciprocal, which round 1.3e-4 of the distinct values of a row otherwise than the fp64 softmax; the
+// scalar kernel's expf and division 0.45e-4, as here).
 template <typename T, int WAVES, int NV>
 struct AnyRow {
   static constexpr int G = WAVES * kWave, V = T::V;
@@ -209,7 +211,7 @@ struct AnyRow {
       s[k] = 0.0f;
       if (!used(k)) continue;
 #pragma unroll
-      for (int i = 0; i < V; ++i) f[k][i] = exp_below<T>(f[k][i] - m);
+      for (int i = 0; i < V; ++i) f[k][i] = exp_nonpositive(f[k][i] - m);
       s[k] = whole(k) ? sum_vector<T>(f[k], 0) : sum_vector<T>(f[k], start(k) - offset(k));
     }
 #pragma unroll
@@ -223,7 +225,7 @@ struct AnyRow {
     for (int k = 0; k < NV; ++k) {
       if (!active || start(k) >= cols) continue;
 #pragma unroll
-      for (int i = 0; i < V; ++i) f[k][i] = quotient<T>(f[k][i], sum, inv);
+      for (int i = 0; i < V; ++i) f[k][i] = quotient(f[k][i], sum, inv);
       store16_at<true>(base, (uint32_t)(offset(k) * T::bytes), pack<T>(f[k]));
     }
   }
@@ -267,7 +269,9 @@ __global__ void __launch_bounds__((WAVES < 4 ? 4 : WAVES) * 64)
 // wave per row would have one, mostly empty. The reductions stay inside a 16-lane DPP row; no LDS and no barrier. Waves
 // are persistent and load their next rows while they work on these.
 // 65536 rows, us as a wave per row / here: fp32 8 columns 20.8 / 4.7, 64 22.5 / 6.5, 128 23.0 / 11.0, 256 23.6 / 20.3;
-// bf16 64 24.5 / 5.9, 131 17.9 / 9.0 (56 in the scalar kernel), 512 24.0 / 21.5.
+// bf16 64 24.5 / 5.9, 131 17.9 / 10.5 (55 in the scalar kernel), 512 24.0 / 21.5.
+// FINE: the exponential and the quotient within an fp32 ulp (fp32 rows, and bf16 rows that would otherwise take the
+// scalar kernel); without it exp_narrow and the reciprocal, as in the row tier (65536 x 64 bf16 5.5 us, FINE 6.7).
 constexpr int kShortLanes = 16;
 
 template <typename Op>
@@ -278,7 +282,7 @@ __device__ __forceinline__ float short_reduce(float v, Op op) {
   return op(v, dpp<kDppMirror>(v));
 }
 
-template <typename T, int NV>
+template <typename T, int NV, bool FINE>
 __global__ void __launch_bounds__(256)
     softmax_short(const void* __restrict__ x, void* __restrict__ y, long long rows, int cols) {
   constexpr int V = T::V, SIDE = kWave / kShortLanes, SETS = NV == 1 ? 4 : 2;
@@ -321,7 +325,7 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
       for (int k = 0; k < NV; ++k) {
 #pragma unroll
-        for (int i = 0; i < V; ++i) f[k][i] = exp_below<T>(f[k][i] - m);
+        for (int i = 0; i < V; ++i) f[k][i] = FINE ? exp_nonpositive(f[k][i] - m) : exp_narrow(f[k][i] - m);
         p[k] = sum_vector<T>(f[k], start(k) - least(start(k), cols - V));
       }
 #pragma unroll
@@ -335,7 +339,7 @@ __global__ void __launch_bounds__(256)
       for (int k = 0; k < NV; ++k) {
         if (!in || start(k) >= cols) continue;
 #pragma unroll
-        for (int i = 0; i < V; ++i) f[k][i] = quotient<T>(f[k][i], sum, inv);
+        for (int i = 0; i < V; ++i) f[k][i] = FINE ? quotient(f[k][i], sum, inv) : f[k][i] * inv;
         store16_at<true>(base, at(first, u, k), pack<T>(f[k]));
       }
     }
@@ -480,10 +484,17 @@ __global__ void __launch_bounds__(256) softmax_coop_cell(int cell, unsigned iter
 // LOOP: some row group has more than one row (groups < rows); without it every workgroup takes one row, and the
 // kernel is compiled without the loop (which costs registers: fewer resident workgroups).
 // ANY: rows of any length (nvec vectors, the last one partial) and element alignment. The row's last vector is moved
-// back to end with the row (AnyRow), its first `skip` elements being another lane's. fp32 chunks are held as x, and the
-// outputs are exp(x - M) / S with the division's remainder taken into account, as the row tier of such rows rounds
-// them.
-template <typename T, int WAVES, int NV, bool NTL, bool NTS, bool LOOP, bool ANY>
+// back to end with the row (AnyRow), its first `skip` elements being another lane's.
+// FINE: the exponential within an fp32 ulp, for fp32 rows and for the bf16 rows that an eager launch takes from the
+// scalar kernel or the row tier; bf16 rows longer than the row tier holds take exp_narrow. (Share of a bf16 row's
+// distinct values that are rounded otherwise than the fp64 softmax's: 512 x 40000 aligned 1.27e-4 in the row tier, here
+// 1.40e-4 with exp_narrow and 0.59e-4 FINE; unaligned 0.59e-4 in the scalar kernel and here.)
+// HOLD: the chunk is held as e = exp(x - m) and written as e * (exp(m - M) / S); otherwise it is held as x, and the
+// exponential is taken again from M. Holding e saves an exponential per element, which long chunks of many rows feel
+// (1024 x 50000 fp32 77 us against 84, bf16 44 against 50), and costs fp32 rows accuracy where the chunk is short
+// (mean relative error of 16 x 128256 fp32: 1.47e-7 in four times longer chunks, 1.57e-7 as e, 1.03e-7 from x). So
+// short chunks and unaligned fp32 rows are held as x.
+template <typename T, int WAVES, int NV, bool NTL, bool NTS, bool LOOP, bool ANY, bool FINE>
 __global__ void __launch_bounds__(WAVES * 64)
     softmax_coop(const void* __restrict__ x, void* __restrict__ y, long long rows, long long nvec, long long cols,
                  int chunks, int groups, int slot0, unsigned tag0, int cell, unsigned wait_ticks) {
@@ -502,7 +513,8 @@ __global__ void __launch_bounds__(WAVES * 64)
   const int wave0 = __builtin_amdgcn_readfirstlane(t0 & ~(kWave - 1));
   const int iters = (int)((rows - group + groups - 1) / groups);
   constexpr bool PREFETCH = LOOP && T::V == 8;
-  constexpr bool HOLD = !(ANY && T::bytes == 4);  // the chunk is held as exp(x - m)
+  constexpr bool HOLD = NV == 64 / T::V && !(ANY && T::bytes == 4);
+  auto exp_of = [](float d) __attribute__((always_inline)) { return FINE ? exp_nonpositive(d) : exp_narrow(d); };
   Regs<NV> next;  // PREFETCH: the next row's raw chunk, loaded during the wait
   // ANY: elements of the row from V before the chunk's first on; a vector past the row's last whole start is moved back
   // to it
@@ -544,9 +556,8 @@ __global__ void __launch_bounds__(WAVES * 64)
       for (int i = 0; i < T::V; ++i) m = ok ? fmaxf(m, f[i]) : m;
     }
     m = group_reduce<WAVES>(m, OpMax{}, slots[0], wave_id(), 0);
-    // the registers take e = exp(x - m) in place of x: one exp per element. A chunk of only -inf and NaN has m = -inf
-    // (fmaxf takes the other operand of a NaN); its elements are taken from 0 instead, -inf to 0 and NaN to NaN, so that
-    // a NaN reaches s, the row's S, and through it every output of the row
+    // a chunk of only -inf and NaN has m = -inf (fmaxf takes the other operand of a NaN): its elements are taken from 0
+    // instead, -inf to 0 and NaN to NaN, so that a NaN reaches s, the row's S, and through it every output of the row
     const float from = m == -INFINITY ? 0.0f : m;
     float e[HOLD ? NV : 1][T::V];
     float s = 0.0f;
@@ -555,24 +566,22 @@ __global__ void __launch_bounds__(WAVES * 64)
       float f[T::V];
       unpack<T>(r.v[k], f);
       const bool ok = k * G + t < count;
-      if constexpr (ANY) {
-        const int start = (k * G + t) * T::V;
 #pragma unroll
-        for (int i = 0; i < T::V; ++i) {
-          f[i] = exp_below<T>(f[i] - from);
-          if constexpr (HOLD) e[k][i] = f[i];
-        }
-        s += (k * G + wave0 + kWave) * T::V <= reach ? sum_vector<T>(f, 0)
-                                                     : sum_vector<T>(f, start - least(start, reach - T::V));
-      } else {
-#pragma unroll
-        for (int i = 0; i < T::V; ++i) e[k][i] = ok ? exp_to<T>(f[i] - from) : 0.0f;
-        s += sum_vector<T>(e[k], 0);
+      for (int i = 0; i < T::V; ++i) {
+        f[i] = exp_of(f[i] - from);
+        if (!ANY) f[i] = ok ? f[i] : 0.0f;
+        if (HOLD) e[k][i] = f[i];
       }
+      int skip = 0;  // ANY: the first elements of the vector, another lane's
+      if (ANY && (k * G + wave0 + kWave) * T::V > reach) {
+        const int start = (k * G + t) * T::V;
+        skip = start - least(start, reach - T::V);
+      }
+      s += sum_vector<T>(f, skip);
     }
     s = group_reduce<WAVES>(s, OpSum{}, slots[1], wave_id(), 0);
-    // x is now held as e: the next row's loads go out before the wait and the stores, into the freed registers (bf16,
-    // whose raw chunk is half the size of e; for fp32 the two together would halve the resident workgroups)
+    // the next row's loads go out before the wait and the stores (bf16; for fp32 the two chunks together would halve the
+    // resident workgroups)
     if constexpr (PREFETCH)
       if (it + 1 < iters) load_chunk(next, row + groups, t);
     if (t == 0) {  // an all -inf chunk publishes (-inf, 0), which adds nothing to the merge; with a NaN in it, (-inf, NaN)
@@ -662,21 +671,19 @@ __global__ void __launch_bounds__(WAVES * 64)
       __syncthreads();
     }
     const float M = ms[0], S = ms[1];
-    // y = e * exp(m - M) / S; an all -inf chunk (e = 0) gives 0, or NaN when the whole row is -inf (S = 0) or S is NaN
-    const float scale = (m == -INFINITY ? 0.0f : expf(m - M)) / S;
-    const float inv = 1.0f / S;
+    // HOLD: an all -inf chunk (e = 0) gives 0, or NaN when the whole row is -inf (S = 0) or S is NaN
+    const float scale = HOLD ? (m == -INFINITY ? 0.0f : expf(m - M)) / S : 1.0f / S;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
       const int i = k * G + t;
       if (i < count) {
         float f[T::V];
-        if constexpr (HOLD) {
+        if constexpr (!HOLD) unpack<T>(r.v[k], f);
 #pragma unroll
-          for (int j = 0; j < T::V; ++j) f[j] = e[k][j] * scale;
-        } else {
-          unpack<T>(r.v[k], f);
-#pragma unroll
-          for (int j = 0; j < T::V; ++j) f[j] = quotient<T>(exp_below<T>(f[j] - M), S, inv);
+        for (int j = 0; j < T::V; ++j) {
+          if constexpr (HOLD) f[j] = e[k][j] * scale;
+          else if constexpr (FINE) f[j] = quotient(exp_of(f[j] - M), S, scale);
+          else f[j] = exp_of(f[j] - M) * scale;
         }
         if constexpr (ANY) store16_at<NTS>(static_cast<char*>(y) + chunk_base(row), offset(k, t), pack<T>(f));
         else store16<NTS>(y, row * nvec + first + i, pack<T>(f));
@@ -839,7 +846,7 @@ int launch_any(int waves, int nv, const void* x, void* y, long long rows, int co
   }
 }
 
-template <typename T, int NV>
+template <typename T, int NV, bool FINE>
 int launch_short_nv(const void* x, void* y, long long rows, int cols, hipStream_t stream) {
   constexpr int ROWS = (NV == 1 ? 4 : 2) * (kWave / kShortLanes);
   const long long cus = rw_host::device_cus(), waves = (rows + ROWS - 1) / ROWS;
@@ -849,17 +856,17 @@ int launch_short_nv(const void* x, void* y, long long rows, int cols, hipStream_
   const int per_block = waves >= 4 * cus ? 4 : 1;
   long long grid = (waves + per_block - 1) / per_block;
   if (grid > cus * per_cu * 4 / per_block) grid = cus * per_cu * 4 / per_block;
-  hipLaunchKernelGGL((softmax_short<T, NV>), dim3((unsigned)grid), dim3(per_block * kWave), 0, stream, x, y, rows,
+  hipLaunchKernelGGL((softmax_short<T, NV, FINE>), dim3((unsigned)grid), dim3(per_block * kWave), 0, stream, x, y, rows,
                      cols);
   return (int)hipGetLastError();
 }
 
-template <typename T>
+template <typename T, bool FINE>
 int launch_short(const void* x, void* y, long long rows, long long cols, hipStream_t stream) {
   const long long nvec = (cols + T::V - 1) / T::V;
-  if (nvec <= kShortLanes) return launch_short_nv<T, 1>(x, y, rows, (int)cols, stream);
-  if (nvec <= 2 * kShortLanes) return launch_short_nv<T, 2>(x, y, rows, (int)cols, stream);
-  return launch_short_nv<T, 4>(x, y, rows, (int)cols, stream);
+  if (nvec <= kShortLanes) return launch_short_nv<T, 1, FINE>(x, y, rows, (int)cols, stream);
+  if (nvec <= 2 * kShortLanes) return launch_short_nv<T, 2, FINE>(x, y, rows, (int)cols, stream);
+  return launch_short_nv<T, 4, FINE>(x, y, rows, (int)cols, stream);
 }
 
 template <typename T, int WAVES>
@@ -973,9 +980,9 @@ int launch_coop_k(Kernel kern, const CoopLaunch& a, long long chunks, long long 
   return (int)hipGetLastError();
 }
 
-template <typename T, int NV, bool NTL, bool ANY>
+template <typename T, int NV, bool NTL, bool ANY, bool FINE>
 int launch_coop_one(const CoopLaunch& a) {
-  auto one = softmax_coop<T, kCoopWaves, NV, NTL, true, false, ANY>;
+  auto one = softmax_coop<T, kCoopWaves, NV, NTL, true, false, ANY, FINE>;
   static int occ = 0;  // resident blocks per CU (idempotent cache)
   if (occ <= 0) occ = blocks_per_cu(one, kCoopWaves * kWave);
   constexpr long long CH = (long long)kCoopWaves * kWave * NV;
@@ -991,8 +998,8 @@ int launch_coop_one(const CoopLaunch& a) {
 // leave CUs without a workgroup; row groups walking several rows (an instantiation of its own: the loop costs
 // registers) when the rows' chunks do not fit on the GPU at once. Returns 1, launching nothing, when one row's chunks
 // do not fit.
-template <typename T, bool NTL, bool ANY>
-int launch_coop(const CoopLaunch& a, bool single_only = false) {
+template <typename T, bool NTL, bool ANY, bool FINE>
+int launch_coop(const CoopLaunch& a, int most_iters = INT_MAX) {
   constexpr int NV = 64 / T::V;
   constexpr long long CH = (long long)kCoopWaves * kWave * NV;
   const int want = rw_host::tune_get(kTuneCoopGroups);
@@ -1005,13 +1012,12 @@ int launch_coop(const CoopLaunch& a, bool single_only = false) {
       while (nv > NV / 4 && grid(nv) < kCoopFill<T> * cus) nv /= 2;
     }
     int rc = 1;  // a shape whose chunks are too many for the GPU or for a row takes the next longer chunks
-    if (nv == NV / 4) rc = launch_coop_one<T, NV / 4, NTL, ANY>(a);
-    if (rc == 1 && nv <= NV / 2) rc = launch_coop_one<T, NV / 2, NTL, ANY>(a);
-    if (rc == 1) rc = launch_coop_one<T, NV, NTL, ANY>(a);
+    if (nv == NV / 4) rc = launch_coop_one<T, NV / 4, NTL, ANY, FINE>(a);
+    if (rc == 1 && nv <= NV / 2) rc = launch_coop_one<T, NV / 2, NTL, ANY, FINE>(a);
+    if (rc == 1) rc = launch_coop_one<T, NV, NTL, ANY, FINE>(a);
     if (rc != 1) return rc;
   }
-  if (single_only) return 1;
-  auto loop = softmax_coop<T, kCoopWaves, NV, NTL, true, true, ANY>;
+  auto loop = softmax_coop<T, kCoopWaves, NV, NTL, true, true, ANY, FINE>;
   static int occ = 0;  // resident blocks per CU (idempotent cache)
   if (occ <= 0) occ = blocks_per_cu(loop, kCoopWaves * kWave);
   const long long chunks = (a.nvec + CH - 1) / CH;
@@ -1021,6 +1027,7 @@ int launch_coop(const CoopLaunch& a, bool single_only = false) {
   long long groups = slots / chunks;
   if (want > 0 && want < groups) groups = want;
   if (groups > a.rows) groups = a.rows;
+  if ((a.rows + groups - 1) / groups > most_iters) return 1;
   return launch_coop_k(loop, a, chunks, groups);
 }
 
@@ -1040,10 +1047,12 @@ bool row_shape_tuned() {
 }
 
 // Rows that the row tier could hold but the co-resident tier takes faster: rows of more than 4096 vectors, which in the
-// row tier are 16 waves x 8 vectors with registers spilled (bf16 always: 600 x 40000 34 -> 19.5 us, 1024 x 50000 56 ->
-// 46, 1024 x 65536 51 -> 50; fp32 when every row's chunks are resident at once: 256 x 32768 15.0 -> 11.0, 512 x 20000
-// 19.0 -> 13.1, but 2048 x 32768 97 -> 103 in row groups), and rows of more than 2048 vectors when they are too few to
-// fill the GPU with one workgroup each (1 x 10000 fp32 4.5 -> 3.9, 16 x 32000 bf16 5.4 -> 4.2; 128 x 16384 fp32 6.0
+// row tier are 16 waves x 8 vectors, with registers spilled unless the row fills them (bf16: 600 x 40000 33.5 -> 22.1
+// us, 1024 x 50000 55.2 -> 49.3, 3000 x 64000 177 -> 145; full rows of 65536 as long as a workgroup has at most three,
+// 400 rows 21.9 -> 19.3, 600 rows 30.5 -> 27.4, but 1024 rows 50.1 -> 52.3; fp32 when every row's chunks are resident
+// at once: 256 x 32768 15.0 -> 12.2, 512 x 20000 19.0 -> 15.8, but 2048 x 32768 97 -> 103 in row groups), and rows of
+// more than 2048 vectors when they are too few to
+// fill the GPU with one workgroup each (1 x 10000 fp32 4.5 -> 3.7, 16 x 32768 bf16 4.8 -> 4.2; 128 x 16384 fp32 6.0
 // either way). A launch that is being captured stays in the row tier, which needs no second node and no tag cell, and
 // so does one in place (its callers look), where a timed-out wait's second read of the row would meet outputs.
 template <typename T>
@@ -1062,16 +1071,17 @@ int launch_typed(const void* x, void* y, long long rows, long long cols, hipStre
   // (four vectors per lane: only with rows enough to keep the GPU full at eight to a wave; 4096 x 257 bf16 3.7 us as a
   // wave per row, 4.3 as short rows; 65536 x 257 19.1 and 17.5)
   if (any && nvec <= (rows >= 8192 ? 4 : 2) * kShortLanes && tier == 0 && !row_shape_tuned())
-    return launch_short<T>(x, y, rows, cols, stream);
+    return vec ? launch_short<T, T::bytes == 4>(x, y, rows, cols, stream)
+               : launch_short<T, true>(x, y, rows, cols, stream);
   if (!vec) {
     const CoopLaunch coop{x, y, rows, nvec, cols, stream};
     if (nvec > (long long)kMaxWaves * kWave * kMaxNv || tier == 4) {
       // (in place, a workgroup whose wait timed out would read a row that others have begun to overwrite)
-      const int rc = x != y ? launch_coop<T, false, true>(coop) : 1;
+      const int rc = x != y ? launch_coop<T, false, true, true>(coop) : 1;
       return rc != 1 ? rc : launch_generic<T>(x, y, rows, cols, stream);
     }
     if (x != y && coop_instead_of_rows<T>(rows, nvec, stream)) {
-      const int rc = launch_coop<T, false, true>(coop, T::bytes == 4);
+      const int rc = launch_coop<T, false, true, true>(coop, T::bytes == 4 ? 1 : INT_MAX);
       if (rc != 1) return rc;
     }
     int waves = rw_host::tune_get(kTuneWaves), nv = rw_host::tune_get(kTuneNv);
@@ -1091,8 +1101,8 @@ int launch_typed(const void* x, void* y, long long rows, long long cols, hipStre
   if (tier == 2) return launch_stream<T>(x, y, rows, nvec, stream);
   const CoopLaunch coop{x, y, rows, nvec, cols, stream};
   if (x != y && nvec <= (long long)kMaxWaves * kWave * kMaxNv && coop_instead_of_rows<T>(rows, nvec, stream)) {
-    // fp32 rows keep the row tier's rounding (x held, the exponential taken again): the instantiation for any rows
-    const int rc = T::bytes == 4 ? launch_coop<T, false, true>(coop, true) : launch_coop<T, false, false>(coop);
+    const int iters = T::bytes == 4 ? 1 : nvec == (long long)kMaxWaves * kWave * kMaxNv ? 3 : INT_MAX;
+    const int rc = launch_coop<T, false, false, true>(coop, iters);
     if (rc != 1) return rc;
   }
   const bool ntl = rw_host::tune_get(kTuneNtLoads) == 1;
@@ -1121,7 +1131,8 @@ int launch_typed(const void* x, void* y, long long rows, long long cols, hipStre
                  : launch_rows<T, false>(waves, nv, x, y, rows, nvec, stream);
     }
   }
-  const int rc = ntl ? launch_coop<T, true, false>(coop) : launch_coop<T, false, false>(coop);
+  constexpr bool kFine = T::bytes == 4;
+  const int rc = ntl ? launch_coop<T, true, false, kFine>(coop) : launch_coop<T, false, false, kFine>(coop);
   if (rc != 1) return rc;
   return launch_stream<T>(x, y, rows, nvec, stream);
 }

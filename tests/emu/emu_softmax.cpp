@@ -109,6 +109,8 @@ int main(int argc, char** argv) {
   oracle_softmax(host.data(), ref.data(), rows, cols, dtype);
   int err = 0;
   long long bad = 0, first = -1;
+  long long other = 0;  // elements whose bits are not the oracle's
+  double error = 0.0;   // fp32: the sum of the relative errors of elements in the normal range
   emu::Graph recorded;
   if (graph) {
     // an eager launch first (a warm-up, as a graph capture usually follows one), then the capture
@@ -145,6 +147,7 @@ int main(int argc, char** argv) {
         std::memcpy(&b, &ref[i * 4], 4);
         // below the normal range one ulp (2^-149) is more than 1e-5 of the value: one ulp is allowed there
         const double tol = std::fmax(1e-5 * std::fabs((double)b), 0x1p-149);
+        if (std::fabs(b) >= 0x1p-126f) error += std::fabs((double)a - b) / std::fabs((double)b);
         ok = std::isnan(b) ? std::isnan(a) : std::fabs((double)a - b) <= tol;
       } else {
         uint16_t a, b;
@@ -152,12 +155,14 @@ int main(int argc, char** argv) {
         std::memcpy(&b, &ref[i * 2], 2);
         ok = nan16(b) ? nan16(a) : !nan16(a) && std::abs(ordered(a) - ordered(b)) <= 1;
       }
+      other += std::memcmp(y + i * esz, &ref[i * esz], esz) != 0;
       if (!ok && first < 0) first = (long long)i;
       bad += !ok;
     }
   }
   const bool input_kept = std::memcmp(x, host.data(), n * esz) == 0;
   const bool ok = !err && !bad && input_kept;
+  std::printf("other bits %lld of %lld, mean error %.4e\n", other, (long long)n * reps, error / (n * reps));
   std::printf("rows %lld cols %lld dtype %d tier %d: %s (err %d, %lld outside tolerance, first %lld, input kept %d)\n",
               rows, cols, dtype, tier, ok ? "ALL OK" : "FAILED", err, bad, first, input_kept);
   hipFree(xb);

@@ -80,6 +80,19 @@ def test_emulated_coresident_nan(emu_softmax, rows, cols, dtype, tier, groups, t
         timeout=300)
 
 
+# bf16 rows by expf and a division (the scalar kernel) or in the row tier before the vector tiers took them: 32-bit
+# arithmetic is off by a few 2^-24 before the one rounding to bf16, whose boundaries lie 1 / 185 of the value's inverse
+# apart on the mean: 3.2e-7 on the mean rounds 6e-5 of the elements otherwise (exp_narrow's error 1.3e-4 and more)
+BITS = [(2000, 200, 1), (9000, 500, 1), (400, 1000, 1), (300, 1001, 0), (600, 301, 0), (12, 40000, 0), (12, 40001, 0)]
+
+
+@pytest.mark.parametrize("rows,cols,offset", BITS)
+def test_emulated_bf16_rounding(emu_softmax, rows, cols, offset):
+    env = dict(os.environ, EMU_CLOCK_STOPPED="1")
+    out = run(emu_softmax, [rows, cols, 1, 0, 1, 0, 0, offset], env=env, concurrent=cols > 32768)
+    assert int(out.split("other bits ")[1].split()[0]) <= 6e-5 * rows * cols, out
+
+
 @pytest.mark.parametrize("rows,cols,dtype,waves", [(5, 4096, 0, 16), (5, 20000, 0, 4), (5, 8192, 1, 16), (5, 2048, 1, 4)])
 def test_emulated_stream_nan(emu_softmax, rows, cols, dtype, waves):
     # with a vector or two per lane, some lanes hold masked elements only
@@ -160,6 +173,47 @@ def test_gpu_nan_among_masked(pkg, oracle, dev, dtype, rows, cols, ticks):
         assert_rel(y.numpy(), oracle.softmax(x.numpy(), "fp32"), 1e-5, "nan", 2.0 ** -147)
     else:
         assert_ulp(bits16(y), oracle.softmax(bits16(x), "bf16"), 1, "nan")
+
+
+def _fp64(rows, cols, dtype, offset, seed, dev):
+    """x at an offset into its buffer, and its softmax in fp64."""
+    g = torch.Generator(device=dev).manual_seed(seed)
+    buf = torch.empty(rows * cols + offset, device=dev, dtype=dtype)
+    x = buf[offset:].view(rows, cols)
+    x.copy_(torch.randn(rows, cols, device=dev, generator=g) * (3 if dtype == torch.bfloat16 else 1))
+    return x, torch.softmax(x.double(), -1)
+
+
+def _softmax_at(pkg, x, offset):
+    y = torch.empty(x.numel() + offset, device=x.device, dtype=x.dtype)[offset:].view_as(x)
+    assert pkg.candidate("softmax")._lib.launch(x.data_ptr(), y.data_ptr(), *x.shape, 0 if x.dtype == torch.float32 else 1,
+                                                256, 1024, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    return y
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols,offset", [(4096, 200, 1), (20000, 500, 1), (2000, 3001, 0), (512, 10000, 1), (600, 40000, 0),
+                                              (600, 40000, 1), (300, 60000, 0), (256, 128256, 1)])
+def test_gpu_bf16_rounding(pkg, dev, rows, cols, offset):
+    # the elements rounded otherwise than the fp64 softmax's, as test_emulated_bf16_rounding; longer rows hold more small
+    # elements, whose x - max is itself rounded (6.6e-5 of 600 x 40000 by expf and a division)
+    print(f"[softmax bits] {rows}x{cols} offset {offset}", flush=True)
+    x, e = _fp64(rows, cols, torch.bfloat16, offset, cols, dev)
+    y = _softmax_at(pkg, x, offset)
+    bits, unit = e.view(torch.int64), 1 << 45  # the lowest bit of bf16's seven in fp64's fraction
+    once = ((bits + unit // 2 - 1 + ((bits >> 45) & 1)) & ~(unit - 1)).view(torch.float64)
+    share = ((y.double() != once) & (e > 1e-37)).double().mean().item()
+    assert share <= 9.5e-5, share
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols,offset", [(16, 50000, 0), (16, 128256, 0), (64, 128256, 0), (4, 262144, 0), (16, 262144, 1)])
+def test_gpu_fp32_error_of_few_long_rows(pkg, dev, rows, cols, offset):
+    # chunks of a half and a quarter of the longest: no further from the fp64 softmax than the longest ones (mean relative
+    # error 1.34e-7 to 1.55e-7 over these shapes; 1.0e-7 to 1.1e-7 with one exponential of x - max)
+    x, e = _fp64(rows, cols, torch.float32, offset, cols, dev)
+    error = ((_softmax_at(pkg, x, offset).double() - e).abs() / e).mean().item()
+    assert error <= 1.3e-7, error
 
 
 @pytest.mark.gpu
