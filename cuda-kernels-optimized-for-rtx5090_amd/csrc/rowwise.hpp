@@ -246,6 +246,27 @@ __device__ __forceinline__ F group_reduce(F v, Op op, F* slots, int wave, int fi
   }
 }
 
+// The sum over the group's waves, as group_reduce, but combined in pairs: the 16 sums of a long row added one after
+// another are off by up to 15 roundings of nearly the whole sum, in pairs by four.
+template <int WAVES>
+__device__ __forceinline__ float group_sum_pairs(float v, float* slots, int wave, int first) {
+  v = wave_sum(v);
+  if constexpr (WAVES == 1) {
+    return v;
+  } else {
+    if ((threadIdx.x & (kWave - 1)) == 0) slots[wave] = v;
+    __syncthreads();
+    float p[WAVES];
+#pragma unroll
+    for (int i = 0; i < WAVES; ++i) p[i] = slots[first + i];
+#pragma unroll
+    for (int d = 1; d < WAVES; d *= 2)
+#pragma unroll
+      for (int i = 0; i < WAVES; i += 2 * d) p[i] += p[i + d];
+    return p[0];
+  }
+}
+
 __device__ __forceinline__ int least(int a, int b) { return a < b ? a : b; }
 __device__ __forceinline__ int wave_id() { return (int)(threadIdx.x >> 6); }
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & (kWave - 1)); }

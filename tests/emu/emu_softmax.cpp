@@ -111,6 +111,7 @@ int main(int argc, char** argv) {
   long long bad = 0, first = -1;
   long long other = 0;  // elements whose bits are not the oracle's
   double error = 0.0;   // fp32: the sum of the relative errors of elements in the normal range
+  double sums = 0.0;    // fp32: the sum over the rows of (sum of the row's outputs - 1)^2, the error of the row's own sum
   emu::Graph recorded;
   if (graph) {
     // an eager launch first (a warm-up, as a graph capture usually follows one), then the capture
@@ -139,6 +140,7 @@ int main(int argc, char** argv) {
     } else {
       err = launch(x, y, rows, cols, dtype, 256, 0, nullptr);
     }
+    double sum = 0.0;
     for (size_t i = 0; i < n && !err; ++i) {
       bool ok;
       if (dtype == 0) {
@@ -147,6 +149,11 @@ int main(int argc, char** argv) {
         std::memcpy(&b, &ref[i * 4], 4);
         // below the normal range one ulp (2^-149) is more than 1e-5 of the value: one ulp is allowed there
         const double tol = std::fmax(1e-5 * std::fabs((double)b), 0x1p-149);
+        sum += a;
+        if (i % cols == (size_t)cols - 1) {
+          sums += (sum - 1.0) * (sum - 1.0);
+          sum = 0.0;
+        }
         if (std::fabs(b) >= 0x1p-126f) error += std::fabs((double)a - b) / std::fabs((double)b);
         ok = std::isnan(b) ? std::isnan(a) : std::fabs((double)a - b) <= tol;
       } else {
@@ -162,7 +169,8 @@ int main(int argc, char** argv) {
   }
   const bool input_kept = std::memcmp(x, host.data(), n * esz) == 0;
   const bool ok = !err && !bad && input_kept;
-  std::printf("other bits %lld of %lld, mean error %.4e\n", other, (long long)n * reps, error / (n * reps));
+  std::printf("other bits %lld of %lld, mean error %.4e, row sums off by %.4e\n", other, (long long)n * reps,
+              error / (n * reps), std::sqrt(sums / (rows * reps)));
   std::printf("rows %lld cols %lld dtype %d tier %d: %s (err %d, %lld outside tolerance, first %lld, input kept %d)\n",
               rows, cols, dtype, tier, ok ? "ALL OK" : "FAILED", err, bad, first, input_kept);
   hipFree(xb);

@@ -93,6 +93,14 @@ def test_emulated_bf16_rounding(emu_softmax, rows, cols, offset):
     assert int(out.split("other bits ")[1].split()[0]) <= 6e-5 * rows * cols, out
 
 
+@pytest.mark.parametrize("rows,cols,offset", [(200, 5003, 0), (200, 8193, 0), (200, 10000, 1), (100, 16383, 0)])
+def test_emulated_fp32_row_sums(emu_softmax, rows, cols, offset):
+    # a row's outputs add up to 1 but for the error of its own sum (a common factor of the row): six additions at nearly
+    # the whole sum, each off by 2.5e-8 on the mean square, are 6e-8; the scalar kernel's sums 6.8e-8 to 9.1e-8 here
+    out = run(emu_softmax, [rows, cols, 0, 0, 1, 0, 0, offset])
+    assert float(out.split("row sums off by ")[1].split()[0]) <= 6.6e-8, out
+
+
 @pytest.mark.parametrize("rows,cols,dtype,waves", [(5, 4096, 0, 16), (5, 20000, 0, 4), (5, 8192, 1, 16), (5, 2048, 1, 4)])
 def test_emulated_stream_nan(emu_softmax, rows, cols, dtype, waves):
     # with a vector or two per lane, some lanes hold masked elements only
