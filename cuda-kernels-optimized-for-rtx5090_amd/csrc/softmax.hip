@@ -943,8 +943,6 @@ bool capturing(hipStream_t stream) {
   return status != hipStreamCaptureStatusNone;
 }
 
-// Co-resident tier with one row per workgroup: chunks of 4 waves x 64 lanes x NV vectors, when every row's chunks fit
-// on the GPU at once. Returns 1, launching nothing, when they do not (or a row has more than kCoopMaxChunks of them).
 struct CoopLaunch {
   const void* x;
   void* y;
@@ -952,8 +950,30 @@ struct CoopLaunch {
   hipStream_t stream;
 };
 constexpr int kCoopWaves = 4;
-template <typename T> constexpr int kCoopFill = 4;
-template <> constexpr int kCoopFill<BF16> = 2;
+
+// The vectors per lane of a launch of one row per workgroup: the longest chunks (64 elements per lane), half or a
+// quarter of them.
+//  - bf16: shorter as long as no CU gets more workgroups. us by workgroups: 24 x 70000 120 5.6, 216 5.3, 432 5.9; 48 x
+//    70000 240 6.1, 432 6.3, 864 7.5; 24 x 128256 192 5.6, 384 6.2, 768 6.9; 1 x 262144 16 5.5, 32 5.0, 64 4.6; 96 x
+//    33000 288 7.8, 480 7.0, 864 7.5.
+//  - fp32, whose long chunks fill the registers: half as long up to four workgroups of the long ones per CU (200 x 50000
+//    800 17.0, 1400 13.6; 24 x 262144 384 11.6, 768 10.8; 96 x 128256 768 17.5, 1536 16.7), and a quarter while those are
+//    under four per CU and, beyond one per CU, at most 32 per row (200 x 20000 600 9.4, 1000 7.8; 1 x 262144 32 5.7, 64
+//    4.9; but 24 x 262144 1536 13.5, 16 x 262144 512 9.0, 1024 10.3).
+template <typename T>
+int coop_nv(long long rows, long long nvec) {
+  constexpr int NV = 64 / T::V;
+  const long long cus = rw_host::device_cus();
+  auto chunks = [&](int n) { return (nvec + kCoopWaves * kWave * n - 1) / (kCoopWaves * kWave * n); };
+  auto grid = [&](int n) { return rows * chunks(n); };
+  int nv = NV;
+  if constexpr (T::bytes == 4) {
+    if (grid(NV) >= 4 * cus) return NV;
+    return grid(NV / 4) < 4 * cus && (grid(NV / 4) <= cus || chunks(NV / 4) <= 32) ? NV / 4 : NV / 2;
+  }
+  while (nv > NV / 4 && (grid(nv / 2) + cus - 1) / cus == (grid(nv) + cus - 1) / cus) nv /= 2;
+  return nv;
+}
 
 // The launch of a co-resident kernel over `groups` row groups of `chunks` workgroups.
 template <typename Kernel>
@@ -982,6 +1002,8 @@ int launch_coop_k(Kernel kern, const CoopLaunch& a, long long chunks, long long 
   return (int)hipGetLastError();
 }
 
+// One row per workgroup: chunks of 4 waves x 64 lanes x NV vectors, when every row's chunks fit on the GPU at once.
+// Returns 1, launching nothing, when they do not (or a row has more than kCoopMaxChunks of them).
 template <typename T, int NV, bool NTL, bool ANY, bool FINE>
 int launch_coop_one(const CoopLaunch& a) {
   auto one = softmax_coop<T, kCoopWaves, NV, NTL, true, false, ANY, FINE>;
@@ -996,8 +1018,8 @@ int launch_coop_one(const CoopLaunch& a) {
 }
 
 // Co-resident tier: chunks of 4 waves x 64 lanes x 64 elements (16 fp32 or 8 bf16 vectors per lane), at most
-// kCoopMaxChunks per row; shorter chunks (half or a quarter as long) when the rows are so few that the long ones would
-// leave CUs without a workgroup; row groups walking several rows (an instantiation of its own: the loop costs
+// kCoopMaxChunks per row; shorter chunks (half or a quarter as long) when the rows are so few that those still leave
+// the GPU lightly filled (coop_nv); row groups walking several rows (an instantiation of its own: the loop costs
 // registers) when the rows' chunks do not fit on the GPU at once. Returns 1, launching nothing, when one row's chunks
 // do not fit.
 template <typename T, bool NTL, bool ANY, bool FINE>
@@ -1008,11 +1030,7 @@ int launch_coop(const CoopLaunch& a, int most_iters = INT_MAX) {
   const long long cus = rw_host::device_cus();
   if (want <= 0 || want >= a.rows) {
     int nv = rw_host::tune_get(kTuneCoopNv);
-    if (nv != NV && nv != NV / 2 && nv != NV / 4) {
-      nv = NV;
-      auto grid = [&](int n) { return a.rows * ((a.nvec + kCoopWaves * kWave * n - 1) / (kCoopWaves * kWave * n)); };
-      while (nv > NV / 4 && grid(nv) < kCoopFill<T> * cus) nv /= 2;
-    }
+    if (nv != NV && nv != NV / 2 && nv != NV / 4) nv = coop_nv<T>(a.rows, a.nvec);
     int rc = 1;  // a shape whose chunks are too many for the GPU or for a row takes the next longer chunks
     if (nv == NV / 4) rc = launch_coop_one<T, NV / 4, NTL, ANY, FINE>(a);
     if (rc == 1 && nv <= NV / 2) rc = launch_coop_one<T, NV / 2, NTL, ANY, FINE>(a);

@@ -169,6 +169,7 @@ int main(int argc, char** argv) {
   }
   const bool input_kept = std::memcmp(x, host.data(), n * esz) == 0;
   const bool ok = !err && !bad && input_kept;
+  std::printf("workgroups %llu, ", emu::last_grid());
   std::printf("other bits %lld of %lld, mean error %.4e, row sums off by %.4e\n", other, (long long)n * reps,
               error / (n * reps), std::sqrt(sums / (rows * reps)));
   std::printf("rows %lld cols %lld dtype %d tier %d: %s (err %d, %lld outside tolerance, first %lld, input kept %d)\n",

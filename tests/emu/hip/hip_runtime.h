@@ -469,8 +469,15 @@ inline unsigned long long realtime_ticks() {
              std::chrono::steady_clock::now().time_since_epoch()).count() / 10;
 }
 
+// The number of workgroups of the last launch.
+inline unsigned long long& last_grid() {
+  static unsigned long long n = 0;
+  return n;
+}
+
 inline void launch(dim3 grid, dim3 block, std::function<void()> body) {
   State& s = S();
+  last_grid() = (unsigned long long)grid.x * grid.y * grid.z;
   if (block.y != 1 || block.z != 1 || block.x > (unsigned)kMaxThreads) fail("block shape", 0);
   s.grid = grid;
   s.block = block;

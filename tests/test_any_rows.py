@@ -93,6 +93,18 @@ def test_emulated_bf16_rounding(emu_softmax, rows, cols, offset):
     assert int(out.split("other bits ")[1].split()[0]) <= 6e-5 * rows * cols, out
 
 
+# one row per workgroup: the workgroups of the chunk length chosen (256 CUs), where half of it would put more on a CU
+# (bf16) and where it would not; fp32 a quarter
+GRIDS = [(48, 33000, 1, 48 * 5), (24, 33000, 1, 24 * 9), (8, 70000, 1, 8 * 18), (20, 70000, 1, 20 * 9), (96, 33000, 1, 96 * 5),
+         (50, 20000, 0, 50 * 5), (110, 20000, 0, 110 * 5)]
+
+
+@pytest.mark.parametrize("rows,cols,dtype,workgroups", GRIDS)
+def test_emulated_chunk_lengths(emu_softmax, rows, cols, dtype, workgroups):
+    out = run(emu_softmax, [rows, cols, dtype, 0, 1, 0, 0, 0, "randn", 1, 1])
+    assert int(out.split("workgroups ")[1].split(",")[0]) == workgroups, out
+
+
 @pytest.mark.parametrize("rows,cols,offset", [(200, 5003, 0), (200, 8193, 0), (200, 10000, 1), (100, 16383, 0)])
 def test_emulated_fp32_row_sums(emu_softmax, rows, cols, offset):
     # a row's outputs add up to 1 but for the error of its own sum (a common factor of the row): six additions at nearly
