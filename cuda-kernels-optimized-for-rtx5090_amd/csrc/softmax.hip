@@ -487,8 +487,8 @@ __global__ void __launch_bounds__(256) softmax_coop_cell(int cell, unsigned iter
 // kernel is compiled without the loop (which costs registers: fewer resident workgroups).
 // ANY: rows of any length (nvec vectors, the last one partial) and element alignment. The row's last vector is moved
 // back to end with the row (AnyRow), its first `skip` elements being another lane's.
-// FINE: the exponential within an fp32 ulp, for fp32 rows and for the bf16 rows that an eager launch takes from the
-// scalar kernel or the row tier; bf16 rows longer than the row tier holds take exp_narrow. (Share of a bf16 row's
+// FINE: the exponential within an fp32 ulp, for fp32 rows, for bf16 rows that the scalar kernel would take and for those
+// that an eager launch takes from the row tier and holds as e; other bf16 rows take exp_narrow. (Share of a bf16 row's
 // distinct values that are rounded otherwise than the fp64 softmax's: 512 x 40000 aligned 1.27e-4 in the row tier, here
 // 1.40e-4 with exp_narrow and 0.59e-4 FINE; unaligned 0.59e-4 in the scalar kernel and here.)
 // HOLD: the chunk is held as e = exp(x - m) and written as e * (exp(m - M) / S); otherwise it is held as x, and the
@@ -1006,7 +1006,8 @@ int launch_coop_k(Kernel kern, const CoopLaunch& a, long long chunks, long long 
 // Returns 1, launching nothing, when they do not (or a row has more than kCoopMaxChunks of them).
 template <typename T, int NV, bool NTL, bool ANY, bool FINE>
 int launch_coop_one(const CoopLaunch& a) {
-  auto one = softmax_coop<T, kCoopWaves, NV, NTL, true, false, ANY, FINE>;
+  // (aligned bf16 chunks held as x round as the row tier does: not FINE)
+  auto one = softmax_coop<T, kCoopWaves, NV, NTL, true, false, ANY, FINE && (ANY || T::bytes == 4 || NV == 64 / T::V)>;
   static int occ = 0;  // resident blocks per CU (idempotent cache)
   if (occ <= 0) occ = blocks_per_cu(one, kCoopWaves * kWave);
   constexpr long long CH = (long long)kCoopWaves * kWave * NV;
@@ -1072,7 +1073,7 @@ bool row_shape_tuned() {
 // 400 rows 21.9 -> 19.3, 600 rows 30.5 -> 27.4, but 1024 rows 50.1 -> 52.3; fp32 when every row's chunks are resident
 // at once: 256 x 32768 15.0 -> 12.2, 512 x 20000 19.0 -> 15.8, but 2048 x 32768 97 -> 103 in row groups), and rows of
 // more than 2048 vectors when they are too few to
-// fill the GPU with one workgroup each (1 x 10000 fp32 4.5 -> 3.7, 16 x 32768 bf16 4.8 -> 4.2; 128 x 16384 fp32 6.0
+// fill the GPU with one workgroup each (1 x 10000 fp32 4.5 -> 3.7, 16 x 32768 bf16 4.8 -> 4.0; 128 x 16384 fp32 6.0
 // either way). A launch that is being captured stays in the row tier, which needs no second node and no tag cell, and
 // so does one in place (its callers look), where a timed-out wait's second read of the row would meet outputs.
 template <typename T>
