@@ -443,9 +443,11 @@ __global__ void __launch_bounds__(WAVES * 64)
 // tags differ), never pass.
 //
 // The wait is bounded by time: after wait_ticks of the 100 MHz s_memrealtime clock with pairs still missing (other
-// kernels holding CUs, so that the row's workgroups are not all resident) the workgroup takes the row's M and S from x
-// itself (every thread an online max and sum over a share of the whole row), so the result stays within the tolerance
-// either way; only the time suffers, by about one read of the row per waiting workgroup.
+// kernels holding CUs, so that the row's workgroups are not all resident) the workgroup takes the missing pairs from x
+// itself, by the operations of their own workgroups in their order, so the outputs are the same bits either way; only
+// the time suffers, by about two reads of each missing chunk per waiting workgroup. In place (aligned rows longer than
+// the row tier holds) a chunk is written only after its pair was published and read back, so that a workgroup that took
+// it from x while it was written finds the pair there afterwards, unless another launch has taken the slot since.
 constexpr int kCoopMaxChunks = 64;   // a row's chunks: one slot each, polled by one lane each of one wave
 constexpr int kCoopSlots = 4096;     // pair slots per parity: the most workgroups one launch may have
 constexpr int kCoopCells = 4096;     // captured launches per device with a tag cell of their own
@@ -491,26 +493,37 @@ __global__ void __launch_bounds__(256) softmax_coop_cell(int cell, unsigned iter
 // that an eager launch takes from the row tier and holds as e; other bf16 rows take exp_narrow. (Share of a bf16 row's
 // distinct values that are rounded otherwise than the fp64 softmax's: 512 x 40000 aligned 1.27e-4 in the row tier, here
 // 1.40e-4 with exp_narrow and 0.59e-4 FINE; unaligned 0.59e-4 in the scalar kernel and here.)
+// The waves per SIMD asked of the compiler are those it reaches by itself without the code behind a wait that ended,
+// which would otherwise cost the loop's bf16 forms one of four (256 x 262144 52.0 us, 54.5 with three).
 // HOLD: the chunk is held as e = exp(x - m) and written as e * (exp(m - M) / S); otherwise it is held as x, and the
 // exponential is taken again from M. Holding e saves an exponential per element, which long chunks of many rows feel
 // (1024 x 50000 fp32 77 us against 84, bf16 44 against 50), and costs fp32 rows accuracy where the chunk is short
 // (mean relative error of 16 x 128256 fp32: 1.47e-7 in four times longer chunks, 1.57e-7 as e, 1.03e-7 from x). So
 // short chunks and unaligned fp32 rows are held as x.
 template <typename T, int WAVES, int NV, bool NTL, bool NTS, bool LOOP, bool ANY, bool FINE>
-__global__ void __launch_bounds__(WAVES * 64)
+__global__ void __launch_bounds__(WAVES * 64, NV * T::V == 64 ? 4 : ANY ? 7 : 8)
     softmax_coop(const void* __restrict__ x, void* __restrict__ y, long long rows, long long nvec, long long cols,
                  int chunks, int groups, int slot0, unsigned tag0, int cell, unsigned wait_ticks) {
   constexpr int G = WAVES * kWave;
   // a captured launch (cell >= 0) reads its first tag from its cell, filled by the kernel node just before it
   if (cell >= 0) tag0 = __hip_atomic_load(&g_coop_cells[cell], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   constexpr long long CH = (long long)G * NV;
-  constexpr int PER = kCoopMaxChunks / kWave;
+  static_assert(kCoopMaxChunks == kWave, "a lane of wave 0 for each chunk's pair");
   __shared__ float slots[2][WAVES];
   __shared__ float ms[2];
-  __shared__ int partial;  // the wait ended before every pair of the row was published
+  __shared__ unsigned long long missing;       // the chunks whose pairs had not come when the wait ended
+  __shared__ float pairs[kCoopMaxChunks][2];  // the row's pairs then
   const int c = (int)(blockIdx.x % (unsigned)chunks), group = (int)(blockIdx.x / (unsigned)chunks);
-  const int first = c * (int)CH;  // < 2^31: at most kCoopMaxChunks chunks of CH vectors
-  const int count = nvec - first < CH ? (int)(nvec - first) : (int)CH;
+  // a chunk's place in the row: its first vector (< 2^31: at most kCoopMaxChunks chunks of CH vectors), its vectors, and
+  // (ANY) the elements from its first to the row's end, at least one
+  struct Part {
+    int first, count, reach;
+  };
+  auto part = [&](int q) __attribute__((always_inline)) {
+    const int first = q * (int)CH;
+    return Part{first, nvec - first < CH ? (int)(nvec - first) : (int)CH, (int)(cols - (long long)first * T::V)};
+  };
+  const Part own = part(c);
   const int t0 = (int)threadIdx.x;
   const int wave0 = __builtin_amdgcn_readfirstlane(t0 & ~(kWave - 1));
   const int iters = (int)((rows - group + groups - 1) / groups);
@@ -520,23 +533,47 @@ __global__ void __launch_bounds__(WAVES * 64)
   Regs<NV> next;  // PREFETCH: the next row's raw chunk, loaded during the wait
   // ANY: elements of the row from V before the chunk's first on; a vector past the row's last whole start is moved back
   // to it
-  const int reach = (int)(cols - (long long)first * T::V);  // the chunk's first element to the row's end: >= 1
-  auto offset = [&](int k, int t) __attribute__((always_inline)) {
-    return (uint32_t)((least((k * G + t) * T::V, reach - T::V) + T::V) * T::bytes);
+  auto offset = [&](const Part& p, int k, int t) __attribute__((always_inline)) {
+    return (uint32_t)((least((k * G + t) * T::V, p.reach - T::V) + T::V) * T::bytes);
   };
-  auto chunk_base = [&](long long row) __attribute__((always_inline)) {
-    return (row * cols + ((long long)first - 1) * T::V) * T::bytes;
+  auto chunk_base = [&](const Part& p, long long row) __attribute__((always_inline)) {
+    return (row * cols + ((long long)p.first - 1) * T::V) * T::bytes;
   };
-  auto load_chunk = [&](Regs<NV>& r, long long row, int t) __attribute__((always_inline)) {
+  auto load_chunk = [&](Regs<NV>& r, const Part& p, long long row, int t) __attribute__((always_inline)) {
     if constexpr (ANY) {
-      const char* base = static_cast<const char*>(x) + chunk_base(row);
+      const char* base = static_cast<const char*>(x) + chunk_base(p, row);
 #pragma unroll
-      for (int k = 0; k < NV; ++k) r.v[k] = load16_at<NTL>(base, offset(k, t));
+      for (int k = 0; k < NV; ++k) r.v[k] = load16_at<NTL>(base, offset(p, k, t));
     } else {
-      load_vectors<G, NV, false, NTL>(r, x, row * nvec + first, count, t);
+      load_vectors<G, NV, false, NTL>(r, x, row * nvec + p.first, p.count, t);
     }
   };
-  if constexpr (PREFETCH) load_chunk(next, group, t0);
+  // the maximum of m and vector k's elements; its elements' exponentials from `from` and their sum
+  auto max_with = [&](const Part& p, const u32x4& v, int k, int t, float m) __attribute__((always_inline)) {
+    float f[T::V];
+    unpack<T>(v, f);
+    const bool ok = k * G + t < p.count;
+#pragma unroll
+    for (int i = 0; i < T::V; ++i) m = ok ? fmaxf(m, f[i]) : m;
+    return m;
+  };
+  auto exps = [&](const Part& p, const u32x4& v, int k, int t, float from, float (&f)[T::V])
+                  __attribute__((always_inline)) {
+    unpack<T>(v, f);
+    const bool ok = k * G + t < p.count;
+#pragma unroll
+    for (int i = 0; i < T::V; ++i) {
+      f[i] = exp_of(f[i] - from);
+      if (!ANY) f[i] = ok ? f[i] : 0.0f;
+    }
+    int skip = 0;  // ANY: the first elements of the vector, another lane's
+    if (ANY && (k * G + wave0 + kWave) * T::V > p.reach) {
+      const int start = (k * G + t) * T::V;
+      skip = start - least(start, p.reach - T::V);
+    }
+    return sum_vector<T>(f, skip);
+  };
+  if constexpr (PREFETCH) load_chunk(next, own, group, t0);
   for (int it = 0; it < iters; ++it) {
     const long long row = group + (long long)it * groups;
     // the lane's offsets are formed anew each iteration (hoisted out of the loop they would hold NV 64-bit offsets in
@@ -547,130 +584,103 @@ __global__ void __launch_bounds__(WAVES * 64)
     unsigned long long(*table)[2] = g_coop_pairs[it & 1] + slot0 + group * chunks;
     Regs<NV> r;
     if constexpr (PREFETCH) r = next;
-    else load_chunk(r, row, t);
+    else load_chunk(r, own, row, t);
     float m = -INFINITY;
 #pragma unroll
-    for (int k = 0; k < NV; ++k) {
-      float f[T::V];
-      unpack<T>(r.v[k], f);
-      const bool ok = k * G + t < count;
-#pragma unroll
-      for (int i = 0; i < T::V; ++i) m = ok ? fmaxf(m, f[i]) : m;
-    }
+    for (int k = 0; k < NV; ++k) m = max_with(own, r.v[k], k, t, m);
     m = group_reduce<WAVES>(m, OpMax{}, slots[0], wave_id(), 0);
     // a chunk of only -inf and NaN has m = -inf (fmaxf takes the other operand of a NaN): its elements are taken from 0
     // instead, -inf to 0 and NaN to NaN, so that a NaN reaches s, the row's S, and through it every output of the row
-    const float from = m == -INFINITY ? 0.0f : m;
-    float e[HOLD ? NV : 1][T::V];
+    float e[NV][T::V];
     float s = 0.0f;
 #pragma unroll
-    for (int k = 0; k < NV; ++k) {
-      float f[T::V];
-      unpack<T>(r.v[k], f);
-      const bool ok = k * G + t < count;
-#pragma unroll
-      for (int i = 0; i < T::V; ++i) {
-        f[i] = exp_of(f[i] - from);
-        if (!ANY) f[i] = ok ? f[i] : 0.0f;
-        if (HOLD) e[k][i] = f[i];
-      }
-      int skip = 0;  // ANY: the first elements of the vector, another lane's
-      if (ANY && (k * G + wave0 + kWave) * T::V > reach) {
-        const int start = (k * G + t) * T::V;
-        skip = start - least(start, reach - T::V);
-      }
-      s += sum_vector<T>(f, skip);
-    }
+    for (int k = 0; k < NV; ++k) s += exps(own, r.v[k], k, t, m == -INFINITY ? 0.0f : m, e[k]);
     s = group_reduce<WAVES>(s, OpSum{}, slots[1], wave_id(), 0);
     // the next row's loads go out before the wait and the stores (bf16; for fp32 the two chunks together would halve the
     // resident workgroups)
     if constexpr (PREFETCH)
-      if (it + 1 < iters) load_chunk(next, row + groups, t);
+      if (it + 1 < iters) load_chunk(next, own, row + groups, t);
     if (t == 0) {  // an all -inf chunk publishes (-inf, 0), which adds nothing to the merge; with a NaN in it, (-inf, NaN)
       __hip_atomic_store(&table[c][0], tag | __float_as_uint(m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __hip_atomic_store(&table[c][1], tag | __float_as_uint(s), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+    // a chunk's pair by the lane of its number in wave 0, for those of the launch's iteration; whether it has come
+    auto look = [&](unsigned long long& wm, unsigned long long& ws) __attribute__((always_inline)) {
+      if ((wm >> 32) != (tag >> 32))
+        wm = __hip_atomic_load(&table[lane_id()][0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if ((ws >> 32) != (tag >> 32))
+        ws = __hip_atomic_load(&table[lane_id()][1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return (wm >> 32) == (tag >> 32) && (ws >> 32) == (tag >> 32);
+    };
+    auto merge = [&](float pm, float ps) __attribute__((always_inline)) {
+      const float M = wave_max(pm);
+      const float S = wave_sum(ps * expf(pm - (M == -INFINITY ? 0.0f : M)));  // (-inf, s): 0, or NaN where s is
+      if (lane_id() == 0) {
+        ms[0] = M;
+        ms[1] = S;
+      }
+    };
     if (wave_id() == 0) {
-      const int lane = lane_id();
-      unsigned long long wm[PER], ws[PER];
-#pragma unroll
-      for (int i = 0; i < PER; ++i) wm[i] = ws[i] = 0;
+      const bool mine = lane_id() < chunks;
+      unsigned long long wm = 0, ws = 0;
       const unsigned long long start = __builtin_amdgcn_s_memrealtime();
-      bool complete = false;
-      while (true) {
-        bool have = true;
-#pragma unroll
-        for (int i = 0; i < PER; ++i) {
-          const int at = i * kWave + lane;
-          if (at < chunks) {
-            if ((wm[i] >> 32) != (tag >> 32))
-              wm[i] = __hip_atomic_load(&table[at][0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if ((ws[i] >> 32) != (tag >> 32))
-              ws[i] = __hip_atomic_load(&table[at][1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            have = have && (wm[i] >> 32) == (tag >> 32) && (ws[i] >> 32) == (tag >> 32);
-          }
-        }
-        if (__ballot(!have) == 0) {
-          complete = true;
-          break;
-        }
+      unsigned long long left;
+      while ((left = __ballot(mine && !look(wm, ws))) != 0) {
         // (the clock is a scalar read, so the decision is the wave's; readfirstlane states it)
         if (__builtin_amdgcn_readfirstlane((int)(__builtin_amdgcn_s_memrealtime() - start > wait_ticks))) break;
         __builtin_amdgcn_s_sleep(1);
       }
-      float pm = -INFINITY, ps = 0.0f;
-#pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        if (i * kWave + lane < chunks) {
-          const float qm = __uint_as_float((unsigned)wm[i]), qs = __uint_as_float((unsigned)ws[i]);
-          const float mm = fmaxf(pm, qm), base = mm == -INFINITY ? 0.0f : mm;
-          ps = ps * expf(pm - base) + qs * expf(qm - base);
-          pm = mm;
-        }
+      const float pm = mine ? __uint_as_float((unsigned)wm) : -INFINITY, ps = mine ? __uint_as_float((unsigned)ws) : 0.0f;
+      if (left == 0) {
+        merge(pm, ps);
+      } else {
+        pairs[lane_id()][0] = pm;
+        pairs[lane_id()][1] = ps;
       }
-      const float M = wave_max(pm);
-      const float S = wave_sum(ps * expf(pm - (M == -INFINITY ? 0.0f : M)));  // (-inf, s): 0, or NaN where s is
-      if (lane == 0) {
-        ms[0] = M;
-        ms[1] = S;
-        partial = complete ? 0 : 1;
-      }
+      if (lane_id() == 0) missing = left;
     }
     __syncthreads();
-    if (partial) {
-      // the row's M and S from x: an online max and sum per thread over its share of the row, merged over the block
-      // (-inf elements add nothing; a NaN makes the sum NaN, as in the pairs)
-      float tm = -INFINITY, ts = 0.0f;
-      for (long long i = t; i < nvec; i += G) {
-        float f[T::V];
-        int skip = 0;
-        if constexpr (ANY) {
-          const int at = least((int)i * T::V, (int)cols - T::V);
-          const char* base = static_cast<const char*>(x) + row * cols * T::bytes;
-          unpack<T>(load16_at<false>(base, (uint32_t)(at * T::bytes)), f);
-          skip = (int)i * T::V - at;
-        } else {
-          unpack<T>(load16<false>(x, row * nvec + i), f);
+    if (__builtin_expect(missing != 0, 0)) {
+      // the missing pairs from x, by the operations and in the order of the chunks' own workgroups (the offsets formed
+      // anew, vector by vector: kept from above, or several loads in flight, they would cost the kernel its registers)
+      int u = t;
+      asm volatile("" : "+v"(u));
+      const unsigned long long out = missing;
+      for (unsigned long long left = out; left; left &= left - 1) {
+        const int q = __builtin_ctzll(left);
+        const Part p = part(q);
+        auto load = [&](int k) __attribute__((always_inline)) {
+          if constexpr (ANY) return load16_at<false>(static_cast<const char*>(x) + chunk_base(p, row), offset(p, k, u));
+          else return load16<false>(x, row * nvec + p.first + least(k * G + u, p.count - 1));
+        };
+        float qm = -INFINITY, qs = 0.0f;
+#pragma unroll 1
+        for (int k = 0; k < NV; ++k) qm = max_with(p, load(k), k, u, qm);
+        qm = group_reduce<WAVES>(qm, OpMax{}, slots[0], wave_id(), 0);
+#pragma unroll 1
+        for (int k = 0; k < NV; ++k) {
+          float f[T::V];
+          qs += exps(p, load(k), k, u, qm == -INFINITY ? 0.0f : qm, f);
         }
-#pragma unroll
-        for (int e = 0; e < T::V; ++e) {
-          if (e < skip || f[e] == -INFINITY) continue;
-          if (f[e] > tm) {
-            ts = ts * expf(tm - f[e]) + 1.0f;
-            tm = f[e];
-          } else {
-            ts += expf(f[e] - tm);
-          }
+        qs = group_reduce<WAVES>(qs, OpSum{}, slots[1], wave_id(), 0);
+        if (threadIdx.x == 0) {
+          pairs[q][0] = qm;
+          pairs[q][1] = qs;
         }
       }
-      const float RM = group_reduce<WAVES>(tm, OpMax{}, slots[0], wave_id(), 0);
-      const float RS = group_reduce<WAVES>(ts * expf(tm - (RM == -INFINITY ? 0.0f : RM)), OpSum{}, slots[1], wave_id(), 0);
-      __syncthreads();  // every wave has read ms and the slots before they are written
-      if (t == 0) {
-        ms[0] = RM;
-        ms[1] = RS;
+      if (wave_id() == 0) {
+        wave_lds_sync();  // lane 0's pairs before the other lanes' reads
+        float pm = pairs[lane_id()][0], ps = pairs[lane_id()][1];
+        unsigned long long wm = 0, ws = 0;
+        // (a pair that has come meanwhile is taken: in place, its workgroup may have written its chunk since)
+        if ((out >> lane_id() & 1) && look(wm, ws)) {
+          pm = __uint_as_float((unsigned)wm);
+          ps = __uint_as_float((unsigned)ws);
+        }
+        merge(pm, ps);
       }
       __syncthreads();
+      if constexpr (!HOLD) load_chunk(r, own, row, u);  // (not kept in registers meanwhile)
     }
     const float M = ms[0], S = ms[1];
     // HOLD: an all -inf chunk (e = 0) gives 0, or NaN when the whole row is -inf (S = 0) or S is NaN
@@ -678,7 +688,7 @@ __global__ void __launch_bounds__(WAVES * 64)
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
       const int i = k * G + t;
-      if (i < count) {
+      if (i < own.count) {
         float f[T::V];
         if constexpr (!HOLD) unpack<T>(r.v[k], f);
 #pragma unroll
@@ -687,12 +697,12 @@ __global__ void __launch_bounds__(WAVES * 64)
           else if constexpr (FINE) f[j] = quotient(exp_of(f[j] - M), S, scale);
           else f[j] = exp_of(f[j] - M) * scale;
         }
-        if constexpr (ANY) store16_at<NTS>(static_cast<char*>(y) + chunk_base(row), offset(k, t), pack<T>(f));
-        else store16<NTS>(y, row * nvec + first + i, pack<T>(f));
+        if constexpr (ANY) store16_at<NTS>(static_cast<char*>(y) + chunk_base(own, row), offset(own, k, t), pack<T>(f));
+        else store16<NTS>(y, row * nvec + own.first + i, pack<T>(f));
       }
     }
     if constexpr (!LOOP) break;
-    __syncthreads();  // ms, partial and the reduction slots are written again by the next row
+    __syncthreads();  // ms, missing and the reduction slots are written again by the next row
   }
 }
 

@@ -169,7 +169,9 @@ int main(int argc, char** argv) {
   }
   const bool input_kept = std::memcmp(x, host.data(), n * esz) == 0;
   const bool ok = !err && !bad && input_kept;
-  std::printf("workgroups %llu, ", emu::last_grid());
+  unsigned long long hash = 1469598103934665603ull;  // FNV-1a of the outputs
+  for (size_t i = 0; i < n * esz; ++i) hash = (hash ^ (unsigned char)y[i]) * 1099511628211ull;
+  std::printf("workgroups %llu, outputs %016llx, ", emu::last_grid(), hash);
   std::printf("other bits %lld of %lld, mean error %.4e, row sums off by %.4e\n", other, (long long)n * reps,
               error / (n * reps), std::sqrt(sums / (rows * reps)));
   std::printf("rows %lld cols %lld dtype %d tier %d: %s (err %d, %lld outside tolerance, first %lld, input kept %d)\n",

@@ -93,6 +93,20 @@ def test_emulated_bf16_rounding(emu_softmax, rows, cols, offset):
     assert int(out.split("other bits ")[1].split()[0]) <= 6e-5 * rows * cols, out
 
 
+SAME = [(5, 50000, 0, 0), (5, 50001, 0, 0), (6, 70000, 0, 2), (6, 70001, 0, 2), (60, 20000, 0, 0), (6, 50000, 1, 2),
+        (6, 50001, 1, 2), (4, 70000, 1, 0), (4, 70001, 1, 0)]
+
+
+@pytest.mark.parametrize("rows,cols,dtype,groups", SAME)
+@pytest.mark.parametrize("pattern", ["randn", "special"])
+def test_emulated_coresident_same_bits(emu_softmax, rows, cols, dtype, groups, pattern):
+    # by the pairs, and with the wait timed out (one workgroup after another: all but a row's last take pairs from x)
+    args = [rows, cols, dtype, 4, 3, 0, groups, 0, pattern, 1]
+    pairs = run(emu_softmax, args, env=dict(os.environ, EMU_CLOCK_STOPPED="1"), concurrent=True)
+    alone = run(emu_softmax, [*args, 1])
+    assert pairs.split("outputs ")[1][:16] == alone.split("outputs ")[1][:16]
+
+
 # one row per workgroup: the workgroups of the chunk length chosen (256 CUs), where half of it would put more on a CU
 # (bf16) and where it would not; fp32 a quarter
 GRIDS = [(48, 33000, 1, 48 * 5), (24, 33000, 1, 24 * 9), (8, 70000, 1, 8 * 18), (20, 70000, 1, 20 * 9), (96, 33000, 1, 96 * 5),
@@ -234,6 +248,23 @@ def test_gpu_fp32_error_of_few_long_rows(pkg, dev, rows, cols, offset):
     x, e = _fp64(rows, cols, torch.float32, offset, cols, dev)
     error = ((_softmax_at(pkg, x, offset).double() - e).abs() / e).mean().item()
     assert error <= 1.3e-7, error
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("rows,cols,offset", [(16, 20000, 0), (5, 50000, 0), (5, 50000, 1), (24, 128256, 0), (1, 262143, 0),
+                                              (300, 49152, 0), (300, 50000, 1), (300, 262144, 0)])
+def test_gpu_timed_out_rows_have_the_same_bits(pkg, dev, dtype, rows, cols, offset):
+    print(f"[softmax timed out] {rows}x{cols} {dtype} offset {offset}", flush=True)
+    x, _ = _fp64(rows, cols, dtype, offset, cols, dev)
+    lib = pkg.candidate("softmax")._lib
+    by_pairs = _softmax_at(pkg, x, offset)
+    try:
+        lib.softmax_tune(7, 1)
+        for _ in range(3):
+            assert torch.equal(_softmax_at(pkg, x, offset), by_pairs)
+    finally:
+        lib.softmax_tune(7, 0)
 
 
 @pytest.mark.gpu
