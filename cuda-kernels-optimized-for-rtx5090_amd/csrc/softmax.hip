@@ -171,7 +171,8 @@ __global__ void __launch_bounds__((WAVES < 4 ? 4 : WAVES) * 64)
 
 // Row tier for rows of any length from one vector up and any element alignment: the lanes' vectors start at the row's
 // first element, wherever it lies, and a vector that would pass the row's end is moved back to end with it. Its first
-// elements are then another lane's (the same bits, and the same results when they are stored twice), so the maximum
+// elements are then another lane's of the same workgroup (the same bits, from the same maximum and sum: the same results
+// when they are stored twice), so the maximum
 // takes every loaded element and the sum leaves out the first `skip` of the vector; only the wave that holds the row's
 // end looks at that, and vectors that lie past the end for a whole wave are not worked on.
 // 8192 x 3001 bf16 62.1 us through the scalar kernel's three passes of 2-byte accesses, 18.3 us here (17.0 with
@@ -697,7 +698,18 @@ __global__ void __launch_bounds__(WAVES * 64, NV * T::V == 64 ? 4 : ANY ? 7 : 8)
           else if constexpr (FINE) f[j] = quotient(exp_of(f[j] - M), S, scale);
           else f[j] = exp_of(f[j] - M) * scale;
         }
-        if constexpr (ANY) store16_at<NTS>(static_cast<char*>(y) + chunk_base(own, row), offset(own, k, t), pack<T>(f));
+        if constexpr (ANY) {
+          if (k == 0 && own.reach < T::V) {
+            // a last chunk of less than a vector (lane 0 alone): the first elements are the chunk before's, which may
+            // round them otherwise
+            const long long end = row * cols + cols;
+#pragma unroll
+            for (int j = 0; j < T::V; ++j)
+              if (j >= T::V - own.reach) store_elem<T>(y, end - T::V + j, f[j]);
+            continue;
+          }
+          store16_at<NTS>(static_cast<char*>(y) + chunk_base(own, row), offset(own, k, t), pack<T>(f));
+        }
         else store16<NTS>(y, row * nvec + own.first + i, pack<T>(f));
       }
     }

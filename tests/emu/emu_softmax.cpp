@@ -13,6 +13,7 @@
 //   NaN, -inf with a NaN or a +inf elsewhere in the row, and only -inf); reps: launches on the same buffers, each checked (the co-resident
 //   tier's pair table is reused by the next launch, under fresh tags); wait_ticks bounds the co-resident tier's wait
 //   (1 makes its workgroups stop waiting and take the row's statistics from x).
+// EMU_ONLY set to a workgroup's number: only that one runs, and the elements it has written are listed.
 // EMU_GRAPH set: after an eager launch, the launch is recorded as a graph (the emulation's capture) and every rep
 // replays it, each with new values in x (seed + rep); odd reps first run an eager launch of the same shape on other
 // values and buffers, which leaves its own pairs in the table. Every replay is checked against the oracle of its x.
@@ -169,6 +170,14 @@ int main(int argc, char** argv) {
   }
   const bool input_kept = std::memcmp(x, host.data(), n * esz) == 0;
   const bool ok = !err && !bad && input_kept;
+  if (std::getenv("EMU_ONLY")) {  // where one workgroup has written (the rest keeps its fill, which no output equals)
+    for (size_t i = 0; i < n; ++i) {
+      unsigned fill = 0;
+      std::memcpy(&fill, y + i * esz, esz);
+      if (fill != (esz == 4 ? 0xA5A5A5A5u : 0xA5A5u)) std::printf("%zu ", i);
+    }
+    std::printf("written\n");
+  }
   unsigned long long hash = 1469598103934665603ull;  // FNV-1a of the outputs
   for (size_t i = 0; i < n * esz; ++i) hash = (hash ^ (unsigned char)y[i]) * 1099511628211ull;
   std::printf("workgroups %llu, outputs %016llx, ", emu::last_grid(), hash);

@@ -489,7 +489,9 @@ inline void launch(dim3 grid, dim3 block, std::function<void()> body) {
       for (unsigned x = 0; x < grid.x; ++x) blocks.push_back(Idx{x, y, z});
   if (s.shuffle_seed >= 0) std::shuffle(blocks.begin(), blocks.end(), s.rng);
   if (!concurrent()) {
+    const char* only = std::getenv("EMU_ONLY");  // this workgroup alone runs
     for (const Idx& b : blocks) {
+      if (only && b.x != (unsigned)std::atoi(only)) continue;
       s.block_idx = b;
       run_block();
     }

@@ -93,6 +93,20 @@ def test_emulated_bf16_rounding(emu_softmax, rows, cols, offset):
     assert int(out.split("other bits ")[1].split()[0]) <= 6e-5 * rows * cols, out
 
 
+@pytest.mark.parametrize("cols,dtype,groups", [(4 * 4096 + 1, 1, 0), (4 * 4096 + 7, 1, 0), (2 * 16384 + 3, 1, 1), (4097, 0, 0),
+                                               (16384 + 3, 0, 1)])
+def test_emulated_last_chunk_writes_its_own(emu_softmax, cols, dtype, groups):
+    # a last chunk of less than a vector, whose workgroup loads the row's last whole vector: the elements of the chunk
+    # before are its workgroup's to write, whose rounding may be another; two rows, so that one group loops
+    own = cols % 4096 if groups == 0 else cols % 16384
+    chunks = cols // (4096 if groups == 0 else 16384) + 1
+    env = dict(os.environ, EMU_ONLY=str(chunks - 1))
+    out = run(emu_softmax, [2 if groups else 1, cols, dtype, 4, 3, 0, groups, 0, "randn", 1, 1], env=env, expect_ok=False)
+    rows = 2 if groups else 1
+    written = [int(i) for i in out.split("written")[0].split()]
+    assert written == [r * cols + i for r in range(rows) for i in range(cols - own, cols)]
+
+
 SAME = [(5, 50000, 0, 0), (5, 50001, 0, 0), (6, 70000, 0, 2), (6, 70001, 0, 2), (60, 20000, 0, 0), (6, 50000, 1, 2),
         (6, 50001, 1, 2), (4, 70000, 1, 0), (4, 70001, 1, 0)]
 
@@ -169,7 +183,7 @@ def _check(pkg, oracle, dev, rows, cols, dtype, offset=0, special=False):
                                        (8191, 256), (8192, 257), (9001, 511), (20000, 512), (513, 255), (700, 513),
                                        (5, 2049), (300, 3001), (9, 8191), (600, 16383), (3, 16384), (40, 20001), (2, 32767),
                                        (300, 20000), (5, 65535), (3, 70001), (2, 262143), (70, 262143), (1, 1048576),
-                                       (2, 1048577)])
+                                       (2, 1048577), (3, 16385), (9, 36869), (300, 49153)])
 def test_gpu_rows(pkg, oracle, dev, dtype, rows, cols):
     _check(pkg, oracle, dev, rows, cols, dtype, offset=1, special=True)
 
