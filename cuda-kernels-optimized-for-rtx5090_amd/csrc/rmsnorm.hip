@@ -136,7 +136,7 @@ __device__ __forceinline__ void norm_row(const Regs<NV>& r, const Regs<NV>& w, v
 #pragma unroll
       for (int e = 0; e < T::V; ++e) {
         f[e] = f[e] * inv;
-        if constexpr (FORM == kAny) apart<T>(f[e]);
+        apart<T>(f[e]);
       }
       if constexpr (HAS_W) {
         float g[T::V];
@@ -144,7 +144,7 @@ __device__ __forceinline__ void norm_row(const Regs<NV>& r, const Regs<NV>& w, v
 #pragma unroll
         for (int e = 0; e < T::V; ++e) {
           f[e] = g[e] * round_to<T>(f[e]);
-          if constexpr (FORM == kAny) apart<T>(f[e]);
+          apart<T>(f[e]);
         }
       }
       at.template store<NTS>(y, row, k, pack<T>(f));
@@ -301,12 +301,18 @@ __global__ void __launch_bounds__(256)
         float f[T::V];
         unpack<T>(s.v[u][k], f);
 #pragma unroll
-        for (int e = 0; e < T::V; ++e) f[e] = f[e] * inv[u];
+        for (int e = 0; e < T::V; ++e) {
+          f[e] = f[e] * inv[u];
+          apart<T>(f[e]);
+        }
         if constexpr (HAS_W) {
           float g[T::V];
           unpack<T>(wr[k], g);
 #pragma unroll
-          for (int e = 0; e < T::V; ++e) f[e] = g[e] * round_to<T>(f[e]);
+          for (int e = 0; e < T::V; ++e) {
+            f[e] = g[e] * round_to<T>(f[e]);
+            apart<T>(f[e]);
+          }
         }
         store16<true>(static_cast<char*>(y) + first * nvec * 16, at(first, u, k), pack<T>(f));
       }
@@ -353,7 +359,11 @@ __global__ void __launch_bounds__(256)
     const float inv = row_inv<T>(acc, cols, eps);
     for (int j = threadIdx.x; j < cols; j += 256) {
       float v = load_elem<T>(src, o + j) * inv;
-      if constexpr (HAS_W) v = load_elem<T>(w, j) * round_to<T>(v);
+      apart<T>(v);
+      if constexpr (HAS_W) {
+        v = load_elem<T>(w, j) * round_to<T>(v);
+        apart<T>(v);
+      }
       store_elem<T>(y, o + j, v);
     }
   }

@@ -74,13 +74,35 @@ def test_gpu_any_rows(pkg, oracle, dev, dtype, rows, cols):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("cols", [7, 64, 256, 1000, 1001, 4096, 5120, 16384, 70000])
+def test_gpu_negative_zeros(pkg, oracle, dev, dtype, cols):
+    # -0 stays -0 through both products in every form of the kernel: short, part and full rows, any rows, scalar rows
+    print(f"[rmsnorm -0] 9x{cols} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(cols)
+    x = torch.randn(9, cols, generator=g).to(dtype)
+    x[:, ::3] = -0.0
+    x[4] = -0.0
+    r = torch.where(torch.rand(9, cols, generator=g) < 0.5, torch.tensor(-0.0), torch.randn(9, cols, generator=g)).to(dtype)
+    w = (torch.rand(cols, generator=g) - 0.5).to(dtype)
+    fp16 = dtype == torch.float16
+    name = "fp16" if fp16 else "bf16"
+    for weight in (w, None):
+        y = pkg.rmsnorm(x.to(dev), None if weight is None else weight.to(dev))
+        ref = oracle.rmsnorm(bits16(x), None if weight is None else bits16(weight), dtype=name)
+        assert same_bits16(bits16(y), ref, fp16)
+    ry, rh = oracle.rmsnorm_add(bits16(x), bits16(r), bits16(w), dtype=name)
+    y, h = pkg.rmsnorm_add(x.to(dev), r.to(dev), w.to(dev))
+    assert same_bits16(bits16(h), rh, fp16) and same_bits16(bits16(y), ry, fp16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("rows,cols", [(1, 8), (5, 64), (16, 80), (17, 96), (4095, 128), (16384, 128), (16401, 136),
                                        (40000, 192), (163841, 128), (70000, 256), (300, 264), (70001, 512)])
 def test_gpu_short_rows(pkg, oracle, dev, dtype, rows, cols):
     print(f"[rmsnorm short] {rows}x{cols} {dtype}", flush=True)
     g = torch.Generator().manual_seed(rows + cols)
-    # (+ 0: no -0, whose weighted fp16 product comes out as +0 on the GPU)
-    x = (torch.randn(rows, cols, generator=g) * torch.rand(rows, 1, generator=g) * 3).to(dtype) + 0
+    x = (torch.randn(rows, cols, generator=g) * torch.rand(rows, 1, generator=g) * 3).to(dtype)
     x[rows // 2, cols // 2] = float("nan")
     x[0] = 0
     w = (torch.rand(cols, generator=g) + 0.5).to(dtype)
