@@ -10,7 +10,8 @@
 //   than rows make each workgroup walk several rows), 0 automatic; offset shifts x and y by that many elements from a
 //   16-byte boundary; pattern: randn (N(0, 4)), special (-inf elements,
 //   an all -inf row, a row of one huge value) or nan (the middle half of every row masked: -inf with one NaN in it, all
-//   NaN, -inf with a NaN or a +inf elsewhere in the row, and only -inf); reps: launches on the same buffers, each checked (the co-resident
+//   NaN, -inf with a NaN or a +inf elsewhere in the row, and only -inf) or pair (0, -0.0173 times the row's number, and
+//   -inf: the exponential itself); reps: launches on the same buffers, each checked (the co-resident
 //   tier's pair table is reused by the next launch, under fresh tags); wait_ticks bounds the co-resident tier's wait
 //   (1 makes its workgroups stop waiting and take the row's statistics from x).
 // EMU_ONLY set to a workgroup's number: only that one runs, and the elements it has written are listed.
@@ -19,6 +20,7 @@
 // values and buffers, which leaves its own pairs in the table. Every replay is checked against the oracle of its x.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -66,7 +68,7 @@ int main(int argc, char** argv) {
   }
   const size_t esz = dtype == 0 ? 4 : 2, n = (size_t)rows * cols;
   const bool graph = std::getenv("EMU_GRAPH") != nullptr;
-  if (pattern != "randn" && pattern != "special" && pattern != "nan") {
+  if (pattern != "randn" && pattern != "special" && pattern != "nan" && pattern != "pair") {
     std::fprintf(stderr, "unknown pattern %s\n", pattern.c_str());
     return 2;
   }
@@ -83,6 +85,7 @@ int main(int argc, char** argv) {
         if (r % 4 == 1) v = -INFINITY;
         if (r % 4 == 2 && c == cols / 2) v = 80.0f;
       }
+      if (pattern == "pair") v = c == 0 ? 0.0f : c == 1 ? -0.0173f * (float)r : -INFINITY;
       if (pattern == "nan") {
         if (c >= cols / 4 && c < cols - cols / 4) v = r % 5 == 1 ? NAN : -INFINITY;
         if (r % 5 == 0 && c == cols / 2) v = NAN;
@@ -112,6 +115,7 @@ int main(int argc, char** argv) {
   long long bad = 0, first = -1;
   long long other = 0;  // elements whose bits are not the oracle's
   double error = 0.0;   // fp32: the sum of the relative errors of elements in the normal range
+  double ulps = 0.0;    // fp32: the largest error in units of the oracle's last place (of 2^-149 below the normal range)
   double sums = 0.0;    // fp32: the sum over the rows of (sum of the row's outputs - 1)^2, the error of the row's own sum
   emu::Graph recorded;
   if (graph) {
@@ -151,6 +155,9 @@ int main(int argc, char** argv) {
         // below the normal range one ulp (2^-149) is more than 1e-5 of the value: one ulp is allowed there
         const double tol = std::fmax(1e-5 * std::fabs((double)b), 0x1p-149);
         sum += a;
+        int exponent = 0;
+        std::frexp(b, &exponent);
+        if (std::isfinite(b)) ulps = std::fmax(ulps, std::fabs((double)a - b) / std::ldexp(1.0, std::max(exponent - 24, -149)));
         if (i % cols == (size_t)cols - 1) {
           sums += (sum - 1.0) * (sum - 1.0);
           sum = 0.0;
@@ -181,6 +188,7 @@ int main(int argc, char** argv) {
   unsigned long long hash = 1469598103934665603ull;  // FNV-1a of the outputs
   for (size_t i = 0; i < n * esz; ++i) hash = (hash ^ (unsigned char)y[i]) * 1099511628211ull;
   std::printf("workgroups %llu, outputs %016llx, ", emu::last_grid(), hash);
+  std::printf("graph nodes %zu, worst %.3f ulps, ", recorded.size(), ulps);
   std::printf("other bits %lld of %lld, mean error %.4e, row sums off by %.4e\n", other, (long long)n * reps,
               error / (n * reps), std::sqrt(sums / (rows * reps)));
   std::printf("rows %lld cols %lld dtype %d tier %d: %s (err %d, %lld outside tolerance, first %lld, input kept %d)\n",

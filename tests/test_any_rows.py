@@ -107,6 +107,27 @@ def test_emulated_last_chunk_writes_its_own(emu_softmax, cols, dtype, groups):
     assert written == [r * cols + i for r in range(rows) for i in range(cols - own, cols)]
 
 
+@pytest.mark.parametrize("cols", [3, 5, 300])
+def test_emulated_exponential(emu_softmax, cols):
+    # rows of 0, d and -inf with d down to -104: exp(d) / (1 + exp(d)) by the exponential (about an ulp), the sum and the
+    # quotient (half an ulp each), against the fp64 value rounded once (half an ulp): 2.5 ulps; by expf in the scalar kernel
+    # (3 columns) as well
+    out = run(emu_softmax, [6000, cols, 0, 0, 1, 0, 0, 0, "pair"])
+    assert float(out.split("worst ")[1].split()[0]) <= 2.5, out
+
+
+# rows, cols, dtype, kernel nodes of a captured launch: rows that an eager launch takes from the row tier stay there (one
+# node), longer ones have the co-resident tier's tag node before theirs
+CAPTURED = [(8, 30000, 0, 1), (8, 30001, 0, 1), (8, 60000, 1, 1), (8, 60001, 1, 1), (2, 33000, 0, 2), (2, 65537, 1, 2)]
+
+
+@pytest.mark.parametrize("rows,cols,dtype,nodes", CAPTURED)
+def test_emulated_captured_launches(emu_softmax, rows, cols, dtype, nodes):
+    env = dict(os.environ, EMU_CLOCK_STOPPED="1", EMU_GRAPH="1")
+    out = run(emu_softmax, [rows, cols, dtype, 0, 1, 0, 0, 0, "randn", 2], env=env, concurrent=True)
+    assert int(out.split("graph nodes ")[1].split(",")[0]) == nodes, out
+
+
 SAME = [(5, 50000, 0, 0), (5, 50001, 0, 0), (6, 70000, 0, 2), (6, 70001, 0, 2), (60, 20000, 0, 0), (6, 50000, 1, 2),
         (6, 50001, 1, 2), (4, 70000, 1, 0), (4, 70001, 1, 0)]
 
@@ -303,8 +324,10 @@ def test_gpu_rows_on_two_streams(pkg, oracle, dev):
 
 @pytest.mark.gpu
 def test_gpu_captured_rows_take_the_row_tier(pkg, oracle, dev):
-    # a captured launch of rows that an eager launch hands to the co-resident tier: replays on new values
+    # a captured launch of rows that an eager launch hands to the co-resident tier, whose rounding is another: replays on
+    # new values give the row tier's bits
     x = torch.empty(8, 30000, device=dev)
+    lib = pkg.candidate("softmax")._lib
     pkg.softmax(x)
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
@@ -317,6 +340,49 @@ def test_gpu_captured_rows_take_the_row_tier(pkg, oracle, dev):
         graph.replay()
         torch.cuda.synchronize()
         assert_rel(y.cpu().numpy(), oracle.softmax(h.numpy(), "fp32"), 1e-5, f"replay {seed}", 2.0 ** -147)
+        assert not torch.equal(y, pkg.softmax(x))
+        try:
+            lib.softmax_tune(5, 1)
+            assert torch.equal(y, pkg.softmax(x))
+        finally:
+            lib.softmax_tune(5, 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cols", [3, 5, 300])
+def test_gpu_exponential(pkg, dev, cols):
+    # as test_emulated_exponential, with the hardware's exp2 (an ulp) inside the exponential: 3 ulps
+    print(f"[softmax exponential] {cols}", flush=True)
+    d = torch.linspace(-103.9, 0, 60000, device=dev)
+    x = torch.full((60000, cols), float("-inf"), device=dev)
+    x[:, 0] = 0
+    x[:, 1] = d
+    y = pkg.softmax(x)[:, 1].double()
+    exact = d.double().exp() / (1 + d.double().exp())
+    ulp = torch.exp2((exact.log2().floor() - 23).clamp(min=-149))
+    worst = ((y - exact).abs() / ulp).max().item()
+    assert worst <= 3, worst
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols,dtype", [(600, 40000, torch.bfloat16), (1024, 50001, torch.bfloat16),
+                                             (500, 20000, torch.float32), (64, 262144, torch.float32)])
+def test_gpu_two_launches_that_fill_the_gpu(pkg, dev, rows, cols, dtype):
+    # on two streams at once, over and over: each has the bits that it has alone
+    print(f"[softmax two] {rows}x{cols} {dtype}", flush=True)
+    xs = [(torch.randn(rows, cols, device=dev, generator=torch.Generator(device=dev).manual_seed(i)) * 3).to(dtype)
+          for i in range(2)]
+    alone = [pkg.softmax(x) for x in xs]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    for _ in range(4):
+        ys = [[], []]
+        for _ in range(5):
+            for i in range(2):
+                with torch.cuda.stream(streams[i]):
+                    ys[i].append(pkg.softmax(xs[i]))
+        torch.cuda.synchronize()
+        assert all(torch.equal(y, alone[i]) for i in range(2) for y in ys[i])
 
 
 @pytest.mark.gpu
