@@ -19,7 +19,7 @@
 // slots across waves) and writes y from the registers; each lane holds the weight vectors of its columns once for all
 // rows. Workgroups are persistent and load their next row while they reduce and store the current one. Rows of any
 // other length from 8 columns up, or otherwise aligned, run the same kernel with element-aligned vectors (Form kAny);
-// aligned rows of at most 32 vectors share waves, four at a time (rmsnorm_short). What is left (rows of fewer than 8
+// aligned rows of at most 32 vectors share waves, four at a time, when there are many of them (rmsnorm_short). What is left (rows of fewer than 8
 // columns, or longer than 16 waves hold) takes a generic kernel (one workgroup per row, scalar accesses, two passes).
 #include <climits>
 #include <cmath>
@@ -372,8 +372,8 @@ __global__ void __launch_bounds__(256)
 // ---- host side ------------------------------------------------------------------------------------------------------
 
 // Tuning slots (0 = automatic): waves per row, vectors per lane, resident blocks per CU, forced generic kernel (1),
-// non-temporal loads (1 on, 2 off).
-enum { kTuneWaves = 0, kTuneNv = 1, kTuneBlocksPerCu = 2, kTuneGeneric = 3, kTuneNtLoads = 4 };
+// non-temporal loads (1 on, 2 off), the short rows' kernel for every row it can hold (1) or none (2).
+enum { kTuneWaves = 0, kTuneNv = 1, kTuneBlocksPerCu = 2, kTuneGeneric = 3, kTuneNtLoads = 4, kTuneShort = 5 };
 
 int pow2_at_least(long long v) {
   int p = 1;
@@ -474,6 +474,15 @@ int launch_short(const Args& a) {
   return (int)hipGetLastError();
 }
 
+// Whether rows of at most 32 vectors share waves: sixteen of them take longer than the row kernel's one, which few rows
+// do not make up for. Kernel times in us, a wave per row / shared: 128 columns bf16 64 rows 2.1 / 2.5, 2048 2.5 / 2.7,
+// 3000 2.7 / 2.7, 8192 4.1 / 3.1; 256 columns 64 rows 2.1 / 3.2, 6000 3.7 / 4.0, 8192 4.3 / 4.1, 32768 11.2 / 7.2.
+bool takes_short(long long rows, long long nvec) {
+  const int want = rw_host::tune_get(kTuneShort);
+  if (want > 0) return want == 1;
+  return rows >= (nvec <= kShortLanes ? 12LL : 28LL) * rw_host::device_cus();
+}
+
 template <typename T, bool HAS_W, bool RES = false>
 int launch_typed(const void* x, const void* w, void* y, long long rows, int cols, float eps, hipStream_t stream,
                  const void* res = nullptr, void* res_out = nullptr) {
@@ -493,7 +502,7 @@ int launch_typed(const void* x, const void* w, void* y, long long rows, int cols
     auto auto_nv = [&](int w) { return pow2_at_least((nvec + (long long)w * kWave - 1) / ((long long)w * kWave)); };
     int waves = rw_host::tune_get(kTuneWaves), nv = rw_host::tune_get(kTuneNv);
     if constexpr (!RES) {
-      if (vec && nvec <= 2 * kShortLanes && waves <= 0 && nv <= 0) {
+      if (vec && nvec <= 2 * kShortLanes && waves <= 0 && nv <= 0 && takes_short(rows, nvec)) {
         // 65536 x 256 bf16 28.0 -> 14.4 us, 65536 x 8 23.7 -> 4.6
         const Args a{x, w, y, res, res_out, rows, nvec, cols, eps, stream, any};
         return nvec <= kShortLanes ? launch_short<T, 1, HAS_W>(a) : launch_short<T, 2, HAS_W>(a);

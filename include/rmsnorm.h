@@ -26,7 +26,8 @@ int rmsnorm_add_launch(const void* x, const void* residual, const void* weight, 
                        long long rows, int cols, int dtype, float eps, int threads, hipStream_t stream);
 
 /* No counterpart in the reference: tuning override for parameter sweeps. Slots: 0 waves per row, 1 vectors per lane,
- * 2 resident blocks per CU, 3 forced generic kernel (1), 4 non-temporal loads (default on; 2 off). Returns 0 or -1. */
+ * 2 resident blocks per CU, 3 forced generic kernel (1), 4 non-temporal loads (default on; 2 off), 5 the
+ * short rows' kernel for every row it can hold (1) or none (2). Returns 0 or -1. */
 int rmsnorm_tune(int slot, int value);
 
 #ifdef __cplusplus

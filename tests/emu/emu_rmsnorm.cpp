@@ -51,6 +51,7 @@ int main(int argc, char** argv) {
     rmsnorm_tune(0, atoi(argv[6]));
     rmsnorm_tune(1, atoi(argv[7]));
     rmsnorm_tune(2, atoi(argv[8]));
+    if (const char* s = std::getenv("EMU_SHORT")) rmsnorm_tune(5, atoi(s));  // the short rows' kernel: 1 always, 2 never
   }
   const int offset = argc > 9 ? atoi(argv[9]) : 0;
   const float eps = 1e-6f;
@@ -98,6 +99,7 @@ int main(int argc, char** argv) {
     for (size_t i = 0; i < n && first < 0; ++i)
       if (got[i] != ry[i]) first = (long long)i;
   }
+  std::printf("workgroups %llu\n", emu::last_grid());
   std::printf("rows %lld cols %d dtype %d mode %d: %s (err %d, first difference %lld)\n", rows, cols, dtype, mode,
               ok ? "ALL OK" : "FAILED", err, first);
   hipFree(xb);

@@ -26,7 +26,14 @@ CASES = [(1, 8, 1, 1), (3, 64, 2, 0), (4, 120, 1, 1), (15, 128, 1, 1), (16, 128,
 
 @pytest.mark.parametrize("rows,cols,dtype,mode", CASES)
 def test_emulated_short_rows(emu_rmsnorm, rows, cols, dtype, mode):
-    run(emu_rmsnorm, [rows, cols, dtype, mode, rows + cols, 0, 0, 0, 0])
+    run(emu_rmsnorm, [rows, cols, dtype, mode, rows + cols, 0, 0, 0, 0], env=dict(os.environ, EMU_SHORT="1"))
+
+
+# where rows begin to share waves (256 CUs): one-wave workgroups of sixteen rows, or four-wave ones of a row a wave
+@pytest.mark.parametrize("rows,cols,workgroups", [(64, 128, 16), (3071, 128, 768), (3072, 128, 192), (64, 256, 16), (7168, 256, 448)])
+def test_emulated_few_short_rows(emu_rmsnorm, rows, cols, workgroups):
+    out = run(emu_rmsnorm, [rows, cols, 1, 1, rows, 0, 0, 0, 0])
+    assert int(out.split("workgroups ")[1].split()[0]) == workgroups, out
 
 
 # rows, cols, mode (0 plain, 1 weighted, 2 add, 3 add in place), waves, nv, offset (elements off a 16-byte boundary)
@@ -96,11 +103,21 @@ def test_gpu_negative_zeros(pkg, oracle, dev, dtype, cols):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("short", [0, 1], ids=["auto", "short"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("rows,cols", [(1, 8), (5, 64), (16, 80), (17, 96), (4095, 128), (16384, 128), (16401, 136),
                                        (40000, 192), (163841, 128), (70000, 256), (300, 264), (70001, 512)])
-def test_gpu_short_rows(pkg, oracle, dev, dtype, rows, cols):
-    print(f"[rmsnorm short] {rows}x{cols} {dtype}", flush=True)
+def test_gpu_short_rows(pkg, oracle, dev, dtype, rows, cols, short):
+    print(f"[rmsnorm short] {rows}x{cols} {dtype} {short}", flush=True)
+    lib = pkg.candidate("rmsnorm")._lib
+    lib.rmsnorm_tune(5, short)
+    try:
+        _short_rows(pkg, lib, oracle, dev, dtype, rows, cols)
+    finally:
+        lib.rmsnorm_tune(5, 0)
+
+
+def _short_rows(pkg, lib, oracle, dev, dtype, rows, cols):
     g = torch.Generator().manual_seed(rows + cols)
     x = (torch.randn(rows, cols, generator=g) * torch.rand(rows, 1, generator=g) * 3).to(dtype)
     x[rows // 2, cols // 2] = float("nan")
@@ -113,7 +130,6 @@ def test_gpu_short_rows(pkg, oracle, dev, dtype, rows, cols):
         ref = oracle.rmsnorm(bits16(x), None if weight is None else bits16(weight), eps=1e-5, dtype=name)
         assert same_bits16(bits16(y), ref, fp16)
     d = x.to(dev)  # in place through the C entry point
-    lib = pkg.candidate("rmsnorm")._lib
     assert lib.launch(d.data_ptr(), d.data_ptr(), rows, cols, 2 if fp16 else 1, 1e-5, 256,
                       torch.cuda.current_stream().cuda_stream) == 0
     assert same_bits16(bits16(d), ref, fp16)
