@@ -102,6 +102,10 @@ __device__ __forceinline__ void apart(float& v) {
   if constexpr (std::is_same<T, F16>::value) asm volatile("" : "+v"(v));
 }
 
+// Whether vectors past the row's end for the whole wave are passed over: 16384 x 5120 bf16 64.2 -> 62.3 us, with a residual
+// 1% slower; 64 x 640, whose lanes hold two vectors, 2.28 -> 2.37.
+template <int FORM, int NV, bool RES> constexpr bool kSkips = FORM == kAny || (FORM == kPart && !RES && NV >= 4);
+
 template <typename T, int WAVES, int NV, int FORM, bool HAS_W, bool RES, bool NTS>
 __device__ __forceinline__ void norm_row(const Regs<NV>& r, const Regs<NV>& w, void* y, void* res_out, long long row,
                                          const Place<FORM, WAVES * kWave>& at, float eps, bool active, double* slots,
@@ -109,8 +113,7 @@ __device__ __forceinline__ void norm_row(const Regs<NV>& r, const Regs<NV>& w, v
   double acc = 0.0;
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
-    // (kPart with a residual measured 1% slower with the skip at 16384 x 5120; without one 64.2 -> 62.3 us)
-    if (!(FORM == kPart && RES) && !at.used(k)) continue;
+    if (kSkips<FORM, NV, RES> && !at.used(k)) continue;
     float f[T::V];
     unpack<T>(r.v[k], f);
     if (FORM == kAny && !at.whole(k)) {
@@ -184,7 +187,7 @@ __global__ void __launch_bounds__((WAVES < 4 ? 4 : WAVES) * 64)
   constexpr int GROUPS = BW / WAVES;
   constexpr int G = WAVES * kWave;
   __shared__ double slots[2][BW];
-  const int wave = FORM == kAny || (FORM == kPart && !RES) ? __builtin_amdgcn_readfirstlane(wave_id()) : wave_id();
+  const int wave = kSkips<FORM, NV, RES> ? __builtin_amdgcn_readfirstlane(wave_id()) : wave_id();
   const int first = (wave / WAVES) * WAVES;
   const Place<FORM, G> at{nvec, cols, (int)threadIdx.x - first * kWave, (wave - first) * kWave};
   const long long step = (long long)gridDim.x * GROUPS;
