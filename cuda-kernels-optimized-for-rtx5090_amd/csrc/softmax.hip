@@ -5,7 +5,7 @@
 // Tiers, chosen by row length in 16-byte vectors (4 fp32 or 8 bf16 elements). The first two have an instantiation for
 // rows whose length is a multiple of the vector width and whose x and y are 16-byte aligned, and one for any other rows
 // of at least one vector (AnyRow):
-//  - short rows (at most 64 vectors): four rows side by side in a wave; see softmax_short.
+//  - many short rows (at most 64 vectors): four rows side by side in a wave; see softmax_short.
 //  - row tier (rows up to 16 waves x 64 lanes x 8 vectors = 32768 fp32 / 65536 bf16 columns): a group of WAVES waves
 //    holds one row in registers, NV 16-byte vectors per lane. A max and a sum of exp(x - max) are reduced over the
 //    group (DPP inside each wave, one LDS slot per wave across waves) and y = exp(x - max) / sum is written from the
@@ -748,9 +748,10 @@ __global__ void __launch_bounds__(256)
 // resident blocks per CU, stream-tier waves, co-resident row groups (fewer forces more rows per workgroup), preferred
 // tier (1 row, 2 stream, 3 generic, 4 co-resident; a tier that cannot take the rows is passed over for the automatic
 // choice), non-temporal loads (1 on, 2 off), the co-resident tier's wait budget in 100 MHz ticks (tests force its
-// fallback with 1), the co-resident tier's vectors per lane (the longest chunks', half or a quarter of it).
+// fallback with 1), the co-resident tier's vectors per lane (the longest chunks', half or a quarter of it), the short
+// rows' kernel for every row it can hold (1) or none (2).
 enum { kTuneWaves = 0, kTuneNv = 1, kTuneBlocksPerCu = 2, kTuneStreamWaves = 3, kTuneCoopGroups = 4, kTuneTier = 5,
-       kTuneNtLoads = 6, kTuneWaitTicks = 7, kTuneCoopNv = 8 };
+       kTuneNtLoads = 6, kTuneWaitTicks = 7, kTuneCoopNv = 8, kTuneShort = 9 };
 constexpr unsigned kCoopWaitTicks = 10000;  // 100 us: tens of times a row's arrival skew, a few launch lengths
 
 bool aligned_to(const void* p, int bytes) { return (reinterpret_cast<uintptr_t>(p) & (uintptr_t)(bytes - 1)) == 0; }
@@ -1104,6 +1105,16 @@ bool coop_instead_of_rows(long long rows, long long nvec, hipStream_t stream) {
   return (nvec > 4096 || (nvec > 2048 && rows <= 32)) && !capturing(stream);
 }
 
+// Whether rows of at most 64 vectors share waves: eight or sixteen of them take longer than the row tier's one, which few
+// rows do not make up for. Kernel times in us, a wave per row / shared: 128 columns fp32 64 rows 2.0 / 2.4, 2048 2.2 /
+// 2.5, 4096 2.9 / 2.6, 16384 6.6 / 3.6; 64 columns bf16 64 rows 2.0 / 2.8, 4096 3.0 / 2.9; more than 32 vectors: bf16 4096
+// x 257 3.6 / 4.8, 8000 x 257 4.6 / 5.3, 65536 x 257 22.4 / 20.0; fp32 4096 x 200 3.1 / 3.6, 65536 x 256 22.9 / 20.2.
+bool takes_short(long long rows, long long nvec) {
+  const int want = rw_host::tune_get(kTuneShort);
+  if (want > 0) return want == 1;
+  return rows >= (nvec <= 2 * kShortLanes ? 16LL : 32LL) * rw_host::device_cus();
+}
+
 template <typename T>
 int launch_typed(const void* x, void* y, long long rows, long long cols, hipStream_t stream) {
   const bool vec = cols % T::V == 0 && rw_host::aligned16(x) && rw_host::aligned16(y);
@@ -1111,9 +1122,7 @@ int launch_typed(const void* x, void* y, long long rows, long long cols, hipStre
   const bool any = cols >= T::V && aligned_to(x, T::bytes) && aligned_to(y, T::bytes);
   if (tier == 3 || !(vec || any)) return launch_generic<T>(x, y, rows, cols, stream);
   const long long nvec = (cols + T::V - 1) / T::V;
-  // (four vectors per lane: only with rows enough to keep the GPU full at eight to a wave; 4096 x 257 bf16 3.7 us as a
-  // wave per row, 4.3 as short rows; 65536 x 257 19.1 and 17.5)
-  if (any && nvec <= (rows >= 8192 ? 4 : 2) * kShortLanes && tier == 0 && !row_shape_tuned())
+  if (any && nvec <= 4 * kShortLanes && tier == 0 && !row_shape_tuned() && takes_short(rows, nvec))
     return vec ? launch_short<T, T::bytes == 4>(x, y, rows, cols, stream)
                : launch_short<T, true>(x, y, rows, cols, stream);
   if (!vec) {

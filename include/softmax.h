@@ -30,7 +30,7 @@ int launch(const void* x, void* y, long long rows, long long cols, int dtype, in
  * automatic choice). Slots: 0 waves per row, 1 vectors per lane, 2 resident blocks per CU, 3 stream-tier waves, 4
  * co-resident row groups, 5 preferred tier (1 row, 2 stream, 3 generic, 4 co-resident; a tier that cannot take the
  * rows is passed over), 6 non-temporal loads (1 on), 7 the co-resident wait budget in 100 MHz ticks, 8 the co-resident
- * tier's vectors per lane. Returns 0 or -1. */
+ * tier's vectors per lane, 9 the short rows' kernel for every row it can hold (1) or none (2). Returns 0 or -1. */
 int softmax_tune(int slot, int value);
 
 #ifdef __cplusplus

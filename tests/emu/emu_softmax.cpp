@@ -57,6 +57,7 @@ int main(int argc, char** argv) {
   const std::string pattern = argc > 9 ? argv[9] : "randn";
   const int reps = argc > 10 ? atoi(argv[10]) : 1;
   if (argc > 11) softmax_tune(7, atoi(argv[11]));
+  if (const char* s = std::getenv("EMU_SHORT")) softmax_tune(9, std::atoi(s));  // the short rows' kernel: 1 always, 2 never
   softmax_tune(5, tier);
   if (tier == 2) {
     softmax_tune(3, waves);

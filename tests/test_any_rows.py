@@ -39,7 +39,16 @@ SHORT = [(1, 4, 0), (3, 5, 0), (17, 63, 0), (16, 64, 0), (9, 65, 0), (33, 127, 0
 @pytest.mark.parametrize("pattern", ["randn", "special"])
 @pytest.mark.parametrize("rows,cols,dtype", SHORT)
 def test_emulated_short_rows(emu_softmax, rows, cols, dtype, pattern):
-    run(emu_softmax, [rows, cols, dtype, 0, cols, 0, 0, cols % 4, pattern])
+    run(emu_softmax, [rows, cols, dtype, 0, cols, 0, 0, cols % 4, pattern], env=dict(os.environ, EMU_SHORT="1"))
+
+
+# where rows begin to share waves (256 CUs): workgroups of one wave of 16 or 8 rows, or of four waves of a row each
+@pytest.mark.parametrize("rows,cols,dtype,offset,workgroups", [(64, 64, 0, 0, 16), (4095, 64, 0, 0, 512), (4096, 64, 0, 0, 256),
+                                                               (64, 128, 1, 1, 16), (4096, 200, 1, 0, 512),
+                                                               (4096, 200, 0, 0, 512), (8192, 200, 0, 0, 256)])
+def test_emulated_few_short_rows(emu_softmax, rows, cols, dtype, offset, workgroups):
+    out = run(emu_softmax, [rows, cols, dtype, 0, rows, 0, 0, offset])
+    assert int(out.split("workgroups ")[1].split(",")[0]) == workgroups, out
 
 
 @pytest.mark.parametrize("dtype,waves,nv", [(0, 1, 8), (0, 2, 4), (0, 16, 1), (1, 1, 8), (1, 8, 2)])
@@ -207,6 +216,20 @@ def _check(pkg, oracle, dev, rows, cols, dtype, offset=0, special=False):
                                        (2, 1048577), (3, 16385), (9, 36869), (300, 49153)])
 def test_gpu_rows(pkg, oracle, dev, dtype, rows, cols):
     _check(pkg, oracle, dev, rows, cols, dtype, offset=1, special=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("short", [1, 2], ids=["short", "row"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("rows,cols,offset", [(3, 8, 0), (70, 9, 0), (1000, 64, 0), (333, 131, 0), (9000, 255, 1), (777, 256, 0),
+                                              (5, 200, 3), (40000, 8, 0), (8193, 100, 0)])
+def test_gpu_short_rows_either_way(pkg, oracle, dev, dtype, rows, cols, offset, short):
+    lib = pkg.candidate("softmax")._lib
+    lib.softmax_tune(9, short)
+    try:
+        _check(pkg, oracle, dev, rows, cols, dtype, offset=offset, special=True)
+    finally:
+        lib.softmax_tune(9, 0)
 
 
 @pytest.mark.gpu
