@@ -19,8 +19,9 @@
 // slots across waves) and writes y from the registers; each lane holds the weight vectors of its columns once for all
 // rows. Workgroups are persistent and load their next row while they reduce and store the current one. Rows of any
 // other length from 8 columns up, or otherwise aligned, run the same kernel with element-aligned vectors (Form kAny);
-// aligned rows of at most 32 vectors share waves, four at a time, when there are many of them (rmsnorm_short). What is left (rows of fewer than 8
-// columns, or longer than 16 waves hold) takes a generic kernel (one workgroup per row, scalar accesses, two passes).
+// aligned rows of at most 32 vectors share waves, four at a time, when there are many of them (rmsnorm_short). What is
+// left (rows of fewer than 8 columns, or longer than 16 waves hold) takes a generic kernel (one workgroup per row,
+// scalar accesses, two passes).
 #include <climits>
 #include <cmath>
 #include <type_traits>
@@ -102,8 +103,8 @@ __device__ __forceinline__ void apart(float& v) {
   if constexpr (std::is_same<T, F16>::value) asm volatile("" : "+v"(v));
 }
 
-// Whether vectors past the row's end for the whole wave are passed over: 16384 x 5120 bf16 64.2 -> 62.3 us, with a residual
-// 1% slower; 64 x 640, whose lanes hold two vectors, 2.28 -> 2.37.
+// Whether vectors past the row's end for the whole wave are passed over: 16384 x 5120 bf16 64.2 -> 62.3 us, with a
+// residual 1% slower; 64 x 640, whose lanes hold two vectors, 2.28 -> 2.37.
 template <int FORM, int NV, bool RES> constexpr bool kSkips = FORM == kAny || (FORM == kPart && !RES && NV >= 4);
 
 template <typename T, int WAVES, int NV, int FORM, bool HAS_W, bool RES, bool NTS>

@@ -14,15 +14,15 @@
 //  - co-resident tier (longer rows, up to 64 chunks of 16384 elements): one pass over x for any number of rows; see
 //    softmax_coop.
 //  - stream tier (longer rows still, aligned): one workgroup per row, two passes, no workspace; see softmax_stream.
-//  - generic tier (what is left: rows shorter than a vector, and unaligned rows beyond the co-resident tier): one
-//    workgroup per row, three scalar passes (max, sum, write).
+//  - generic tier (what is left: rows shorter than a vector, and unaligned rows beyond the co-resident tier or, in
+//    place, beyond the row tier): one workgroup per row, three scalar passes (max, sum, write).
 // The library allocates no device memory: the co-resident tier exchanges its chunk pairs through a static device
 // table whose entries carry a per-launch tag, so nothing has to be cleared between launches; launches recorded into a
 // HIP graph take fresh tags at every replay (see softmax_coop).
-// Aligned rows of the row tier and the stream tier multiply by the fp32 reciprocal of the row sum (the reference divides,
-// softmax/kernel.cu:240; the two differ by at most 1.5 ulp in fp32 and are within the 1e-5 relative tolerance of the
-// fp64 oracle); rows of other lengths and alignments, short fp32 rows and the fp32 chunks held as x take the quotient
-// (quotient below), the generic tier the division.
+// Aligned rows of the row tier and the stream tier multiply by the fp32 reciprocal of the row sum (the reference
+// divides, softmax/kernel.cu:240; the two differ by at most 1.5 ulp in fp32 and are within the 1e-5 relative tolerance
+// of the fp64 oracle); rows of other lengths and alignments, short fp32 rows and the fp32 chunks held as x take the
+// quotient (quotient below), the generic tier the division.
 #include <climits>
 #include <cmath>
 #include <mutex>
@@ -171,13 +171,12 @@ __global__ void __launch_bounds__((WAVES < 4 ? 4 : WAVES) * 64)
 
 // Row tier for rows of any length from one vector up and any element alignment: the lanes' vectors start at the row's
 // first element, wherever it lies, and a vector that would pass the row's end is moved back to end with it. Its first
-// elements are then another lane's of the same workgroup (the same bits, from the same maximum and sum: the same results
-// when they are stored twice), so the maximum
-// takes every loaded element and the sum leaves out the first `skip` of the vector; only the wave that holds the row's
-// end looks at that, and vectors that lie past the end for a whole wave are not worked on.
-// 8192 x 3001 bf16 62.1 us through the scalar kernel's three passes of 2-byte accesses, 18.3 us here (17.0 with
-// exp_narrow and the reciprocal, which round 1.3e-4 of the distinct values of a row otherwise than the fp64 softmax; the
-// scalar kernel's expf and division 0.45e-4, as here).
+// elements are then another lane's of the same workgroup (the same bits, from the same maximum and sum: the same
+// results when they are stored twice), so the maximum takes every loaded element and the sum leaves out the first
+// `skip` of the vector; only the wave that holds the row's end looks at that, and vectors that lie past the end for a
+// whole wave are not worked on. 8192 x 3001 bf16: 62.1 us through the scalar kernel's three passes of 2-byte accesses,
+// 18.3 us here (17.0 with exp_narrow and the reciprocal, which round 1.3e-4 of the distinct values of a row otherwise
+// than the fp64 softmax; the scalar kernel's expf and division 0.45e-4, as here).
 template <typename T, int WAVES, int NV>
 struct AnyRow {
   static constexpr int G = WAVES * kWave, V = T::V;
@@ -215,8 +214,8 @@ struct AnyRow {
       for (int i = 0; i < V; ++i) f[k][i] = exp_nonpositive(f[k][i] - m);
       s[k] = whole(k) ? sum_vector<T>(f[k], 0) : sum_vector<T>(f[k], start(k) - offset(k));
     }
-    // in pairs, as within a vector and over the waves: the error of a long chain of additions is kept out (unaligned fp32
-    // rows of 10000, 2-norm of the error: 8.5e-8 in the scalar kernel, 9.6e-8 with the waves one after another)
+    // in pairs, as within a vector and over the waves: the error of a long chain of additions is kept out (unaligned
+    // fp32 rows of 10000, 2-norm of the error: 8.5e-8 in the scalar kernel, 9.6e-8 with the waves one after another)
 #pragma unroll
     for (int d = 1; d < NV; d *= 2)
 #pragma unroll
@@ -271,10 +270,10 @@ __global__ void __launch_bounds__((WAVES < 4 ? 4 : WAVES) * 64)
 // wave, and a wave takes SETS times four rows per step, so that lanes hold data and several loads are in flight where a
 // wave per row would have one, mostly empty. The reductions stay inside a 16-lane DPP row; no LDS and no barrier. Waves
 // are persistent and load their next rows while they work on these.
-// 65536 rows, us as a wave per row / here: fp32 8 columns 20.8 / 4.7, 64 22.5 / 6.5, 128 23.0 / 11.0, 256 23.6 / 20.3;
-// bf16 64 24.5 / 5.9, 131 17.9 / 10.5 (55 in the scalar kernel), 512 24.0 / 21.5.
+// 65536 rows, us as a wave per row / here: fp32 8 columns 20.3 / 4.7, 64 21.8 / 6.4, 128 22.0 / 10.9, 256 22.9 / 20.2;
+// bf16 64 23.6 / 5.4, 131 22.2 / 10.1 (54 in the scalar kernel), 512 23.5 / 21.5.
 // FINE: the exponential and the quotient within an fp32 ulp (fp32 rows, and bf16 rows that would otherwise take the
-// scalar kernel); without it exp_narrow and the reciprocal, as in the row tier (65536 x 64 bf16 5.5 us, FINE 6.7).
+// scalar kernel); without it exp_narrow and the reciprocal, as in the row tier (65536 x 64 bf16 5.4 us, FINE 6.7).
 constexpr int kShortLanes = 16;
 
 template <typename Op>
@@ -421,15 +420,16 @@ __global__ void __launch_bounds__(WAVES * 64)
   }
 }
 
-// Co-resident tier: long rows in chunks of WAVES x 64 x NV vectors, one workgroup per chunk, every workgroup of a launch
-// resident at once (the grid never exceeds the GPU's resident slots of this kernel): x is read once (1R + 1W). The
-// grid is `groups` row groups of `chunks` workgroups; group g handles rows g, g + groups, ..., one row per iteration,
-// so any number of rows keeps one pass over x. Per iteration, each workgroup holds its chunk in registers as
-// e = exp(x - m) in fp32 (one exp per element), reduces it to its online-softmax pair (m, s = sum of e), and publishes
-// the pair into its slot of the device-scope pair table; wave 0 polls the group's slots until every chunk's pair of
-// this row is there, merges them in a fixed order (the online-softmax merge, the same lanes and order in every
+// Co-resident tier: long rows in chunks of WAVES x 64 x NV vectors, one workgroup per chunk, every workgroup of a
+// launch resident at once (the grid never exceeds the GPU's resident slots of this kernel): x is read once (1R + 1W).
+// The grid is `groups` row groups of `chunks` workgroups; group g handles rows g, g + groups, ..., one row per
+// iteration, so any number of rows keeps one pass over x. Per iteration, each workgroup holds its chunk in registers,
+// as x or as e = exp(x - m) in fp32 (HOLD below), reduces it to its online-softmax pair (m, s = sum of e), and
+// publishes the pair into its slot of the device-scope pair table; wave 0 polls the group's slots until every chunk's
+// pair of this row is there, merges them in a fixed order (the online-softmax merge, the same lanes and order in every
 // workgroup of the row, so all agree bit for bit; softmax/kernel.cu:121-152 is the reference's form of it), and the
-// chunk is written as e * (exp(m - M) / S), within 3 fp32 ulp of the once-rounded value before the output's rounding.
+// chunk is written as exp(x - M) / S or as e * (exp(m - M) / S), the latter within 3 fp32 ulp of the once-rounded value
+// before the output's rounding.
 //
 // The pair table needs no clearing: each pair is two 64-bit words, (tag << 32 | m bits) and (tag << 32 | s bits),
 // stored with device-coherent stores, and a word counts only when its tag is this launch's tag for the iteration.
@@ -490,17 +490,17 @@ __global__ void __launch_bounds__(256) softmax_coop_cell(int cell, unsigned iter
 // kernel is compiled without the loop (which costs registers: fewer resident workgroups).
 // ANY: rows of any length (nvec vectors, the last one partial) and element alignment. The row's last vector is moved
 // back to end with the row (AnyRow), its first `skip` elements being another lane's.
-// FINE: the exponential within an fp32 ulp, for fp32 rows, for bf16 rows that the scalar kernel would take and for those
-// that an eager launch takes from the row tier and holds as e; other bf16 rows take exp_narrow. (Share of a bf16 row's
-// distinct values that are rounded otherwise than the fp64 softmax's: 512 x 40000 aligned 1.27e-4 in the row tier, here
-// 1.40e-4 with exp_narrow and 0.59e-4 FINE; unaligned 0.59e-4 in the scalar kernel and here.)
-// The waves per SIMD asked of the compiler are those it reaches by itself without the code behind a wait that ended,
-// which would otherwise cost the loop's bf16 forms one of four (256 x 262144 52.0 us, 54.5 with three).
+// FINE: the exponential within an fp32 ulp, for fp32 rows, for bf16 rows that the scalar kernel would take and for
+// those that an eager launch takes from the row tier and holds as e; other bf16 rows take exp_narrow. (Share of a bf16
+// row's distinct values that are rounded otherwise than the fp64 softmax's: 512 x 40000 aligned 1.27e-4 in the row
+// tier, here 1.40e-4 with exp_narrow and 0.59e-4 FINE; unaligned 0.59e-4 in the scalar kernel and here.)
 // HOLD: the chunk is held as e = exp(x - m) and written as e * (exp(m - M) / S); otherwise it is held as x, and the
 // exponential is taken again from M. Holding e saves an exponential per element, which long chunks of many rows feel
-// (1024 x 50000 fp32 77 us against 84, bf16 44 against 50), and costs fp32 rows accuracy where the chunk is short
-// (mean relative error of 16 x 128256 fp32: 1.47e-7 in four times longer chunks, 1.57e-7 as e, 1.03e-7 from x). So
-// short chunks and unaligned fp32 rows are held as x.
+// (1024 x 50000 fp32 77 us against 84, bf16 44 against 50), and costs fp32 rows accuracy where the chunk is short (mean
+// relative error of 16 x 128256 fp32: 1.47e-7 in four times longer chunks, 1.57e-7 as e, 1.03e-7 from x). So short
+// chunks and unaligned fp32 rows are held as x.
+// The waves per SIMD asked of the compiler are those it reaches by itself without the code behind a wait that ended,
+// which would otherwise cost the loop's bf16 forms one of four (256 x 262144 52.0 us, 54.5 with three).
 template <typename T, int WAVES, int NV, bool NTL, bool NTS, bool LOOP, bool ANY, bool FINE>
 __global__ void __launch_bounds__(WAVES * 64, NV * T::V == 64 ? 4 : ANY ? 7 : 8)
     softmax_coop(const void* __restrict__ x, void* __restrict__ y, long long rows, long long nvec, long long cols,
@@ -515,8 +515,8 @@ __global__ void __launch_bounds__(WAVES * 64, NV * T::V == 64 ? 4 : ANY ? 7 : 8)
   __shared__ unsigned long long missing;       // the chunks whose pairs had not come when the wait ended
   __shared__ float pairs[kCoopMaxChunks][2];  // the row's pairs then
   const int c = (int)(blockIdx.x % (unsigned)chunks), group = (int)(blockIdx.x / (unsigned)chunks);
-  // a chunk's place in the row: its first vector (< 2^31: at most kCoopMaxChunks chunks of CH vectors), its vectors, and
-  // (ANY) the elements from its first to the row's end, at least one
+  // a chunk's place in the row: its first vector (< 2^31: at most kCoopMaxChunks chunks of CH vectors), its vectors,
+  // and (ANY) the elements from its first to the row's end, at least one
   struct Part {
     int first, count, reach;
   };
@@ -597,11 +597,11 @@ __global__ void __launch_bounds__(WAVES * 64, NV * T::V == 64 ? 4 : ANY ? 7 : 8)
 #pragma unroll
     for (int k = 0; k < NV; ++k) s += exps(own, r.v[k], k, t, m == -INFINITY ? 0.0f : m, e[k]);
     s = group_reduce<WAVES>(s, OpSum{}, slots[1], wave_id(), 0);
-    // the next row's loads go out before the wait and the stores (bf16; for fp32 the two chunks together would halve the
-    // resident workgroups)
+    // the next row's loads go out before the wait and the stores (bf16; for fp32 the two chunks together would halve
+    // the resident workgroups)
     if constexpr (PREFETCH)
       if (it + 1 < iters) load_chunk(next, own, row + groups, t);
-    if (t == 0) {  // an all -inf chunk publishes (-inf, 0), which adds nothing to the merge; with a NaN in it, (-inf, NaN)
+    if (t == 0) {  // an all -inf chunk publishes (-inf, 0), which adds nothing to the merge; with a NaN, (-inf, NaN)
       __hip_atomic_store(&table[c][0], tag | __float_as_uint(m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __hip_atomic_store(&table[c][1], tag | __float_as_uint(s), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -631,7 +631,8 @@ __global__ void __launch_bounds__(WAVES * 64, NV * T::V == 64 ? 4 : ANY ? 7 : 8)
         if (__builtin_amdgcn_readfirstlane((int)(__builtin_amdgcn_s_memrealtime() - start > wait_ticks))) break;
         __builtin_amdgcn_s_sleep(1);
       }
-      const float pm = mine ? __uint_as_float((unsigned)wm) : -INFINITY, ps = mine ? __uint_as_float((unsigned)ws) : 0.0f;
+      const float pm = mine ? __uint_as_float((unsigned)wm) : -INFINITY;
+      const float ps = mine ? __uint_as_float((unsigned)ws) : 0.0f;
       if (left == 0) {
         merge(pm, ps);
       } else {
@@ -835,9 +836,8 @@ int launch_any_k(const void* x, void* y, long long rows, int cols, hipStream_t s
   if (occ <= 0) occ = blocks_per_cu(kern, BW * kWave);
   int per_cu = rw_host::tune_get(kTuneBlocksPerCu);
   // fp32 rows of four vectors a lane and more: the resident waves of launch_rows_k; otherwise about 24 waves per CU,
-  // whose loads are fewer or whose rows take more work per byte (8192 x 3001 fp32 as 4 waves x 4 vectors: 33.7 us with
-  // two blocks per CU, 34.8 with four; bf16 as 2 waves x 4 vectors: 17.3 with three, 16.9 with six; 65536 x 131 bf16:
-  // 23.5 with two, 17.7 with six)
+  // whose loads are fewer or whose rows take more work per byte (8192 x 3001 fp32 as 4 waves x 4 vectors: 33.5 us with
+  // two blocks per CU, 34.3 with four; bf16 as 2 waves x 4 vectors: 19.9 with two, 18.6 with three, 18.2 with six)
   if (per_cu <= 0) {
     const int resident = T::bytes == 4 && NV >= 4 ? (WAVES == 8 ? 16 : 8) : 24;
     per_cu = resident / BW > 1 ? resident / BW : 1;
@@ -913,8 +913,8 @@ int launch_stream(const void* x, void* y, long long rows, long long nvec, hipStr
 }
 
 // The co-resident tier's tags of eager launches: per device, the next unused one of the host's half of the tag space,
-// [1, 2^31) (0 is never handed out: it is the pair table's contents at load). A launch takes one per iteration; when the
-// range would pass 2^31 - 1, the table is cleared on the launch's stream and the tags start again at 1.
+// [1, 2^31) (0 is never handed out: it is the pair table's contents at load). A launch takes one per iteration; when
+// the range would pass 2^31 - 1, the table is cleared on the launch's stream and the tags start again at 1.
 unsigned coop_tags(int dev, unsigned n, hipStream_t stream, int* err) {
   static std::mutex mu;
   static unsigned next[64];
@@ -979,10 +979,10 @@ constexpr int kCoopWaves = 4;
 //  - bf16: shorter as long as no CU gets more workgroups. us by workgroups: 24 x 70000 120 5.6, 216 5.3, 432 5.9; 48 x
 //    70000 240 6.1, 432 6.3, 864 7.5; 24 x 128256 192 5.6, 384 6.2, 768 6.9; 1 x 262144 16 5.5, 32 5.0, 64 4.6; 96 x
 //    33000 288 7.8, 480 7.0, 864 7.5.
-//  - fp32, whose long chunks fill the registers: half as long up to four workgroups of the long ones per CU (200 x 50000
-//    800 17.0, 1400 13.6; 24 x 262144 384 11.6, 768 10.8; 96 x 128256 768 17.5, 1536 16.7), and a quarter while those are
-//    under four per CU and, beyond one per CU, at most 32 per row (200 x 20000 600 9.4, 1000 7.8; 1 x 262144 32 5.7, 64
-//    4.9; but 24 x 262144 1536 13.5, 16 x 262144 512 9.0, 1024 10.3).
+//  - fp32, whose long chunks fill the registers: half as long up to four workgroups of the long ones per CU (200 x
+//    50000 800 17.0, 1400 13.6; 24 x 262144 384 11.6, 768 10.8; 96 x 128256 768 17.5, 1536 16.7), and a quarter while
+//    those are under four per CU and, beyond one per CU, at most 32 per row (200 x 20000 600 9.4, 1000 7.8; 1 x 262144
+//    32 5.7, 64 4.9; but 24 x 262144 1536 13.5, 16 x 262144 512 9.0, 1024 10.3).
 template <typename T>
 int coop_nv(long long rows, long long nvec) {
   constexpr int NV = 64 / T::V;
@@ -1105,10 +1105,11 @@ bool coop_instead_of_rows(long long rows, long long nvec, hipStream_t stream) {
   return (nvec > 4096 || (nvec > 2048 && rows <= 32)) && !capturing(stream);
 }
 
-// Whether rows of at most 64 vectors share waves: eight or sixteen of them take longer than the row tier's one, which few
-// rows do not make up for. Kernel times in us, a wave per row / shared: 128 columns fp32 64 rows 2.0 / 2.4, 2048 2.2 /
-// 2.5, 4096 2.9 / 2.6, 16384 6.6 / 3.6; 64 columns bf16 64 rows 2.0 / 2.8, 4096 3.0 / 2.9; more than 32 vectors: bf16 4096
-// x 257 3.6 / 4.8, 8000 x 257 4.6 / 5.3, 65536 x 257 22.4 / 20.0; fp32 4096 x 200 3.1 / 3.6, 65536 x 256 22.9 / 20.2.
+// Whether rows of at most 64 vectors share waves: eight or sixteen of them take longer than the row tier's one, which
+// few rows do not make up for. Kernel times in us, a wave per row / shared: 128 columns fp32 64 rows 2.0 / 2.4, 2048
+// 2.2 / 2.5, 4096 2.9 / 2.6, 16384 6.6 / 3.6; 64 columns bf16 64 rows 2.0 / 2.8, 4096 3.0 / 2.9; more than 32 vectors:
+// bf16 4096 x 257 3.6 / 4.8, 8000 x 257 4.6 / 5.3, 65536 x 257 22.4 / 20.0; fp32 4096 x 200 3.1 / 3.6, 65536 x 256 22.9
+// / 20.2.
 bool takes_short(long long rows, long long nvec) {
   const int want = rw_host::tune_get(kTuneShort);
   if (want > 0) return want == 1;
@@ -1141,7 +1142,7 @@ int launch_typed(const void* x, void* y, long long rows, long long cols, hipStre
     if (!pow2_to(waves, kMaxWaves)) {
       waves = pow2_at_least(((nvec + 3) / 4 + kWave - 1) / kWave);
       // (fp32 rows for 16 waves of 4 vectors: 8 waves of 8 when there are rows for two such blocks per CU, 1024 x 16383
-      // 25.6 -> 24.3 us; bf16 600 x 32001 20.5 us as 16 x 4, 21.0 as 8 x 8)
+      // 24.1 -> 22.0 us; bf16 600 x 32001 23.4 us as 16 x 4, 24.2 as 8 x 8)
       if (T::bytes == 4 && waves == kMaxWaves && rows >= 2LL * rw_host::device_cus()) waves = kMaxWaves / 2;
       waves = waves > kMaxWaves ? kMaxWaves : waves;
     }

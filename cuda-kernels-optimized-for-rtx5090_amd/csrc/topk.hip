@@ -961,8 +961,9 @@ struct Tile {
 
   // max_key() of an fp32 tile by way of the signed maxima gm of its groups of 8 elements, which filter_groups takes:
   // the minima are looked at only when some lane of the wave holds no element from 0 up. About 60 of a wave's 590
-  // vector instructions fewer (k = 50: 128 x 128256 18.34 -> 18.2 us, 64 x 151936 15.9 -> 15.65, 8 x 128256 9.6 ->
-  // 9.4). (The wide kernel's group keys without the minima measured 0.1 to 0.3 us slower.)
+  // vector instructions fewer (k = 50: 64 x 151936 15.92 -> 15.72 us, 8 x 128256 9.52 -> 9.20, 16 x 32000 9.12 -> 8.83;
+  // 128 x 128256 k = 8 16.90 -> 16.66, k = 50 18.05 either way). (The wide kernel's group keys without the minima
+  // measured 0.1 to 0.3 us slower.)
   __device__ __forceinline__ uint32_t max_key_groups(int (&gm)[NV / 2]) const {
     group_maxima(gm);
     int mx = INT_MIN;
