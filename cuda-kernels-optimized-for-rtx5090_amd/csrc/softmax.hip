@@ -979,10 +979,11 @@ constexpr int kCoopWaves = 4;
 //  - bf16: shorter as long as no CU gets more workgroups. us by workgroups: 24 x 70000 120 5.6, 216 5.3, 432 5.9; 48 x
 //    70000 240 6.1, 432 6.3, 864 7.5; 24 x 128256 192 5.6, 384 6.2, 768 6.9; 1 x 262144 16 5.5, 32 5.0, 64 4.6; 96 x
 //    33000 288 7.8, 480 7.0, 864 7.5.
-//  - fp32, whose long chunks fill the registers: half as long up to four workgroups of the long ones per CU (200 x
-//    50000 800 17.0, 1400 13.6; 24 x 262144 384 11.6, 768 10.8; 96 x 128256 768 17.5, 1536 16.7), and a quarter while
-//    those are under four per CU and, beyond one per CU, at most 32 per row (200 x 20000 600 9.4, 1000 7.8; 1 x 262144
-//    32 5.7, 64 4.9; but 24 x 262144 1536 13.5, 16 x 262144 512 9.0, 1024 10.3).
+//  - fp32, whose long chunks fill the registers: half as long up to four workgroups of the long ones per CU (200 x 50000
+//    800 17.0, 1400 13.6; 24 x 262144 384 11.6, 768 10.8; 96 x 128256 768 17.5, 1536 16.7), and a quarter while those
+//    are under four per CU and, beyond one per CU, at most 16 per row (200 x 20000 600 9.4, 1000 7.8; 1 x 262144 32 5.7,
+//    64 4.9; but 16 x 128256 256 6.3, 512 6.6; 24 x 70000 216 5.8, 432 6.2; 24 x 262144 1536 13.5; 16 x 262144 512 9.0,
+//    1024 10.3).
 template <typename T>
 int coop_nv(long long rows, long long nvec) {
   constexpr int NV = 64 / T::V;
@@ -992,7 +993,7 @@ int coop_nv(long long rows, long long nvec) {
   int nv = NV;
   if constexpr (T::bytes == 4) {
     if (grid(NV) >= 4 * cus) return NV;
-    return grid(NV / 4) < 4 * cus && (grid(NV / 4) <= cus || chunks(NV / 4) <= 32) ? NV / 4 : NV / 2;
+    return grid(NV / 4) < 4 * cus && (grid(NV / 4) <= cus || chunks(NV / 4) <= 16) ? NV / 4 : NV / 2;
   }
   while (nv > NV / 4 && (grid(nv / 2) + cus - 1) / cus == (grid(nv) + cus - 1) / cus) nv /= 2;
   return nv;

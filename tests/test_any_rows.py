@@ -154,7 +154,8 @@ def test_emulated_coresident_same_bits(emu_softmax, rows, cols, dtype, groups, p
 # one row per workgroup: the workgroups of the chunk length chosen (256 CUs), where half of it would put more on a CU
 # (bf16) and where it would not; fp32 a quarter
 GRIDS = [(48, 33000, 1, 48 * 5), (24, 33000, 1, 24 * 9), (8, 70000, 1, 8 * 18), (20, 70000, 1, 20 * 9), (96, 33000, 1, 96 * 5),
-         (50, 20000, 0, 50 * 5), (110, 20000, 0, 110 * 5)]
+         (50, 20000, 0, 50 * 5), (110, 20000, 0, 110 * 5),
+         (14, 70000, 0, 14 * 18), (16, 70000, 0, 16 * 9)]
 
 
 @pytest.mark.parametrize("rows,cols,dtype,workgroups", GRIDS)
