@@ -51,7 +51,8 @@ int main(int argc, char** argv) {
     rmsnorm_tune(0, atoi(argv[6]));
     rmsnorm_tune(1, atoi(argv[7]));
     rmsnorm_tune(2, atoi(argv[8]));
-    if (const char* s = std::getenv("EMU_SHORT")) rmsnorm_tune(5, atoi(s));  // the short rows' kernel: 1 always, 2 never
+    // the short rows' kernel: 1 always, 2 never
+    if (const char* s = std::getenv("EMU_SHORT")) rmsnorm_tune(5, atoi(s));
   }
   const int offset = argc > 9 ? atoi(argv[9]) : 0;
   const float eps = 1e-6f;

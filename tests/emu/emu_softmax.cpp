@@ -57,7 +57,8 @@ int main(int argc, char** argv) {
   const std::string pattern = argc > 9 ? argv[9] : "randn";
   const int reps = argc > 10 ? atoi(argv[10]) : 1;
   if (argc > 11) softmax_tune(7, atoi(argv[11]));
-  if (const char* s = std::getenv("EMU_SHORT")) softmax_tune(9, std::atoi(s));  // the short rows' kernel: 1 always, 2 never
+  // the short rows' kernel: 1 always, 2 never
+  if (const char* s = std::getenv("EMU_SHORT")) softmax_tune(9, std::atoi(s));
   softmax_tune(5, tier);
   if (tier == 2) {
     softmax_tune(3, waves);
@@ -116,8 +117,8 @@ int main(int argc, char** argv) {
   long long bad = 0, first = -1;
   long long other = 0;  // elements whose bits are not the oracle's
   double error = 0.0;   // fp32: the sum of the relative errors of elements in the normal range
-  double ulps = 0.0;    // fp32: the largest error in units of the oracle's last place (of 2^-149 below the normal range)
-  double sums = 0.0;    // fp32: the sum over the rows of (sum of the row's outputs - 1)^2, the error of the row's own sum
+  double ulps = 0.0;    // fp32: the largest error in units of the oracle's last place (2^-149 below the normal range)
+  double sums = 0.0;    // fp32: the sum over the rows of (the sum of the row's outputs - 1)^2, the error of its own sum
   emu::Graph recorded;
   if (graph) {
     // an eager launch first (a warm-up, as a graph capture usually follows one), then the capture
@@ -158,7 +159,8 @@ int main(int argc, char** argv) {
         sum += a;
         int exponent = 0;
         std::frexp(b, &exponent);
-        if (std::isfinite(b)) ulps = std::fmax(ulps, std::fabs((double)a - b) / std::ldexp(1.0, std::max(exponent - 24, -149)));
+        const double ulp = std::ldexp(1.0, std::max(exponent - 24, -149));
+        if (std::isfinite(b)) ulps = std::fmax(ulps, std::fabs((double)a - b) / ulp);
         if (i % cols == (size_t)cols - 1) {
           sums += (sum - 1.0) * (sum - 1.0);
           sum = 0.0;

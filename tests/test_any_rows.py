@@ -26,14 +26,15 @@ EDGES = {0: [4, 5, 255, 257, 1023, 1025, 2047, 4097, 8191], 1: [8, 9, 511, 513, 
 
 @pytest.mark.parametrize("dtype,cols", [(d, c) for d in EDGES for c in EDGES[d]])
 def test_emulated_row_edges(emu_softmax, dtype, cols):
-    # offset 1: the buffers begin one element past a 16-byte boundary (and rows of a whole number of vectors are unaligned)
+    # offset 1: the buffers begin one element past a 16-byte boundary (and rows of a whole number of vectors are
+    # unaligned)
     run(emu_softmax, [9, cols, dtype, 1, cols, 0, 0, 1, "special"])
 
 
 # rows of one vector to 64 of them (fp32 4 to 256 columns, bf16 8 to 512) in softmax_short, numbers of rows that leave a
 # wave's sets empty or take several steps
-SHORT = [(1, 4, 0), (3, 5, 0), (17, 63, 0), (16, 64, 0), (9, 65, 0), (33, 127, 0), (8200, 130, 0), (1, 8, 1), (70, 9, 1),
-         (15, 127, 1), (40, 129, 1), (8, 256, 1), (8193, 257, 1)]
+SHORT = [(1, 4, 0), (3, 5, 0), (17, 63, 0), (16, 64, 0), (9, 65, 0), (33, 127, 0), (8200, 130, 0), (1, 8, 1),
+         (70, 9, 1), (15, 127, 1), (40, 129, 1), (8, 256, 1), (8193, 257, 1)]
 
 
 @pytest.mark.parametrize("pattern", ["randn", "special"])
@@ -43,7 +44,8 @@ def test_emulated_short_rows(emu_softmax, rows, cols, dtype, pattern):
 
 
 # where rows begin to share waves (256 CUs): workgroups of one wave of 16 or 8 rows, or of four waves of a row each
-@pytest.mark.parametrize("rows,cols,dtype,offset,workgroups", [(64, 64, 0, 0, 16), (4095, 64, 0, 0, 512), (4096, 64, 0, 0, 256),
+@pytest.mark.parametrize("rows,cols,dtype,offset,workgroups", [(64, 64, 0, 0, 16), (4095, 64, 0, 0, 512),
+                                                               (4096, 64, 0, 0, 256),
                                                                (64, 128, 1, 1, 16), (4096, 200, 1, 0, 512),
                                                                (4096, 200, 0, 0, 512), (8192, 200, 0, 0, 256)])
 def test_emulated_few_short_rows(emu_softmax, rows, cols, dtype, offset, workgroups):
@@ -57,7 +59,8 @@ def test_emulated_row_shapes(emu_softmax, dtype, waves, nv, env):
     run(emu_softmax, [21, 1999, dtype, 1, 5, waves, nv, 3, "randn"], env=dict(os.environ, **env))
 
 
-# rows, cols, dtype, row groups: chunks of 16384 elements and of a quarter of them (few rows), a last chunk of one vector
+# rows, cols, dtype, row groups: chunks of 16384 elements and of a quarter of them (few rows), a last chunk of one
+# vector
 COOP = [(2, 65539, 0, 0), (1, 4 * 4096 + 1, 0, 0), (3, 40001, 1, 0), (5, 16384 * 2 + 5, 0, 2), (5, 16384 * 3 - 1, 1, 3)]
 
 
@@ -102,31 +105,31 @@ def test_emulated_bf16_rounding(emu_softmax, rows, cols, offset):
     assert int(out.split("other bits ")[1].split()[0]) <= 6e-5 * rows * cols, out
 
 
-@pytest.mark.parametrize("cols,dtype,groups", [(4 * 4096 + 1, 1, 0), (4 * 4096 + 7, 1, 0), (2 * 16384 + 3, 1, 1), (4097, 0, 0),
-                                               (16384 + 3, 0, 1)])
+@pytest.mark.parametrize("cols,dtype,groups", [(4 * 4096 + 1, 1, 0), (4 * 4096 + 7, 1, 0), (2 * 16384 + 3, 1, 1),
+                                               (4097, 0, 0), (16384 + 3, 0, 1)])
 def test_emulated_last_chunk_writes_its_own(emu_softmax, cols, dtype, groups):
     # a last chunk of less than a vector, whose workgroup loads the row's last whole vector: the elements of the chunk
     # before are its workgroup's to write, whose rounding may be another; two rows, so that one group loops
     own = cols % 4096 if groups == 0 else cols % 16384
     chunks = cols // (4096 if groups == 0 else 16384) + 1
     env = dict(os.environ, EMU_ONLY=str(chunks - 1))
-    out = run(emu_softmax, [2 if groups else 1, cols, dtype, 4, 3, 0, groups, 0, "randn", 1, 1], env=env, expect_ok=False)
     rows = 2 if groups else 1
+    out = run(emu_softmax, [rows, cols, dtype, 4, 3, 0, groups, 0, "randn", 1, 1], env=env, expect_ok=False)
     written = [int(i) for i in out.split("written")[0].split()]
     assert written == [r * cols + i for r in range(rows) for i in range(cols - own, cols)]
 
 
 @pytest.mark.parametrize("cols", [3, 5, 300])
 def test_emulated_exponential(emu_softmax, cols):
-    # rows of 0, d and -inf with d down to -104: exp(d) / (1 + exp(d)) by the exponential (about an ulp), the sum and the
-    # quotient (half an ulp each), against the fp64 value rounded once (half an ulp): 2.5 ulps; by expf in the scalar kernel
-    # (3 columns) as well
+    # rows of 0, d and -inf with d down to -104: exp(d) / (1 + exp(d)) by the exponential (about an ulp), the sum and
+    # the quotient (half an ulp each), against the fp64 value rounded once (half an ulp): 2.5 ulps; by expf in the
+    # scalar kernel (3 columns) as well
     out = run(emu_softmax, [6000, cols, 0, 0, 1, 0, 0, 0, "pair"])
     assert float(out.split("worst ")[1].split()[0]) <= 2.5, out
 
 
-# rows, cols, dtype, kernel nodes of a captured launch: rows that an eager launch takes from the row tier stay there (one
-# node), longer ones have the co-resident tier's tag node before theirs
+# rows, cols, dtype, kernel nodes of a captured launch: rows that an eager launch takes from the row tier stay there
+# (one node), longer ones have the co-resident tier's tag node before theirs
 CAPTURED = [(8, 30000, 0, 1), (8, 30001, 0, 1), (8, 60000, 1, 1), (8, 60001, 1, 1), (2, 33000, 0, 2), (2, 65537, 1, 2)]
 
 
@@ -153,8 +156,8 @@ def test_emulated_coresident_same_bits(emu_softmax, rows, cols, dtype, groups, p
 
 # one row per workgroup: the workgroups of the chunk length chosen (256 CUs), where half of it would put more on a CU
 # (bf16) and where it would not; fp32 a quarter
-GRIDS = [(48, 33000, 1, 48 * 5), (24, 33000, 1, 24 * 9), (8, 70000, 1, 8 * 18), (20, 70000, 1, 20 * 9), (96, 33000, 1, 96 * 5),
-         (50, 20000, 0, 50 * 5), (110, 20000, 0, 110 * 5),
+GRIDS = [(48, 33000, 1, 48 * 5), (24, 33000, 1, 24 * 9), (8, 70000, 1, 8 * 18), (20, 70000, 1, 20 * 9),
+         (96, 33000, 1, 96 * 5), (50, 20000, 0, 50 * 5), (110, 20000, 0, 110 * 5),
          (14, 70000, 0, 14 * 18), (16, 70000, 0, 16 * 9)]
 
 
@@ -172,7 +175,8 @@ def test_emulated_fp32_row_sums(emu_softmax, rows, cols, offset):
     assert float(out.split("row sums off by ")[1].split()[0]) <= 6.6e-8, out
 
 
-@pytest.mark.parametrize("rows,cols,dtype,waves", [(5, 4096, 0, 16), (5, 20000, 0, 4), (5, 8192, 1, 16), (5, 2048, 1, 4)])
+@pytest.mark.parametrize("rows,cols,dtype,waves", [(5, 4096, 0, 16), (5, 20000, 0, 4), (5, 8192, 1, 16),
+                                                   (5, 2048, 1, 4)])
 def test_emulated_stream_nan(emu_softmax, rows, cols, dtype, waves):
     # with a vector or two per lane, some lanes hold masked elements only
     run(emu_softmax, [rows, cols, dtype, 2, 3, waves, 0, 0, "nan"])
@@ -212,7 +216,8 @@ def _check(pkg, oracle, dev, rows, cols, dtype, offset=0, special=False):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
 @pytest.mark.parametrize("rows,cols", [(3, 8), (70, 9), (40000, 8), (5000, 63), (70001, 64), (16385, 131), (9000, 255),
                                        (8191, 256), (8192, 257), (9001, 511), (20000, 512), (513, 255), (700, 513),
-                                       (5, 2049), (300, 3001), (9, 8191), (600, 16383), (3, 16384), (40, 20001), (2, 32767),
+                                       (5, 2049), (300, 3001), (9, 8191), (600, 16383), (3, 16384), (40, 20001),
+                                       (2, 32767),
                                        (300, 20000), (5, 65535), (3, 70001), (2, 262143), (70, 262143), (1, 1048576),
                                        (2, 1048577), (3, 16385), (9, 36869), (300, 49153)])
 def test_gpu_rows(pkg, oracle, dev, dtype, rows, cols):
@@ -222,8 +227,8 @@ def test_gpu_rows(pkg, oracle, dev, dtype, rows, cols):
 @pytest.mark.gpu
 @pytest.mark.parametrize("short", [1, 2], ids=["short", "row"])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
-@pytest.mark.parametrize("rows,cols,offset", [(3, 8, 0), (70, 9, 0), (1000, 64, 0), (333, 131, 0), (9000, 255, 1), (777, 256, 0),
-                                              (5, 200, 3), (40000, 8, 0), (8193, 100, 0)])
+@pytest.mark.parametrize("rows,cols,offset", [(3, 8, 0), (70, 9, 0), (1000, 64, 0), (333, 131, 0), (9000, 255, 1),
+                                              (777, 256, 0), (5, 200, 3), (40000, 8, 0), (8193, 100, 0)])
 def test_gpu_short_rows_either_way(pkg, oracle, dev, dtype, rows, cols, offset, short):
     lib = pkg.candidate("softmax")._lib
     lib.softmax_tune(9, short)
@@ -243,8 +248,8 @@ def test_gpu_offsets(pkg, oracle, dev, dtype, offset):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
-@pytest.mark.parametrize("rows,cols", [(5, 3001), (5, 4096), (5, 30000), (5, 49152), (5, 49999), (40, 70000), (5, 70001),
-                                       (300, 70000), (300, 70001), (5, 1200000)])
+@pytest.mark.parametrize("rows,cols", [(5, 3001), (5, 4096), (5, 30000), (5, 49152), (5, 49999), (40, 70000),
+                                       (5, 70001), (300, 70000), (300, 70001), (5, 1200000)])
 @pytest.mark.parametrize("ticks", [0, 1])
 def test_gpu_nan_among_masked(pkg, oracle, dev, dtype, rows, cols, ticks):
     # as test_emulated_coresident_nan: the row's middle half masked, in the row tiers and in the co-resident tier
@@ -279,17 +284,18 @@ def _fp64(rows, cols, dtype, offset, seed, dev):
 
 def _softmax_at(pkg, x, offset):
     y = torch.empty(x.numel() + offset, device=x.device, dtype=x.dtype)[offset:].view_as(x)
-    assert pkg.candidate("softmax")._lib.launch(x.data_ptr(), y.data_ptr(), *x.shape, 0 if x.dtype == torch.float32 else 1,
-                                                256, 1024, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    dtype = 0 if x.dtype == torch.float32 else 1
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert pkg.candidate("softmax")._lib.launch(x.data_ptr(), y.data_ptr(), *x.shape, dtype, 256, 1024, stream) == 0
     return y
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows,cols,offset", [(4096, 200, 1), (20000, 500, 1), (2000, 3001, 0), (512, 10000, 1), (600, 40000, 0),
-                                              (600, 40000, 1), (300, 60000, 0), (256, 128256, 1)])
+@pytest.mark.parametrize("rows,cols,offset", [(4096, 200, 1), (20000, 500, 1), (2000, 3001, 0), (512, 10000, 1),
+                                              (600, 40000, 0), (600, 40000, 1), (300, 60000, 0), (256, 128256, 1)])
 def test_gpu_bf16_rounding(pkg, dev, rows, cols, offset):
-    # the elements rounded otherwise than the fp64 softmax's, as test_emulated_bf16_rounding; longer rows hold more small
-    # elements, whose x - max is itself rounded (6.6e-5 of 600 x 40000 by expf and a division)
+    # the elements rounded otherwise than the fp64 softmax's, as test_emulated_bf16_rounding; longer rows hold more
+    # small elements, whose x - max is itself rounded (6.6e-5 of 600 x 40000 by expf and a division)
     print(f"[softmax bits] {rows}x{cols} offset {offset}", flush=True)
     x, e = _fp64(rows, cols, torch.bfloat16, offset, cols, dev)
     y = _softmax_at(pkg, x, offset)
@@ -300,10 +306,11 @@ def test_gpu_bf16_rounding(pkg, dev, rows, cols, offset):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows,cols,offset", [(16, 50000, 0), (16, 128256, 0), (64, 128256, 0), (4, 262144, 0), (16, 262144, 1)])
+@pytest.mark.parametrize("rows,cols,offset", [(16, 50000, 0), (16, 128256, 0), (64, 128256, 0), (4, 262144, 0),
+                                              (16, 262144, 1)])
 def test_gpu_fp32_error_of_few_long_rows(pkg, dev, rows, cols, offset):
-    # chunks of a half and a quarter of the longest: no further from the fp64 softmax than the longest ones (mean relative
-    # error 1.34e-7 to 1.55e-7 over these shapes; 1.0e-7 to 1.1e-7 with one exponential of x - max)
+    # chunks of a half and a quarter of the longest: no further from the fp64 softmax than the longest ones (mean
+    # relative error 1.34e-7 to 1.55e-7 over these shapes; 1.0e-7 to 1.1e-7 with one exponential of x - max)
     x, e = _fp64(rows, cols, torch.float32, offset, cols, dev)
     error = ((_softmax_at(pkg, x, offset).double() - e).abs() / e).mean().item()
     assert error <= 1.3e-7, error
@@ -311,8 +318,8 @@ def test_gpu_fp32_error_of_few_long_rows(pkg, dev, rows, cols, offset):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
-@pytest.mark.parametrize("rows,cols,offset", [(16, 20000, 0), (5, 50000, 0), (5, 50000, 1), (24, 128256, 0), (1, 262143, 0),
-                                              (300, 49152, 0), (300, 50000, 1), (300, 262144, 0)])
+@pytest.mark.parametrize("rows,cols,offset", [(16, 20000, 0), (5, 50000, 0), (5, 50000, 1), (24, 128256, 0),
+                                              (1, 262143, 0), (300, 49152, 0), (300, 50000, 1), (300, 262144, 0)])
 def test_gpu_timed_out_rows_have_the_same_bits(pkg, dev, dtype, rows, cols, offset):
     print(f"[softmax timed out] {rows}x{cols} {dtype} offset {offset}", flush=True)
     x, _ = _fp64(rows, cols, dtype, offset, cols, dev)
@@ -348,8 +355,8 @@ def test_gpu_rows_on_two_streams(pkg, oracle, dev):
 
 @pytest.mark.gpu
 def test_gpu_captured_rows_take_the_row_tier(pkg, oracle, dev):
-    # a captured launch of rows that an eager launch hands to the co-resident tier, whose rounding is another: replays on
-    # new values give the row tier's bits
+    # a captured launch of rows that an eager launch hands to the co-resident tier, whose rounding is another: replays
+    # on new values give the row tier's bits
     x = torch.empty(8, 30000, device=dev)
     lib = pkg.candidate("softmax")._lib
     pkg.softmax(x)

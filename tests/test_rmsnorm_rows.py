@@ -1,7 +1,7 @@
 """RMSNorm of short rows (rmsnorm_short: sixteen lanes per row, sixteen rows per wave and step): rows of one vector, of
 just under, exactly and just over one and two vectors per lane, and numbers of rows that leave sets, waves and blocks
-partly empty or take several steps; and of rows of any length and element alignment (the row kernel's kAny form), where a
-row's last vector, a wave's share or the next shape begins, with the fused residual in place, whose last vector overlaps
+partly empty or take several steps; and of rows of any length and element alignment (the row kernel's kAny form), where
+a row's last vector, a wave's share or the next shape begins, with the fused residual in place, whose last vector overlaps
 another lane's. Bit for bit against the oracle, as every RMSNorm path. The emulated cases run the kernels' source on the
 CPU between guard pages."""
 
@@ -20,8 +20,8 @@ def emu_rmsnorm(tmp_path_factory):
 
 
 # rows, cols, dtype (1 bf16, 2 fp16), mode (0 plain, 1 weighted), seed
-CASES = [(1, 8, 1, 1), (3, 64, 2, 0), (4, 120, 1, 1), (15, 128, 1, 1), (16, 128, 2, 1), (17, 136, 1, 1), (65, 192, 2, 0),
-         (100, 248, 1, 1), (33, 256, 1, 1)]
+CASES = [(1, 8, 1, 1), (3, 64, 2, 0), (4, 120, 1, 1), (15, 128, 1, 1), (16, 128, 2, 1), (17, 136, 1, 1),
+         (65, 192, 2, 0), (100, 248, 1, 1), (33, 256, 1, 1)]
 
 
 @pytest.mark.parametrize("rows,cols,dtype,mode", CASES)
@@ -30,7 +30,8 @@ def test_emulated_short_rows(emu_rmsnorm, rows, cols, dtype, mode):
 
 
 # where rows begin to share waves (256 CUs): one-wave workgroups of sixteen rows, or four-wave ones of a row a wave
-@pytest.mark.parametrize("rows,cols,workgroups", [(64, 128, 16), (3071, 128, 768), (3072, 128, 192), (64, 256, 16), (7168, 256, 448)])
+@pytest.mark.parametrize("rows,cols,workgroups", [(64, 128, 16), (3071, 128, 768), (3072, 128, 192), (64, 256, 16),
+                                                  (7168, 256, 448)])
 def test_emulated_few_short_rows(emu_rmsnorm, rows, cols, workgroups):
     out = run(emu_rmsnorm, [rows, cols, 1, 1, rows, 0, 0, 0, 0])
     assert int(out.split("workgroups ")[1].split()[0]) == workgroups, out
@@ -49,8 +50,8 @@ def test_emulated_any_rows(emu_rmsnorm, rows, cols, mode, waves, nv, offset, env
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
-@pytest.mark.parametrize("rows,cols", [(3, 9), (700, 100), (513, 511), (600, 513), (2000, 1129), (1100, 2049), (300, 5121),
-                                       (520, 4095), (40, 16385), (20, 65533), (2, 65537)])
+@pytest.mark.parametrize("rows,cols", [(3, 9), (700, 100), (513, 511), (600, 513), (2000, 1129), (1100, 2049),
+                                       (300, 5121), (520, 4095), (40, 16385), (20, 65533), (2, 65537)])
 def test_gpu_any_rows(pkg, oracle, dev, dtype, rows, cols):
     print(f"[rmsnorm any] {rows}x{cols} {dtype}", flush=True)
     g = torch.Generator().manual_seed(rows + cols)
@@ -89,7 +90,8 @@ def test_gpu_negative_zeros(pkg, oracle, dev, dtype, cols):
     x = torch.randn(9, cols, generator=g).to(dtype)
     x[:, ::3] = -0.0
     x[4] = -0.0
-    r = torch.where(torch.rand(9, cols, generator=g) < 0.5, torch.tensor(-0.0), torch.randn(9, cols, generator=g)).to(dtype)
+    r = torch.randn(9, cols, generator=g).to(dtype)
+    r[:, ::2] = -0.0
     w = (torch.rand(cols, generator=g) - 0.5).to(dtype)
     fp16 = dtype == torch.float16
     name = "fp16" if fp16 else "bf16"
